@@ -22,7 +22,7 @@
 #include "orth_common.h"
 
 namespace orth {
-hipError_t launch_general(const ForwardArgs &a, hipStream_t stream);
+hipError_t launch_general(const ForwardArgs &a, int cus, hipStream_t stream);
 hipError_t launch_dequant(const ForwardArgs &a, float *out, hipStream_t stream);
 hipError_t launch_pack_base(const void *w, int wdt, int64_t N, int64_t K, int64_t G, const void *s_in,
                             int sdt, uint8_t *q, void *s_out, hipStream_t stream);
@@ -572,7 +572,7 @@ int launch_kernel(const ForwardArgs &a, const void *plan, int kernel, int dev, h
             e = pf(a.has_ortho ? plan : nullptr);
         }
     } else {
-        e = launch_general(a, stream);
+        e = launch_general(a, g_dev[dev].cus, stream);
     }
     if (e != hipSuccess) return fail_hip(e, "kernel launch");
     return rc;

@@ -210,6 +210,28 @@ __device__ __forceinline__ void int4x8_to_bf16_biased(uint32_t w, uint32_t out[4
     out[3] = ((w >> 12) & 0x000F000Fu) ^ 0x43084308u;  // (3,7)
 }
 
+// Exact BF16 integers q in natural order, word i holding weights 2 i and
+// 2 i + 1: the nibble XOR 8 as a byte, converted to FP32 minus 8 (exact), the
+// high halves packed (an integer of magnitude at most 8 fits them).
+__device__ __forceinline__ void int4x8_to_bf16_exact(uint32_t w, uint32_t out[4]) {
+    const uint32_t u = w ^ 0x88888888u;
+    const uint32_t lo = u & 0x0F0F0F0Fu, hi = (u >> 4) & 0x0F0F0F0Fu;
+    // (the byte conversions written out: from C++ the compiler makes a field
+    // extract, an integer subtract and a conversion of each)
+    float e[4], o[4];
+    asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(e[0]) : "v"(lo));
+    asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(e[1]) : "v"(lo));
+    asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(e[2]) : "v"(lo));
+    asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(e[3]) : "v"(lo));
+    asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(o[0]) : "v"(hi));
+    asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(o[1]) : "v"(hi));
+    asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(o[2]) : "v"(hi));
+    asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(o[3]) : "v"(hi));
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        out[i] = __builtin_amdgcn_perm(__float_as_uint(o[i] - 8.0f), __float_as_uint(e[i] - 8.0f), 0x07060302u);
+}
+
 // Reorder 8 consecutive fp16 (as 4 words (0,1)(2,3)(4,5)(6,7)) into the
 // interleaved order (0,4)(1,5)(2,6)(3,7) used by int4x8_to_f16_interleaved.
 __device__ __forceinline__ u32x4 permute_x8(u32x4 d) {

@@ -161,7 +161,16 @@ static hipError_t launch_general_io(const ForwardArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t launch_general(const ForwardArgs &a, hipStream_t stream) {
+bool float_supported(const ForwardArgs &a);  // orth_float.hip
+hipError_t launch_float(const ForwardArgs &a, int cus, hipStream_t stream);
+
+hipError_t launch_general(const ForwardArgs &a, int cus, hipStream_t stream) {
+    // FP32 activations: the matrix-core kernels (orth_float.hip) take the same
+    // time for any batch of a tile, the general kernel's grows with M * N.
+    // They cross near M * N = 2^17: 4096 -> 4096 with group-128 scales, alpha =
+    // 1, 72 against 61 us at 24 tokens, 72 / 80 at 32, 101 / 1,292 at 512;
+    // 4096 -> 11008 75 / 62 at 8, 79 / 118 at 16; 1024 -> 4096 26 / 27 at 24.
+    if (a.M * a.N >= (1 << 17) && float_supported(a)) return launch_float(a, cus, stream);
     if (a.io_dtype == ORTH_DT_F32) return launch_general_io<ORTH_DT_F32>(a, stream);
     if (a.io_dtype == ORTH_DT_BF16) return launch_general_io<ORTH_DT_BF16>(a, stream);
     return launch_general_io<ORTH_DT_F16>(a, stream);

@@ -232,6 +232,34 @@ __device__ __forceinline__ void int4x8_to_bf16_exact(uint32_t w, uint32_t out[4]
         out[i] = __builtin_amdgcn_perm(__float_as_uint(o[i] - 8.0f), __float_as_uint(e[i] - 8.0f), 0x07060302u);
 }
 
+// Eight FP32 values as three bfloat16 vectors with v = p0 + p1 + p2 exactly
+// (finite v of at least 2^-100 in magnitude, or 0).  An infinity stays one in
+// p0 with p1 = p2 = 0; of a NaN at least p1 is one.
+__device__ __forceinline__ void split_bf16x3(const f32x4 &a, const f32x4 &b, u32x4 p[3]) {
+    uint32_t h[3][8];
+    float top = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float v = e < 4 ? a[e & 3] : b[e & 3];
+        const uint32_t u = __float_as_uint(v);
+        const float r1 = v - __uint_as_float(u & 0xffff0000u);
+        const uint32_t r = __float_as_uint(r1);
+        h[0][e] = u;
+        h[1][e] = r;
+        h[2][e] = __float_as_uint(r1 - __uint_as_float(r & 0xffff0000u));
+        top = fmaxf(top, fabsf(v));
+    }
+    if (top == __builtin_inff()) {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            if (fabsf(e < 4 ? a[e & 3] : b[e & 3]) == __builtin_inff()) h[1][e] = h[2][e] = 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) p[i][j] = __builtin_amdgcn_perm(h[i][2 * j + 1], h[i][2 * j], 0x07060302u);
+}
+
 // Reorder 8 consecutive fp16 (as 4 words (0,1)(2,3)(4,5)(6,7)) into the
 // interleaved order (0,4)(1,5)(2,6)(3,7) used by int4x8_to_f16_interleaved.
 __device__ __forceinline__ u32x4 permute_x8(u32x4 d) {

@@ -41,17 +41,17 @@ def bound(lay, x, alpha):
     return adds * 2.0 ** -23 * (np.abs(x).astype(np.float64) @ w.T) + 1e-30
 
 
-# the general kernel's last batch and the first of these kernels (M * N = 2^17),
-# ragged token and row tiles, one K step, odd and even steps per scale group,
-# one scale per row over an odd number of steps, 8 / 4 / 2 tokens per sparse
-# workgroup (K = 4096, 9216, 11008), more entries per row than one batch of
-# loads holds, FP32 scales and values
+# the dispatch's edges (M * N = 2^17 with FP32 scales, else 200,000 or
+# 300,000), ragged token and row tiles, one K step, odd and even steps per
+# scale group, one scale per row over an odd number of steps, 8 / 4 / 2 tokens
+# per sparse workgroup (K = 4096, 9216, 11008), more entries per row than one
+# batch of loads holds, FP32 scales and values
 @pytest.mark.parametrize("K,N,group,M,density,alpha,wide", [
-    (4096, 1024, 128, 127, 0.01, 1.0, False), (4096, 1024, 128, 128, 0.01, 1.0, False),
-    (64, 2050, 64, 65, 0.05, 1.0, False), (192, 2049, 192, 129, 0.05, 0.5, False),
-    (320, 1111, None, 130, 0.2, 1.0, True), (1024, 1000, 256, 191, 0.0, 1.0, False),
-    (9216, 520, 128, 253, 0.01, 1.0, False), (11008, 700, 128, 200, 0.02, 1.0, True),
-    (8192, 300, 64, 440, 0.01, 0.0, False)])
+    (4096, 1024, 128, 127, 0.01, 1.0, True), (4096, 1024, 128, 128, 0.01, 1.0, True),
+    (4096, 1200, 128, 250, 0.01, 1.0, False), (64, 4650, 64, 65, 0.05, 1.0, False),
+    (192, 2333, 192, 129, 0.05, 0.5, False), (320, 1111, None, 130, 0.2, 1.0, True),
+    (1024, 1600, 256, 191, 0.0, 1.0, False), (9216, 1000, 128, 253, 0.01, 1.0, False),
+    (11008, 1010, 128, 200, 0.02, 1.0, False), (8192, 460, 64, 440, 0.01, 0.0, False)])
 def test_float_parity(oracle_mod, K, N, group, M, density, alpha, wide):
     lay = W.make_layer(K, N, group, density, 7000 + K + M)
     x = np.random.Generator(np.random.PCG64(M)).normal(0, 1, (M, K)).astype(np.float32)
@@ -63,7 +63,7 @@ def test_float_parity(oracle_mod, K, N, group, M, density, alpha, wide):
 
 def test_float_small_and_large_activations_keep_their_bits(oracle_mod):
     """Magnitudes over 40 binades, values whose 24 bits are all ones."""
-    K, N, M = 512, 1100, 130
+    K, N, M = 512, 2400, 130
     lay = W.make_layer(K, N, 128, 0.02, 7100)
     g = np.random.Generator(np.random.PCG64(1))
     x = np.ldexp(np.float32(2) - np.float32(2 ** -23), g.integers(-20, 20, (M, K))).astype(np.float32)
@@ -73,7 +73,7 @@ def test_float_small_and_large_activations_keep_their_bits(oracle_mod):
 
 
 def test_float_infinities_and_nan_stay_with_their_token():
-    K, N, M = 256, 2048, 70
+    K, N, M = 256, 4400, 70
     lay = W.make_layer(K, N, 128, 0.02, 7200)
     x = W.make_x(M, K, 7201).astype(np.float32)
     clean = run(lay, x, 1.0)
@@ -96,7 +96,7 @@ def test_float_infinities_and_nan_stay_with_their_token():
 def test_float_odd_csr_and_bias(oracle_mod):
     """Duplicate and unsorted columns and columns out of range, as given; the
     bias is added to the finished output."""
-    K, N, M = 256, 1030, 140
+    K, N, M = 256, 2150, 140
     lay = W.make_layer(K, N, 128, 0.05, 7300)
     lay.col[:] = lay.col[::-1].copy()
     lay.col[::7] = lay.col[3]

@@ -13,6 +13,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <string>
+#include <vector>
 
 #include "orth_hip.h"
 
@@ -113,25 +114,35 @@ orth_hip_layer_t describe(const at::Tensor &q, const at::Tensor &s, const at::Te
     return L;
 }
 
+// A plan's pointer and size (none: null, 0).
+const void *plan_ptr(const c10::optional<at::Tensor> &plan, const at::Device &dev, int64_t *bytes) {
+    *bytes = 0;
+    if (!plan.has_value() || !plan->defined() || plan->numel() == 0) return nullptr;
+    req(plan->device() == dev && plan->scalar_type() == at::kByte, "plan must be a uint8 tensor on input's device");
+    *bytes = plan->numel();
+    return ptr(*plan);
+}
+
+// A bias's pointer and dtype (none: null).
+const void *bias_ptr(const c10::optional<at::Tensor> &bias, const at::Device &dev, int64_t N, int32_t *dtype) {
+    *dtype = 0;
+    if (!bias.has_value() || !bias->defined()) return nullptr;
+    req(bias->device() == dev && io_dtype(*bias) >= 0 && bias->numel() == N && bias->is_contiguous(),
+        "bias must be a contiguous float tensor of " + std::to_string(N) + " elements on input's device");
+    *dtype = io_dtype(*bias);
+    return ptr(*bias);
+}
+
 void launch(const orth_hip_layer_t &L, const c10::optional<at::Tensor> &plan, const c10::optional<at::Tensor> &bias,
             const at::Tensor &x, at::Tensor &y) {
     const at::Device dev = x.device();
-    const bool has_plan = plan.has_value() && plan->defined() && plan->numel() > 0;
-    if (has_plan)
-        req(plan->device() == dev && plan->scalar_type() == at::kByte, "plan must be a uint8 tensor on input's device");
-    const void *bp = nullptr;
+    int64_t pbytes = 0;
     int32_t bdt = 0;
-    if (bias.has_value() && bias->defined()) {
-        req(bias->device() == dev && io_dtype(*bias) >= 0 && bias->numel() == y.size(1) && bias->is_contiguous(),
-            "bias must be a contiguous float tensor of " + std::to_string(y.size(1)) +
-                " elements on input's device");
-        bp = ptr(*bias);
-        bdt = io_dtype(*bias);
-    }
+    const void *pp = plan_ptr(plan, dev, &pbytes);
+    const void *bp = bias_ptr(bias, dev, y.size(1), &bdt);
     c10::DeviceGuard guard(dev);
     hipStream_t st = c10::hip::getCurrentHIPStream(dev.index()).stream();
-    check_rc(orth_layer_forward_hip_ex(&L, has_plan ? ptr(*plan) : nullptr, has_plan ? plan->numel() : 0, bp, bdt,
-                                       ptr(x), ptr(y), x.size(0), io_dtype(x), st));
+    check_rc(orth_layer_forward_hip_ex(&L, pp, pbytes, bp, bdt, ptr(x), ptr(y), x.size(0), io_dtype(x), st));
 }
 
 // forward_planned(q, s, v, c, rp, input, output, alpha, plan=None, bias=None)
@@ -160,6 +171,52 @@ at::Tensor linear(const at::Tensor &x, const at::Tensor &q, const at::Tensor &s,
     return y;
 }
 
+// linear_group(x2d, [(q, s, v, c, rp, out_features, alpha, plan, bias), ...])
+// -> [y, ...]: orth_layers_forward_hip over layers that read one input, the
+// outputs allocated.
+std::vector<at::Tensor> linear_group(const at::Tensor &x, const py::sequence &layers) {
+    req(x.is_cuda(), "OrthoLinear runs on a ROCm GPU only; move the modules and the input to a cuda device");
+    req(x.dim() == 2, "input must be 2-D [M, K]");
+    const size_t n = layers.size();
+    req(n >= 1 && n <= ORTH_GROUP_MAX, "a group holds 1.." + std::to_string(ORTH_GROUP_MAX) + " layers, got " +
+                                           std::to_string(n));
+    const at::Device dev = x.device();
+    c10::DeviceGuard guard(dev);
+    const at::Tensor xc = x.contiguous();
+    std::vector<at::Tensor> ys, keep;  // keep: contiguous copies of biases, until the launch
+    orth_hip_layer_t L[ORTH_GROUP_MAX];
+    const orth_hip_layer_t *lp[ORTH_GROUP_MAX];
+    const void *plans[ORTH_GROUP_MAX], *biases[ORTH_GROUP_MAX];
+    int64_t pbytes[ORTH_GROUP_MAX];
+    int32_t bdt[ORTH_GROUP_MAX];
+    void *out[ORTH_GROUP_MAX];
+    for (size_t l = 0; l < n; l++) {
+        const py::tuple t = py::cast<py::tuple>(layers[l]);
+        req(t.size() == 9, "a layer is (q, scales, values, columns, row_ptr, out_features, alpha, plan, bias)");
+        const int64_t N = py::cast<int64_t>(t[5]);
+        ys.push_back(at::empty({xc.size(0), N}, xc.options()));
+        check_io(xc, ys[l]);
+        // (the weight tensors are the caller's: alive for the call)
+        L[l] = describe(py::cast<at::Tensor>(t[0]), py::cast<at::Tensor>(t[1]), py::cast<at::Tensor>(t[2]),
+                        py::cast<at::Tensor>(t[3]), py::cast<at::Tensor>(t[4]), xc.size(1), N,
+                        py::cast<double>(t[6]), dev);
+        lp[l] = &L[l];
+        const auto plan = py::cast<c10::optional<at::Tensor>>(t[7]);
+        plans[l] = plan_ptr(plan, dev, &pbytes[l]);
+        auto bias = py::cast<c10::optional<at::Tensor>>(t[8]);
+        if (bias.has_value() && bias->defined()) {
+            keep.push_back(bias->contiguous());
+            bias = keep.back();
+        }
+        biases[l] = bias_ptr(bias, dev, N, &bdt[l]);
+        out[l] = ptr(ys[l]);
+    }
+    hipStream_t st = c10::hip::getCurrentHIPStream(dev.index()).stream();
+    check_rc(orth_layers_forward_hip(lp, plans, pbytes, biases, bdt, (int32_t)n, ptr(xc), out, xc.size(0),
+                                     io_dtype(xc), st));
+    return ys;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_torch_ops, m) {
@@ -172,5 +229,7 @@ PYBIND11_MODULE(_torch_ops, m) {
           py::arg("input"), py::arg("q_weight"), py::arg("q_scales"), py::arg("ortho_values"),
           py::arg("ortho_col_indices"), py::arg("ortho_row_ptr"), py::arg("out_features"), py::arg("alpha"),
           py::arg("plan") = py::none(), py::arg("bias") = py::none());
+    m.def("linear_group", &linear_group, "several layers over one 2-D input: the outputs allocated and written",
+          py::arg("input"), py::arg("layers"));
     m.def("abi_version", &orth_hip_abi_version);
 }

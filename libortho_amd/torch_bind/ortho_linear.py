@@ -298,7 +298,42 @@ class OrthoLinear(nn.Module):
         K = modules[0].in_features
         if any(m.in_features != K for m in modules):
             raise ValueError("the layers of a group must share in_features")
-        x_flat = x.reshape(-1, K).contiguous()
+        T = _lib.torch_ops()
+        if T is None:
+            return OrthoLinear._forward_group_ctypes(modules, x)
+        layers, late = [], []
+        for m in modules:
+            bufs = m._buffers
+            b = m._parameters["bias"]
+            fuse = b is not None and not (torch.is_grad_enabled() and b.requires_grad) and b.device == x.device
+            late.append(b if b is not None and not fuse else None)
+            layers.append((bufs["base_weight"], bufs["base_scales"], bufs["ortho_values"], bufs["ortho_col_indices"],
+                           bufs["ortho_row_ptr"], m.out_features, float(m.alpha),
+                           m._call_plan() if m.alpha > 0 else None, b.detach() if fuse else None))
+        outs = T.linear_group(x if x.dim() == 2 else x.reshape(-1, K), layers)
+        for out, b in zip(outs, late):
+            if b is not None:
+                out += b
+        return outs if x.dim() == 2 else [out.view(*x.shape[:-1], out.shape[1]) for out in outs]
+
+    def _call_plan(self):
+        """The plan of a forward call on the current stream: forward's fast
+        check, else :meth:`_ortho_plan`."""
+        bufs = self._buffers
+        vals = bufs["ortho_values"]
+        if vals.numel() == 0:
+            return None
+        f = self.__dict__.get("_plan_fast")
+        if f is not None and f[0] is vals and f[1] is bufs["ortho_col_indices"] and f[2] is bufs["ortho_row_ptr"] and \
+                f[3] == (vals._version, vals.data_ptr(), f[1]._version, f[2]._version) and \
+                f[4] == _C._raw_stream(vals.get_device()):
+            return self._plan
+        return self._ortho_plan()
+
+    @staticmethod
+    def _forward_group_ctypes(modules, x: torch.Tensor):
+        """forward_group through the ctypes binding (when the compiled one is absent)."""
+        x_flat = x.reshape(-1, modules[0].in_features).contiguous()
         outs, plans, biases, late = [], [], [], []
         for m in modules:
             outs.append(torch.empty(x_flat.shape[0], m.out_features, device=x.device, dtype=x.dtype))

@@ -207,3 +207,31 @@ def test_ortholinear_forward_group(gpu):
                 ref = m(x)
                 assert y.shape == ref.shape
                 assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype,shape", [(torch.float16, (3, 1024)), (torch.bfloat16, (2, 5, 1024)),
+                                         (torch.float16, (1024,)), (torch.float16, (0, 1024))])
+def test_group_binding_gives_the_ctypes_results(gpu, dtype, shape):
+    """forward_group's one call into the compiled binding: the outputs (and
+    their shapes) of the ctypes path, with a fused bias, a bias autograd must
+    see, alpha off and an empty ortho term among the layers."""
+    from libortho_amd.torch_bind import OrthoLinear
+    mods = []
+    for i, (N, density, bias) in enumerate([(256, 0.02, False), (520, 0.02, True), (128, 0.0, True), (384, 0.02, False)]):
+        lay = W.make_layer(1024, N, 128, density, 8800 + i)
+        m = OrthoLinear(1024, N, bias=bias, group_size=128, device="cuda")
+        d = W.to_device(lay)
+        m.load_state_dict({"base_weight": d["q"], "base_scales": d["scales"], "ortho_values": d["vals"],
+                           "ortho_col_indices": d["col"], "ortho_row_ptr": d["row_ptr"],
+                           **({"bias": torch.randn(N)} if bias else {})})
+        mods.append(m)
+    mods[2].bias.requires_grad_(False)
+    mods[3].set_alpha(0.0)
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(1)).cuda().to(dtype)
+    got = OrthoLinear.forward_group(mods, x)
+    want = OrthoLinear._forward_group_ctypes(mods, x)
+    for g, w, m in zip(got, want, mods):
+        assert g.shape == w.shape == (*shape[:-1], m.out_features) and g.dtype == w.dtype
+        assert torch.equal(g, w) and g.requires_grad == w.requires_grad
+    with pytest.raises(RuntimeError):
+        OrthoLinear.forward_group(mods, x.double())

@@ -71,6 +71,7 @@ hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, vo
 hipError_t launch_sieve_split(const void *w, int dt, int64_t N, int64_t K, const void *h, int hdt, int64_t h_stride,
                               int score_dt, int use_rank, int64_t rank, float thresh, void *w_base, void *w_ortho,
                               float *score, void *sel, int ieee_div, hipStream_t stream);
+int64_t sieve_select_bytes();
 int64_t sieve_hdiag_slices(int64_t n);
 hipError_t launch_sieve_hdiag(const void *x, int dt, int64_t n, int64_t K, float *partial, void *out, int ieee_div,
                               hipStream_t stream);
@@ -875,7 +876,7 @@ int orth_sieve_quantize_hip(const void *w, int32_t w_dtype, int64_t out_features
     return ORTH_OK;
 }
 
-int64_t orth_sieve_select_bytes(void) { return 1040; }
+int64_t orth_sieve_select_bytes(void) { return sieve_select_bytes(); }
 
 int orth_sieve_split_hip(const void *w, int32_t w_dtype, int64_t out_features, int64_t in_features,
                          const void *h_inv, int32_t h_dtype, int64_t h_stride, int32_t score_dtype,

@@ -10,19 +10,29 @@
 //                            w_base = q * s, non-finite results 0.  Every
 //                            intermediate is rounded to w's dtype, as the
 //                            torch ops round each result.
-//  hessian_sieve (:25-76)   the same pass also writes the residual w - w_base
-//                            and the score residual^2 / (H_inv + 1e-6); with a
-//                            sparsity target, the k-th largest score is found by
-//                            a radix select over the order-preserving key of
-//                            each FP32 score (NaN largest, as torch.topk),
-//                            8 bits per pass; then w_ortho = residual * (score > t).
+//  hessian_sieve (:25-76)   the same pass also writes the score residual^2 /
+//                            (H_inv + 1e-6); with a sparsity target, the k-th
+//                            largest score is found by a radix select over the
+//                            order-preserving key of each FP32 score (NaN
+//                            largest, as torch.topk): 11 bits counted in the
+//                            first pass itself, 11 in a pass over the scores
+//                            that also collects those of the found prefix, 10
+//                            over the collected ones; then w_ortho = residual *
+//                            (score > t), both formed again from w and w_base.
 //  compute_hessian_diag_approx (:79-95)  diag(X^T X) / n + 1e-6: the
 //                            diagonal only (column sums of squares, FP32
 //                            partial sums over row slices added in slice
 //                            order), not the K x K product.
 //
 // Off the forward path: these run once per weight matrix when a model is
-// split, and are measured as load-time work.
+// split, and are measured as load-time work.  The split is bound by memory:
+// w read and w_base and the scores written, the scores read once, w and
+// w_base read and w_ortho written, 28 bytes an FP32 weight.  4096 x 4096 FP32,
+// 2 % kept: 106 us (40 + 16 + 5 + 36 in the passes, 5 TB/s), against 371 us with
+// the residual stored, four 8-bit passes over all scores (58 us each, on a
+// handful of histogram bins' LDS atomics) and a one-thread scan after each.
+#include <atomic>
+
 #include "orth_common.h"
 
 namespace orth {
@@ -49,10 +59,9 @@ __device__ __forceinline__ float sieve_unkey(uint32_t k) {
 
 struct SieveArgs {
     const void *w;
-    int dt;
     int64_t N, K;
     void *w_base;
-    void *resid;        // w_ortho buffer: the residual, masked later (or null)
+    void *w_ortho;      // or null: quantise only
     float *score;       // [N*K] score values (exact in FP32), or null
     const void *h;      // H_inv: element k at h[k * h_stride]
     int hdt;
@@ -60,6 +69,9 @@ struct SieveArgs {
     int score_dt;       // dtype of the score (torch's promotion of w's and H's)
     int ieee_div;       // 1: division by a host scalar as IEEE division (CPU
                         // tensors), 0: as a product with its FP32 reciprocal
+    struct SieveSel *sel;  // radix select, or null: the threshold below
+    uint32_t rank;
+    float thresh;
 };
 
 // v / d for a host scalar d, as torch computes it on the tensor's device.
@@ -67,105 +79,345 @@ __device__ __forceinline__ float sieve_scalar_div(float v, float d, int ieee_div
     return ieee_div ? v / d : v * (1.0f / d);
 }
 
-__global__ void __launch_bounds__(kSieveNT) sieve_quant_kernel(SieveArgs a) {
-    __shared__ float red[kSieveNT / 64];
-    const int64_t r = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int64_t base = r * a.K;
-    float m = 0.f;
-    for (int64_t k = tid; k < a.K; k += kSieveNT) m = sieve_max_nan(m, fabsf(load_as_f32(a.w, a.dt, base + k)));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = sieve_max_nan(m, __shfl_xor(m, off, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = m;
-    __syncthreads();
-    m = red[0];
-#pragma unroll
-    for (int i = 1; i < kSieveNT / 64; i++) m = sieve_max_nan(m, red[i]);
-    // clamp(min=1e-8): the bound in w's dtype (0 in FP16), NaN kept
-    const float lo = round_as(a.dt, 1e-8f);
-    const float mc = (m != m) ? m : fmaxf(m, lo);
-    const float s = round_as(a.dt, sieve_scalar_div(mc, 7.0f, a.ieee_div));
-    for (int64_t k = tid; k < a.K; k += kSieveNT) {
-        const float wv = load_as_f32(a.w, a.dt, base + k);
-        float t = rintf(round_as(a.dt, wv / s));
-        t = (t != t) ? t : fminf(fmaxf(t, -8.f), 7.f);
-        float wb = round_as(a.dt, t * s);
-        if (!__builtin_isfinite(wb)) wb = 0.f;
-        store_from_f32(a.w_base, a.dt, base + k, wb);
-        if (a.resid) {
-            const float rr = round_as(a.dt, wv - wb);
-            store_from_f32(a.resid, a.dt, base + k, rr);
-            const float r2 = round_as(a.dt, rr * rr);
-            const float hs = round_as(a.hdt, load_as_f32(a.h, a.hdt, k * a.h_stride) + 1e-6f);
-            a.score[base + k] = round_as(a.score_dt, r2 / hs);
-        }
-    }
-}
-
-// Radix-select state: the key prefix found so far, its mask, the rank still
-// sought within the prefix (1 = largest), and the histogram of the pass.
+// Radix-select state: a histogram per level (a few copies, each added to by
+// every fourth workgroup, so that fewer atomics meet on one counter), the
+// bins found so far with the rank left within them, and the collected
+// scores per workgroup of the second pass (-1: too many for its part of the
+// buffer).
+constexpr int kSelBins = 2048, kSelCopies = 4, kSelWgs = 1024;
 struct SieveSel {
-    uint32_t prefix, mask, k, pad;
-    uint32_t hist[256];
+    uint32_t hist[3][kSelCopies][kSelBins];
+    uint32_t bin[2], left[2];
+    int32_t count[kSelWgs];
 };
+constexpr int kSvNT = 512;                      // threads of the split's passes
+constexpr int kSvLdsCols = 16384;               // columns of h + 1e-6 a workgroup keeps in LDS
+constexpr int kSvCache = 4;                     // vectors of a row per thread kept in registers
+constexpr int kSvLanes = 4;                     // LDS histograms, by lane
 
-__global__ void sieve_sel_init_kernel(SieveSel *st, uint32_t k) {
-    const int t = threadIdx.x;
-    st->hist[t] = 0;
-    if (t == 0) {
-        st->prefix = 0;
-        st->mask = 0;
-        st->k = k;
-        st->pad = 0;
-    }
+int64_t sieve_select_bytes() { return (int64_t)sizeof(SieveSel); }
+
+__global__ void __launch_bounds__(256) sieve_sel_init_kernel(SieveSel *st) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 3 * kSelCopies * kSelBins) (&st->hist[0][0][0])[i] = 0u;
 }
 
-__global__ void __launch_bounds__(kSieveNT) sieve_hist_kernel(const float *score, int64_t n, SieveSel *st,
-                                                              int shift) {
-    __shared__ uint32_t h[256];
-    const int tid = threadIdx.x;
-    h[tid] = 0;
-    __syncthreads();
-    const uint32_t prefix = st->prefix, mask = st->mask;
-    for (int64_t i = (int64_t)blockIdx.x * kSieveNT + tid; i < n; i += (int64_t)gridDim.x * kSieveNT) {
-        const uint32_t key = sieve_key(score[i]);
-        if ((key & mask) == prefix) atomicAdd(&h[(key >> shift) & 255u], 1u);
+// The bin of level `lv` (from the top) that holds the k-th largest key, and
+// the rank within it; every thread of the workgroup gets both.  Workgroup 0
+// records them for the later passes.
+__device__ void sieve_pick(SieveSel *st, int lv, uint32_t k, uint32_t &bin, uint32_t &left) {
+    __shared__ uint32_t part[kSvNT / 64], found[2];
+    constexpr int PER = kSelBins / kSvNT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint32_t c[PER], sum = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        c[j] = 0;
+#pragma unroll
+        for (int i = 0; i < kSelCopies; i++) c[j] += st->hist[lv][i][tid * PER + j];
+        sum += c[j];
     }
+    uint32_t incl = sum;  // keys in this thread's bins and those of later lanes, then of later waves
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_down(incl, off);
+        if (lane + off < 64) incl += v;
+    }
+    if (lane == 0) part[wave] = incl;
     __syncthreads();
-    if (h[tid]) atomicAdd(&st->hist[tid], h[tid]);
-}
-
-// One thread: the bin (from the top) that holds the k-th largest key; the
-// histogram is cleared for the next pass.
-__global__ void sieve_pick_kernel(SieveSel *st, int shift) {
-    if (threadIdx.x == 0) {
-        uint32_t k = st->k;
-        for (int b = 255; b >= 0; b--) {
-            const uint32_t c = st->hist[b];
-            if (k <= c) {
-                st->prefix |= (uint32_t)b << shift;
-                st->mask |= 255u << shift;
-                break;
-            }
-            k -= c;
+    uint32_t above = incl - sum;
+    for (int w = wave + 1; w < kSvNT / 64; w++) above += part[w];
+#pragma unroll
+    for (int j = PER - 1; j >= 0; j--) {
+        if (k > above && k <= above + c[j]) {  // (one bin of one thread)
+            found[0] = (uint32_t)(tid * PER + j);
+            found[1] = k - above;
         }
-        st->k = k;
+        above += c[j];
     }
     __syncthreads();
-    st->hist[threadIdx.x] = 0;
+    bin = found[0];
+    left = found[1];
+    if (blockIdx.x == 0 && tid == 0 && lv < 2) {
+        st->bin[lv] = bin;
+        st->left[lv] = left;
+    }
 }
 
-// w_ortho = residual * (score > t): t the selected k-th largest score
-// (from_sel) or the caller's threshold rounded to the score's dtype (torch
-// compares a tensor with a host scalar in the tensor's dtype); NaN compares
-// false.
-__global__ void __launch_bounds__(kSieveNT) sieve_mask_kernel(void *resid, int dt, const float *score, int64_t n,
-                                                              const SieveSel *st, int from_sel, float thresh,
-                                                              int score_dt) {
-    const float t = from_sel ? sieve_unkey(st->prefix) : round_as(score_dt, thresh);
-    for (int64_t i = (int64_t)blockIdx.x * kSieveNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kSieveNT) {
-        const float r = load_as_f32(resid, dt, i);
-        store_from_f32(resid, dt, i, round_as(dt, r * (score[i] > t ? 1.f : 0.f)));
+// a * b as an FP32 product of its own: rounded to FP16 at once the compiler
+// makes it a fused multiply-add with +0, which turns a product of -0 into +0.
+__device__ __forceinline__ float sieve_mul(float a, float b) {
+    float p = a * b;
+    asm("" : "+v"(p));
+    return p;
+}
+
+// V consecutive elements from i, as floats.
+template <int DT, int V>
+__device__ __forceinline__ void sieve_load(const void *p, int64_t i, float v[V]) {
+    if constexpr (V == 1) {
+        v[0] = load_as_f32(p, DT, i);
+    } else if constexpr (DT == ORTH_DT_F32) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(p) + i);
+#pragma unroll
+        for (int e = 0; e < V; e++) v[e] = a[e];
+    } else {
+        const uint2 a = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(p) + i);
+        const uint32_t u[2] = {a.x, a.y};
+#pragma unroll
+        for (int e = 0; e < V; e++) {
+            const uint16_t b = (uint16_t)(u[e >> 1] >> (16 * (e & 1)));
+            v[e] = DT == ORTH_DT_F16 ? (float)__builtin_bit_cast(f16, b) : bf16_bits_to_f32(b);
+        }
+    }
+}
+
+template <int DT, int V>
+__device__ __forceinline__ void sieve_store(void *p, int64_t i, const float v[V]) {
+    if constexpr (V == 1) {
+        store_from_f32(p, DT, i, v[0]);
+    } else if constexpr (DT == ORTH_DT_F32) {
+        *reinterpret_cast<f32x4 *>(static_cast<float *>(p) + i) = f32x4{v[0], v[1], v[2], v[3]};
+    } else {
+        uint32_t u[V];
+#pragma unroll
+        for (int e = 0; e < V; e++)
+            u[e] = DT == ORTH_DT_F16 ? (uint32_t)__builtin_bit_cast(uint16_t, (f16)v[e]) : (uint32_t)f32_to_bf16_bits(v[e]);
+        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p) + i) = uint2{u[0] | (u[1] << 16), u[2] | (u[3] << 16)};
+    }
+}
+
+// h + 1e-6 in h's dtype: in LDS for every column (HL), else of column k from
+// memory.
+template <bool HL>
+__device__ __forceinline__ float sieve_h(const SieveArgs &a, const float *hs, int64_t k) {
+    if constexpr (HL) return hs[k];
+    else return round_as(a.hdt, load_as_f32(a.h, a.hdt, k * a.h_stride) + 1e-6f);
+}
+
+template <bool HL>
+__device__ __forceinline__ void sieve_stage_h(const SieveArgs &a, float *hs) {
+    if constexpr (HL)
+        for (int64_t k = threadIdx.x; k < a.K; k += kSvNT)
+            hs[k] = round_as(a.hdt, load_as_f32(a.h, a.hdt, k * a.h_stride) + 1e-6f);
+}
+
+// The residual and the score of an element, as the torch ops round them
+// (S32: the score's dtype is FP32; else one of the two others, by a select).
+template <int DT, bool S32>
+__device__ __forceinline__ float sieve_score(float wv, float wb, float hs, bool s16, float &resid) {
+    resid = round_as(DT, wv - wb);
+    const float sc = round_as(DT, sieve_mul(resid, resid)) / hs;
+    if constexpr (S32) return sc;
+    const float f = (float)(f16)sc, b = bf16_bits_to_f32(f32_to_bf16_bits(sc));
+    return s16 ? f : b;
+}
+
+// Rows blockIdx.x, + gridDim.x, ...: max|w|, w_base, and with a score buffer
+// the scores, their top 11 key bits counted when a rank is selected.  V
+// elements per load (4: aligned rows).  A row's first kSvCache vectors per
+// thread stay in registers between the two sweeps.
+// (4 waves per SIMD: two workgroups a CU, one's loads beside the other's
+// divisions)
+template <int DT, int V, bool HL, bool S32>
+__global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4))) sieve_quant_kernel(SieveArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    float *hs = reinterpret_cast<float *>(smem);
+    uint32_t *hist = reinterpret_cast<uint32_t *>(smem + (HL ? a.K * 4 : 0));
+    __shared__ float red[2][kSvNT / 64];
+    const int tid = threadIdx.x;
+    const bool count = a.score && a.sel, s16 = a.score_dt == ORTH_DT_F16;  // (uniform)
+    if (a.score) sieve_stage_h<HL>(a, hs);
+    if (count)
+        for (int i = tid; i < kSvLanes * kSelBins; i += kSvNT) hist[i] = 0u;
+    __syncthreads();
+    uint32_t *mine = hist + (tid & (kSvLanes - 1)) * kSelBins;
+    int par = 0;
+    for (int64_t r = blockIdx.x; r < a.N; r += gridDim.x, par ^= 1) {
+        const int64_t base = r * a.K;
+        float w[kSvCache][V];
+        float m = 0.f;
+        for (int64_t b0 = 0; b0 < a.K; b0 += (int64_t)kSvCache * kSvNT * V) {
+            float t[kSvCache][V];
+#pragma unroll
+            for (int j = 0; j < kSvCache; j++) {
+                // (past the end: the row's last vector again, which changes no maximum)
+                const int64_t k = min(b0 + ((int64_t)j * kSvNT + tid) * V, a.K - V);
+                sieve_load<DT, V>(a.w, base + k, t[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < kSvCache; j++)
+#pragma unroll
+                for (int e = 0; e < V; e++) {
+                    m = sieve_max_nan(m, fabsf(t[j][e]));
+                    if (b0 == 0) w[j][e] = t[j][e];
+                }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) m = sieve_max_nan(m, __shfl_xor(m, off, 64));
+        if ((tid & 63) == 0) red[par][tid >> 6] = m;
+        __syncthreads();  // (the other copy is written next, after every wave has read this one)
+        m = red[par][0];
+#pragma unroll
+        for (int i = 1; i < kSvNT / 64; i++) m = sieve_max_nan(m, red[par][i]);
+        // clamp(min=1e-8): the bound in w's dtype (0 in FP16), NaN kept
+        const float lo = round_as(DT, 1e-8f);
+        const float mc = (m != m) ? m : fmaxf(m, lo);
+        const float s = round_as(DT, sieve_scalar_div(mc, 7.0f, a.ieee_div));
+        for (int64_t b0 = 0; b0 < a.K; b0 += (int64_t)kSvCache * kSvNT * V) {
+#pragma unroll
+            for (int j = 0; j < kSvCache; j++) {
+                const int64_t k = b0 + ((int64_t)j * kSvNT + tid) * V;
+                if (k >= a.K) continue;
+                if (b0 > 0) sieve_load<DT, V>(a.w, base + k, w[j]);
+                float wb[V], sc[V];
+#pragma unroll
+                for (int e = 0; e < V; e++) {
+                    float t = rintf(round_as(DT, w[j][e] / s));
+                    t = (t != t) ? t : fminf(fmaxf(t, -8.f), 7.f);
+                    wb[e] = round_as(DT, sieve_mul(t, s));
+                    if (!__builtin_isfinite(wb[e])) wb[e] = 0.f;
+                }
+                sieve_store<DT, V>(a.w_base, base + k, wb);
+                if (a.score) {
+#pragma unroll
+                    for (int e = 0; e < V; e++) {
+                        float rr;
+                        sc[e] = sieve_score<DT, S32>(w[j][e], wb[e], sieve_h<HL>(a, hs, k + e), s16, rr);
+                        if (count) atomicAdd(&mine[sieve_key(sc[e]) >> 21], 1u);
+                    }
+                    sieve_store<ORTH_DT_F32, V>(a.score, base + k, sc);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // one vector's divisions at a time: registers
+            }
+        }
+    }
+    if (count) {
+        __syncthreads();
+        for (int i = tid; i < kSelBins; i += kSvNT) {
+            uint32_t c = 0;
+#pragma unroll
+            for (int l = 0; l < kSvLanes; l++) c += hist[l * kSelBins + i];
+            if (c) atomicAdd(&a.sel->hist[0][blockIdx.x % kSelCopies][i], c);
+        }
+    }
+}
+
+// Workgroup b takes scores [b seg, b seg + seg): counts the next 11 key bits
+// of those of the found prefix and lists their keys in its part of `list`
+// (cap keys; more: the last pass reads the scores again).
+template <int V>
+__global__ void __launch_bounds__(kSvNT) sieve_collect_kernel(const float *score, int64_t n, int64_t seg,
+                                                              SieveSel *st, uint32_t rank, uint32_t *list,
+                                                              int64_t cap) {
+    __shared__ uint32_t h[kSelBins];
+    __shared__ int32_t cnt;
+    const int tid = threadIdx.x, lane = tid & 63;
+    for (int i = tid; i < kSelBins; i += kSvNT) h[i] = 0u;
+    if (tid == 0) cnt = 0;
+    uint32_t bin, left;
+    sieve_pick(st, 0, rank, bin, left);
+    const int64_t i0 = (int64_t)blockIdx.x * seg, i1 = min(n, i0 + seg);
+    uint32_t *out = list + (int64_t)blockIdx.x * cap;
+    constexpr int U = 4;
+    for (int64_t ib = i0 + (int64_t)tid * V; ib < i1; ib += (int64_t)U * kSvNT * V) {
+        float v[U][V];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t i = ib + (int64_t)u * kSvNT * V;
+            if (i < i1) sieve_load<ORTH_DT_F32, V>(score, i, v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (ib + (int64_t)u * kSvNT * V >= i1) continue;
+#pragma unroll
+            for (int e = 0; e < V; e++) {
+                const uint32_t key = sieve_key(v[u][e]);
+                if ((key >> 21) == bin) {
+                    atomicAdd(&h[(key >> 10) & (kSelBins - 1)], 1u);
+                    const int32_t at = atomicAdd(&cnt, 1);
+                    if (at < cap) out[at] = key;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < kSelBins; i += kSvNT)
+        if (h[i]) atomicAdd(&st->hist[1][blockIdx.x % kSelCopies][i], h[i]);
+    if (tid == 0) st->count[blockIdx.x] = cnt <= cap ? cnt : -1;
+}
+
+// The last 10 key bits of the scores that share the 22 found.
+__global__ void __launch_bounds__(kSvNT) sieve_refine_kernel(const float *score, int64_t n, int64_t seg, SieveSel *st,
+                                                             const uint32_t *list, int64_t cap) {
+    __shared__ uint32_t h[1024];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < 1024; i += kSvNT) h[i] = 0u;
+    uint32_t bin, left;
+    sieve_pick(st, 1, st->left[0], bin, left);
+    const uint32_t prefix = (st->bin[0] << 11) | bin;
+    const int32_t cnt = st->count[blockIdx.x];
+    if (cnt >= 0) {
+        const uint32_t *in = list + (int64_t)blockIdx.x * cap;
+        for (int i = tid; i < cnt; i += kSvNT) {
+            const uint32_t key = in[i];
+            if ((key >> 10) == prefix) atomicAdd(&h[key & 1023u], 1u);
+        }
+    } else {
+        const int64_t i0 = (int64_t)blockIdx.x * seg, i1 = min(n, i0 + seg);
+        for (int64_t i = i0 + tid; i < i1; i += kSvNT) {
+            const uint32_t key = sieve_key(score[i]);
+            if ((key >> 10) == prefix) atomicAdd(&h[key & 1023u], 1u);
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < 1024; i += kSvNT)
+        if (h[i]) atomicAdd(&st->hist[2][blockIdx.x % kSelCopies][i], h[i]);
+}
+
+// w_ortho = residual * (score > t): t the selected k-th largest score or the
+// caller's threshold rounded to the score's dtype (torch compares a tensor
+// with a host scalar in the tensor's dtype); NaN compares false.  Both are
+// formed again from w and w_base: the residual is not stored in between.
+template <int DT, int V, bool HL, bool S32>
+__global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4))) sieve_mask_kernel(SieveArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    float *hs = reinterpret_cast<float *>(smem);
+    const int tid = threadIdx.x;
+    sieve_stage_h<HL>(a, hs);
+    const bool s16 = a.score_dt == ORTH_DT_F16;
+    float t = round_as(a.score_dt, a.thresh);
+    if (a.sel) {
+        uint32_t bin, left;
+        sieve_pick(a.sel, 2, a.sel->left[1], bin, left);
+        t = sieve_unkey((a.sel->bin[0] << 21) | (a.sel->bin[1] << 10) | bin);
+    }
+    __syncthreads();
+    for (int64_t r = blockIdx.x; r < a.N; r += gridDim.x) {
+        const int64_t base = r * a.K;
+        for (int64_t b0 = 0; b0 < a.K; b0 += (int64_t)kSvCache * kSvNT * V) {
+            float w[kSvCache][V], wb[kSvCache][V];
+#pragma unroll
+            for (int j = 0; j < kSvCache; j++) {
+                const int64_t k = min(b0 + ((int64_t)j * kSvNT + tid) * V, a.K - V);
+                sieve_load<DT, V>(a.w, base + k, w[j]);
+                sieve_load<DT, V>(a.w_base, base + k, wb[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < kSvCache; j++) {
+                const int64_t k = b0 + ((int64_t)j * kSvNT + tid) * V;
+                if (k >= a.K) continue;
+                float o[V];
+#pragma unroll
+                for (int e = 0; e < V; e++) {
+                    float rr;
+                    const float sc = sieve_score<DT, S32>(w[j][e], wb[j][e], sieve_h<HL>(a, hs, k + e), s16, rr);
+                    o[e] = sieve_mul(rr, sc > t ? 1.f : 0.f);
+                }
+                sieve_store<DT, V>(a.w_ortho, base + k, o);
+                __builtin_amdgcn_sched_barrier(0);  // (as above)
+            }
+        }
     }
 }
 
@@ -198,9 +450,74 @@ __global__ void __launch_bounds__(kSieveNT) sieve_hdiag_final_kernel(const float
     store_from_f32(out, dt, k, round_as(dt, q + 1e-6f));
 }
 
-static unsigned sieve_grid(int64_t n) {
-    const int64_t b = (n + kSieveNT - 1) / kSieveNT;
-    return (unsigned)(b < 4096 ? (b > 0 ? b : 1) : 4096);
+// 4 elements per load where every row of the four arrays starts aligned.
+static bool sieve_vec(const SieveArgs &a, int dt) {
+    const int64_t al = dt == ORTH_DT_F32 ? 16 : 8;
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.w_base) |
+                        reinterpret_cast<uintptr_t>(a.w_ortho);
+    return a.K % 4 == 0 && p % al == 0 && reinterpret_cast<uintptr_t>(a.score) % 16 == 0;
+}
+
+template <int DT, int V, bool HL, bool S32>
+static hipError_t sieve_launch_t(const SieveArgs &a, hipStream_t stream) {
+    const int64_t n = a.N * a.K;
+    const unsigned rows = (unsigned)(a.N < kSelWgs ? a.N : kSelWgs);
+    const uint32_t hb = HL ? (uint32_t)a.K * 4 : 0;
+    // more than 64 KB of dynamic LDS must be allowed once per device (the
+    // attribute call is idempotent, so two threads racing to set it is harmless)
+    static std::atomic<int> allowed[64];
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev >= 0 && dev < 64 && !allowed[dev].load(std::memory_order_acquire)) {
+        const int most = kSvLdsCols * 4 + kSvLanes * kSelBins * 4;
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(sieve_quant_kernel<DT, V, HL, S32>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, most);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void *>(sieve_mask_kernel<DT, V, HL, S32>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, most);
+        if (e != hipSuccess) return e;
+        allowed[dev].store(1, std::memory_order_release);
+    }
+    if (a.sel)
+        hipLaunchKernelGGL(sieve_sel_init_kernel, dim3(3 * kSelCopies * kSelBins / 256), dim3(256), 0, stream, a.sel);
+    hipLaunchKernelGGL((sieve_quant_kernel<DT, V, HL, S32>), dim3(rows), dim3(kSvNT),
+                       hb + (a.sel ? kSvLanes * kSelBins * 4 : 0), stream, a);
+    if (!a.w_ortho) return hipGetLastError();
+    if (a.sel) {
+        // segments of whole vectors; their keys' list is the w_ortho buffer,
+        // which the last pass overwrites
+        const int64_t seg = ((n + kSelWgs - 1) / kSelWgs + 3) & ~int64_t(3);
+        const unsigned wgs = (unsigned)((n + seg - 1) / seg);
+        uint32_t *list = static_cast<uint32_t *>(a.w_ortho);
+        const int64_t cap = reinterpret_cast<uintptr_t>(a.w_ortho) % 4 == 0 ? n * (DT == ORTH_DT_F32 ? 4 : 2) / 4 / kSelWgs : 0;
+        if (n % 4 == 0 && reinterpret_cast<uintptr_t>(a.score) % 16 == 0)
+            hipLaunchKernelGGL((sieve_collect_kernel<4>), dim3(wgs), dim3(kSvNT), 0, stream, a.score, n, seg, a.sel,
+                               a.rank, list, cap);
+        else
+            hipLaunchKernelGGL((sieve_collect_kernel<1>), dim3(wgs), dim3(kSvNT), 0, stream, a.score, n, seg, a.sel,
+                               a.rank, list, cap);
+        hipLaunchKernelGGL(sieve_refine_kernel, dim3(wgs), dim3(kSvNT), 0, stream, a.score, n, seg, a.sel, list, cap);
+    }
+    hipLaunchKernelGGL((sieve_mask_kernel<DT, V, HL, S32>), dim3(rows), dim3(kSvNT), hb, stream, a);
+    return hipGetLastError();
+}
+
+template <int DT, bool S32>
+static hipError_t sieve_launch_s(const SieveArgs &a, hipStream_t stream) {
+    if (a.K > kSvLdsCols) return sieve_launch_t<DT, 1, false, S32>(a, stream);
+    return sieve_vec(a, DT) ? sieve_launch_t<DT, 4, true, S32>(a, stream) : sieve_launch_t<DT, 1, true, S32>(a, stream);
+}
+
+template <int DT>
+static hipError_t sieve_launch_d(const SieveArgs &a, hipStream_t stream) {
+    return a.score_dt == ORTH_DT_F32 ? sieve_launch_s<DT, true>(a, stream) : sieve_launch_s<DT, false>(a, stream);
+}
+
+static hipError_t sieve_launch(const SieveArgs &a, int dt, hipStream_t stream) {
+    if (dt == ORTH_DT_F32) return sieve_launch_d<ORTH_DT_F32>(a, stream);
+    if (dt == ORTH_DT_F16) return sieve_launch_d<ORTH_DT_F16>(a, stream);
+    return sieve_launch_d<ORTH_DT_BF16>(a, stream);
 }
 
 hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, void *w_base, int ieee_div,
@@ -208,12 +525,11 @@ hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, vo
     SieveArgs a{};
     a.ieee_div = ieee_div;
     a.w = w;
-    a.dt = dt;
     a.N = N;
     a.K = K;
     a.w_base = w_base;
-    hipLaunchKernelGGL(sieve_quant_kernel, dim3((unsigned)N), dim3(kSieveNT), 0, stream, a);
-    return hipGetLastError();
+    a.score_dt = ORTH_DT_F32;  // (no score is formed)
+    return sieve_launch(a, dt, stream);
 }
 
 hipError_t launch_sieve_split(const void *w, int dt, int64_t N, int64_t K, const void *h, int hdt, int64_t h_stride,
@@ -222,37 +538,20 @@ hipError_t launch_sieve_split(const void *w, int dt, int64_t N, int64_t K, const
     SieveArgs a{};
     a.ieee_div = ieee_div;
     a.w = w;
-    a.dt = dt;
     a.N = N;
     a.K = K;
     a.w_base = w_base;
-    a.resid = w_ortho;
+    a.w_ortho = w_ortho;
     a.score = score;
     a.h = h;
     a.hdt = hdt;
     a.h_stride = h_stride;
     a.score_dt = score_dt;
-    hipLaunchKernelGGL(sieve_quant_kernel, dim3((unsigned)N), dim3(kSieveNT), 0, stream, a);
-    const int64_t n = N * K;
-    SieveSel *st = static_cast<SieveSel *>(sel);
-    int from_sel = 0;
-    if (use_rank) {
-        if (rank > 0) {
-            hipLaunchKernelGGL(sieve_sel_init_kernel, dim3(1), dim3(256), 0, stream, st, (uint32_t)rank);
-            for (int shift = 24; shift >= 0; shift -= 8) {
-                hipLaunchKernelGGL(sieve_hist_kernel, dim3(sieve_grid(n)), dim3(kSieveNT), 0, stream, score, n, st,
-                                   shift);
-                hipLaunchKernelGGL(sieve_pick_kernel, dim3(1), dim3(256), 0, stream, st, shift);
-            }
-            from_sel = 1;
-        } else {
-            // k == 0: the reference keeps nothing (threshold max + 1)
-            thresh = __builtin_nanf("");
-        }
-    }
-    hipLaunchKernelGGL(sieve_mask_kernel, dim3(sieve_grid(n)), dim3(kSieveNT), 0, stream, w_ortho, dt, score, n,
-                       st, from_sel, thresh, score_dt);
-    return hipGetLastError();
+    a.sel = use_rank && rank > 0 ? static_cast<SieveSel *>(sel) : nullptr;
+    a.rank = (uint32_t)rank;
+    // rank 0: the reference keeps nothing (threshold max + 1)
+    a.thresh = use_rank ? __builtin_nanf("") : thresh;
+    return sieve_launch(a, dt, stream);
 }
 
 int64_t sieve_hdiag_slices(int64_t n) {

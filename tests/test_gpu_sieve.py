@@ -99,6 +99,28 @@ def test_hessian_sieve_matches_oracle(gpu, dt, hdt, target):
     assert bits_equal(wo, torch.from_numpy(wo_o))
 
 
+@pytest.mark.parametrize("dt,hdt,N,K,target,tied", [
+    ("f32", "f32", 2100, 260, 0.02, False),    # more rows than workgroups
+    ("f16", "f32", 1500, 1027, 0.3, False),    # rows that start unaligned: one element a load
+    ("bf16", "bf16", 1030, 2052, 0.02, False),
+    ("f16", "f32", 24, 16388, 0.01, False),    # more columns than the workgroup's LDS holds of h
+    ("f32", "f32", 20, 16384, 0.02, False),    # as many; several register blocks per row
+    ("f16", "f32", 1100, 512, 0.4, True),      # one score everywhere: more collected keys than a 16-bit
+    ("f32", "f32", 1100, 512, 0.4, True)])     # w_ortho's part of the list holds, or as many
+def test_hessian_sieve_select_edges(gpu, dt, hdt, N, K, target, tied):
+    from libortho_amd.tools.sieve import hessian_sieve
+    w = make_w(dt, N, K, seed=5, device=gpu)
+    h = (torch.rand(K, generator=torch.Generator().manual_seed(6)) + 0.1).to(TD[hdt]).to(gpu)
+    if tied:
+        w = torch.full((N, K), 2.0 ** -7)
+        w[:, 0] = 7 * 2.0 ** -5
+        w, h = w.to(TD[dt]).to(gpu), torch.ones(K, dtype=TD[hdt], device=gpu)
+    wb, wo = hessian_sieve(w, h, sparsity_target=target)
+    wb_o, wo_o, _ = SO.hessian_sieve(w.float().cpu().numpy(), dt, h.float().cpu().numpy(), hdt, sparsity_target=target)
+    assert bits_equal(wb, torch.from_numpy(wb_o))
+    assert bits_equal(wo, torch.from_numpy(wo_o))
+
+
 def test_hessian_sieve_matrix_h_and_ties(gpu):
     """H_inv given as a matrix (its diagonal is used) and a score with many
     exact ties at the threshold (the k-th largest value is the same whatever

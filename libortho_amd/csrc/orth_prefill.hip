@@ -161,73 +161,100 @@ __device__ __forceinline__ uint32_t value_bits_f16(const void *vals, int dtype, 
     return __builtin_bit_cast(uint16_t, (f16)v);
 }
 
+constexpr int kPlanNT = 1024;
+constexpr int kPlanWRows = kPlanBN / (kPlanNT / 64);  // rows per wave
+
 // One workgroup per block of kPlanBN output rows.  Counting sort of the
-// block's CSR entries by 64-column step, stable in (row, CSR position).
-__global__ void __launch_bounds__(256) plan_build_kernel(ForwardArgs a, PlanHeader *h,
-                                                         int32_t *offsets, uint32_t *entries,
-                                                         uint16_t *chunks, int nksteps) {
-    extern __shared__ __align__(16) int32_t cnt[];  // [nksteps][BN], then partials[256]
-    int32_t *partials = cnt + nksteps * kPlanBN;
+// block's CSR entries by 64-column step, stable in (row, CSR position).  A
+// wave takes 8 rows, 64 entries of a row at a time: in a row whose columns
+// ascend strictly the entries of a step are consecutive, so an entry's place
+// among them is its distance from the first.  Other rows are walked entry by
+// entry by one lane.  (Each row walked by one thread, three times, with the
+// chunk table on the way: 72 us for 4096 -> 11008 at 1 %.)
+__global__ void __launch_bounds__(kPlanNT) plan_build_kernel(ForwardArgs a, PlanHeader *h,
+                                                             int32_t *offsets, uint32_t *entries, int nksteps) {
+    extern __shared__ __align__(16) int32_t cnt[];  // [nksteps][BN]
+    __shared__ int32_t wtot[kPlanNT / 64];
     __shared__ int32_t s_flags;
-    __shared__ int32_t s_total;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t b = blockIdx.x;
     const int L = nksteps * kPlanBN;
-    for (int i = tid; i < L; i += 256) cnt[i] = 0;
+    for (int i = tid; i < L; i += kPlanNT) cnt[i] = 0;
     if (tid == 0) s_flags = 0;
-    __syncthreads();
 
-    const int r = tid;
-    const int64_t n = b * kPlanBN + r;
-    int32_t rs = 0, re = 0;
+    // the rows' ranges (row_ptr of rows 8 w .. 8 w + 8 in lanes 0 .. 8) and first 64 columns
+    const int64_t n0 = b * kPlanBN + wave * kPlanWRows;
+    const int32_t rp = a.row_ptr[min(n0 + min(lane, kPlanWRows), a.N)];
     uint32_t myflags = 0;
-    if (r < kPlanBN && n < a.N) {
-        const int64_t ra = a.row_ptr[n], rb = a.row_ptr[n + 1];
-        if (ra < 0 || rb < ra || rb > a.nnz) myflags |= kPlanMalformed;
-        csr_row_range(a.row_ptr, n, a.nnz, rs, re);
-        int32_t prev = -1, praw = INT32_MIN;
-        const int nch = chunks ? (int)(a.K / 128) : 0;
-        uint16_t *crow = chunks ? chunks + n * (int64_t)(nch + 1) : nullptr;
-        int cnext = 0;  // next chunk boundary to record
-        for (int32_t j = rs; j < re; j++) {
-            const int32_t c = a.col[j];
-            if (c <= praw) myflags |= kPlanUnsorted;
-            praw = c;
-            // boundaries 128 cb <= c end before entry j (meaningful when sorted)
-            if (crow)
-                for (; cnext <= nch && (int64_t)cnext * 128 <= (int64_t)c; cnext++)
-                    crow[cnext] = (uint16_t)min(j - rs, 65535);
-            if (c >= 0 && c < a.K) {
-                cnt[(c / kPlanBK) * kPlanBN + r] += 1;
-                if (c <= prev) myflags |= kPlanNonCanonical;
-                prev = c;
+    int32_t rs[kPlanWRows], re[kPlanWRows], c0[kPlanWRows];
+#pragma unroll
+    for (int i = 0; i < kPlanWRows; i++) {
+        const int32_t ra = __shfl(rp, i), rb = __shfl(rp, i + 1), nnz = (int32_t)a.nnz;
+        const bool live = n0 + i < a.N;
+        if (live && (ra < 0 || rb < ra || rb > nnz)) myflags |= kPlanMalformed;
+        rs[i] = min(max(ra, 0), nnz);  // (csr_row_range)
+        re[i] = live ? min(max(rb, rs[i]), nnz) : rs[i];
+        c0[i] = a.col[min((int64_t)rs[i] + lane, (int64_t)max(re[i] - 1, 0))];
+        if (re[i] - rs[i] > 65535) myflags |= kPlanUnsorted;  // counts past 16 bits
+    }
+    __syncthreads();  // the counters are zero
+
+    uint32_t slow = 0;  // rows whose columns do not ascend strictly (uniform)
+#pragma unroll
+    for (int i = 0; i < kPlanWRows; i++) {
+        const int r = wave * kPlanWRows + i;
+        bool bad = false;
+        int32_t last = INT32_MIN;
+        for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
+            const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
+            const int32_t up = __shfl_up(c, 1);
+            if (jb + lane < re[i] && c <= (lane ? up : last) && (lane || jb > rs[i])) bad = true;
+            last = __shfl(c, 63);
+        }
+        if (__ballot(bad)) {
+            slow |= 1u << i;
+            if (lane == 0) {
+                myflags |= kPlanUnsorted;
+                int32_t prev = -1;
+                for (int32_t j = rs[i]; j < re[i]; j++) {
+                    const int32_t c = a.col[j];
+                    if (c >= 0 && c < a.K) {
+                        cnt[(c / kPlanBK) * kPlanBN + r] += 1;
+                        if (c <= prev) myflags |= kPlanNonCanonical;
+                        prev = c;
+                    }
+                }
+            }
+        } else {
+            for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
+                const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
+                if (jb + lane < re[i] && c >= 0 && c < a.K) atomicAdd(&cnt[(c / kPlanBK) * kPlanBN + r], 1);
             }
         }
-        if (crow)
-            for (; cnext <= nch; cnext++) crow[cnext] = (uint16_t)min(re - rs, 65535);
-        if (re - rs > 65535) myflags |= kPlanUnsorted;  // counts past 16 bits
     }
     if (myflags) atomicOr(&s_flags, (int32_t)myflags);
     __syncthreads();
 
     // exclusive scan of cnt in (step, row) order: per-thread segments
-    const int seg = (L + 255) / 256;
-    const int lo = tid * seg, hi = min(L, lo + seg);
+    const int seg = (L + kPlanNT - 1) / kPlanNT;
+    const int lo = min(L, tid * seg), hi = min(L, lo + seg);
     int32_t local = 0;
     for (int i = lo; i < hi; i++) local += cnt[i];
-    partials[tid] = local;
-    __syncthreads();
-    if (tid == 0) {
-        int32_t run = 0;
-        for (int i = 0; i < 256; i++) {
-            const int32_t v = partials[i];
-            partials[i] = run;
-            run += v;
-        }
-        s_total = run;
+    int32_t incl = local;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
     }
+    if (lane == 63) wtot[wave] = incl;
     __syncthreads();
-    int32_t run = partials[tid];
+    int32_t run = incl - local, total = 0;
+#pragma unroll
+    for (int w = 0; w < kPlanNT / 64; w++) {
+        if (w < wave) run += wtot[w];
+        total += wtot[w];
+    }
     for (int i = lo; i < hi; i++) {
         const int32_t v = cnt[i];
         cnt[i] = run;
@@ -241,22 +268,42 @@ __global__ void __launch_bounds__(256) plan_build_kernel(ForwardArgs a, PlanHead
     int64_t base = a.row_ptr[nfirst], end = a.row_ptr[nlast];
     base = base < 0 ? 0 : (base > a.nnz ? a.nnz : base);
     end = end < base ? base : (end > a.nnz ? a.nnz : end);
-    const int64_t total = s_total;
     const bool fits = base + total <= end;
     int32_t *off = offsets + b * (nksteps + 1);
-    for (int kt = tid; kt <= nksteps; kt += 256) {
+    for (int kt = tid; kt <= nksteps; kt += kPlanNT) {
         int64_t o = kt < nksteps ? cnt[kt * kPlanBN] : total;
         off[kt] = (int32_t)(base + (fits ? o : 0));
     }
-    __syncthreads();  // the placement below advances the same counters
-    if (fits && r < kPlanBN && n < a.N) {
-        for (int32_t j = rs; j < re; j++) {
-            const int32_t c = a.col[j];
-            if (c >= 0 && c < a.K) {
-                const int kt = c / kPlanBK;
-                const int32_t pos = cnt[kt * kPlanBN + r]++;
-                entries[base + pos] = ((uint32_t)r << 24) | ((uint32_t)(c - kt * kPlanBK) << 16) |
+    __syncthreads();  // the walk of the unsorted rows below advances the same counters
+    if (fits) {
+#pragma unroll
+        for (int i = 0; i < kPlanWRows; i++) {
+            const int r = wave * kPlanWRows + i;
+            auto put = [&](int32_t pos, int32_t c, int64_t j) {
+                entries[base + pos] = ((uint32_t)r << 24) | ((uint32_t)(c & (kPlanBK - 1)) << 16) |
                                       value_bits_f16(a.vals, a.val_dtype, j);
+            };
+            if (slow & (1u << i)) {
+                if (lane == 0)
+                    for (int32_t j = rs[i]; j < re[i]; j++) {
+                        const int32_t c = a.col[j];
+                        if (c >= 0 && c < a.K) put(cnt[(c / kPlanBK) * kPlanBN + r]++, c, j);
+                    }
+                continue;
+            }
+            int64_t first = rs[i];       // the first entry of the last step so far
+            int32_t last = INT32_MIN;    // and that step
+            for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
+                const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
+                const bool ok = jb + lane < re[i] && c >= 0 && c < a.K;
+                const int32_t kt = c >> 6;  // (negative or past K: a step of its own, not written)
+                const int32_t up = __shfl_up(kt, 1);
+                const uint64_t heads = __ballot(kt != (lane ? up : last));
+                const uint64_t below = heads & (~0ull >> (63 - lane));
+                const int64_t f = below ? jb + (63 - __builtin_clzll(below)) : first;
+                if (ok) put(cnt[kt * kPlanBN + r] + (int32_t)(jb + lane - f), c, jb + lane);
+                first = __shfl((int)(f - rs[i]), 63) + (int64_t)rs[i];
+                last = __shfl(kt, 63);
             }
         }
     }
@@ -266,56 +313,177 @@ __global__ void __launch_bounds__(256) plan_build_kernel(ForwardArgs a, PlanHead
     }
 }
 
-// One workgroup of 64 per (16-row group, cell) of `ncells` cells of
-// `cols` columns: thread r < 16 counts its row's entries of the cell, thread
-// 0 lays out the rows, then each thread writes its row's entries in CSR
-// order (those past the record are counted in header word 1).
-__global__ void __launch_bounds__(64) plan_cell_kernel(ForwardArgs a, uint32_t *out, int words, int ncells,
-                                                       int cols, uint32_t kind) {
-    __shared__ int32_t cnt[16], start[17];
-    const int64_t g = blockIdx.x / ncells;
-    const int c = (int)(blockIdx.x - g * ncells);
-    const int t = threadIdx.x;
-    uint32_t *rec = out + (g * ncells + c) * (int64_t)words;
-    const int cap = words - kCellHdrWords;
-    const int64_t c0 = (int64_t)c * cols, c1 = min(c0 + cols, a.K);
-    int32_t rs = 0, re = 0;
-    const int64_t n = g * 16 + t;
-    if (t < 16) {
-        if (n < a.N) csr_row_range(a.row_ptr, n, a.nnz, rs, re);
-        int32_t k = 0;
-        for (int32_t j = rs; j < re; j++) {
-            const int32_t cc = a.col[j];
-            k += (cc >= c0 && cc < c1) ? 1 : 0;
+// The chunk table and the cell records of a 16-row group (K % 128 == 0), one
+// workgroup each: the group's entries are staged in LDS with coalesced loads;
+// where every row's columns ascend (not necessarily strictly), a chunk's or a
+// cell's entries of a row are a run found by binary search, and the records
+// are written word by word.  Otherwise each row's entries are walked in CSR
+// order by one thread per row and cell.  (A workgroup of 64 per cell, whose
+// 16 row threads walked the CSR twice, took 28-35 us for each of the two
+// kinds of record of 4096 -> 11008 at 1 %.)
+constexpr int kPlanRowsNT = 256;
+constexpr int kPlanStage = 4096;     // entries of a group kept in LDS (more: read from memory)
+constexpr int kPlanMaxCells = 16;    // 4 quarters + 12 slices of at most 12,288 columns
+
+struct PlanRowsArgs {
+    uint16_t *chunks;
+    uint32_t *qrec, *srec;           // or null
+    int qwords, swords, nslices, qcols;
+};
+
+__global__ void __launch_bounds__(kPlanRowsNT) plan_rows_kernel(ForwardArgs a, PlanRowsArgs p) {
+    __shared__ int32_t col_s[kPlanStage];
+    __shared__ uint16_t val_s[kPlanStage];
+    __shared__ int32_t tab[16][kPlanMaxK / 128 + 1];
+    __shared__ int32_t rs[16], re[16], start[kPlanMaxCells][17], span[2];
+    const int tid = threadIdx.x;
+    const int64_t g = blockIdx.x;
+    const int r = tid >> 4, l = tid & 15;  // 16 lanes per row
+    const int nch = (int)(a.K / 128);
+    if (tid < 16) {
+        int32_t s = 0, e = 0;
+        if (g * 16 + tid < a.N) csr_row_range(a.row_ptr, g * 16 + tid, a.nnz, s, e);
+        rs[tid] = s;
+        re[tid] = e;
+        int32_t mn = e > s ? s : INT32_MAX, mx = e > s ? e : 0;
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            mn = min(mn, __shfl_xor(mn, off));
+            mx = max(mx, __shfl_xor(mx, off));
         }
-        cnt[t] = k;
+        if (tid == 0) {
+            span[0] = mn;
+            span[1] = mx;
+        }
     }
     __syncthreads();
-    if (t == 0) {
-        int32_t run = 0;
-        for (int r = 0; r < 16; r++) {
-            start[r] = run;
-            run += cnt[r];
+    const int32_t gmin = span[0];
+    const int64_t many = (int64_t)span[1] - gmin;  // (negative: no entries)
+    const bool staged = many <= kPlanStage;         // (uniform)
+    if (staged) {
+        for (int i = tid; i < many; i += kPlanRowsNT) {
+            col_s[i] = a.col[gmin + i];
+            val_s[i] = (uint16_t)value_bits_f16(a.vals, a.val_dtype, gmin + i);
         }
-        start[16] = run;
-        rec[0] = plan_cell_tag(kind, a.N, a.K, a.nnz, words, g, c);
-        rec[1] = (uint32_t)(run > cap ? run - cap : 0);
-        rec[18] = rec[19] = 0u;
+        __syncthreads();
     }
-    __syncthreads();
-    for (int i = t; i < cap; i += 64) rec[kCellHdrWords + i] = 0xffffu;
-    __syncthreads();
-    if (t < 16) {
-        const int32_t b = min(start[t], cap), e = min(start[t + 1], cap);
-        rec[2 + t] = (uint32_t)b | ((uint32_t)e << 16);
-        int32_t w = start[t];
-        for (int32_t j = rs; j < re; j++) {
-            const int32_t cc = a.col[j];
-            if (cc >= c0 && cc < c1) {
-                if (w < cap) rec[kCellHdrWords + w] = (uint32_t)(cc - c0) | (value_bits_f16(a.vals, a.val_dtype, j) << 16);
-                w++;
+    auto col = [&](int32_t j) -> int32_t { return staged ? col_s[j - gmin] : a.col[j]; };
+    auto val = [&](int32_t j) -> uint32_t { return staged ? (uint32_t)val_s[j - gmin] : value_bits_f16(a.vals, a.val_dtype, j); };
+    int bad = 0;
+    for (int32_t j = rs[r] + 1 + l; j < re[r]; j += 16) bad |= col(j) < col(j - 1) ? 1 : 0;
+    const bool sorted = __syncthreads_or(bad) == 0;
+    const int ncq = p.qrec ? 4 : 0, ncells = ncq + (p.srec ? p.nslices : 0);
+    // cell ci's first column, width, record and tag kind
+    auto cell_c0 = [&](int ci) -> int64_t { return ci < ncq ? (int64_t)ci * p.qcols : (int64_t)(ci - ncq) * 1024; };
+    auto cell_cols = [&](int ci) -> int { return ci < ncq ? p.qcols : 1024; };
+    auto cell_words = [&](int ci) -> int { return ci < ncq ? p.qwords : p.swords; };
+    auto cell_rec = [&](int ci) -> uint32_t * {
+        return ci < ncq ? p.qrec + (g * 4 + ci) * (int64_t)p.qwords : p.srec + (g * p.nslices + ci - ncq) * (int64_t)p.swords;
+    };
+    auto cell_tag = [&](int ci) -> uint32_t {
+        return plan_cell_tag(ci < ncq ? kCellQuarter : kCellSlice, a.N, a.K, a.nnz, cell_words(ci), g, ci < ncq ? ci : ci - ncq);
+    };
+    if (sorted) {
+        for (int c = l; c <= nch; c += 16) {  // entries with column < 128 c
+            int32_t lo = rs[r], hi = re[r];
+            while (lo < hi) {
+                const int32_t mid = lo + ((hi - lo) >> 1);
+                if ((int64_t)col(mid) < (int64_t)128 * c) lo = mid + 1;
+                else hi = mid;
+            }
+            tab[r][c] = lo - rs[r];
+            if (p.chunks && g * 16 + r < a.N) p.chunks[(g * 16 + r) * (int64_t)(nch + 1) + c] = (uint16_t)min(lo - rs[r], 65535);
+        }
+        __syncthreads();
+        {
+            const int ci = r, row = l;  // 16 cells x 16 rows: the rows' starts within each cell
+            int32_t n = 0;
+            if (ci < ncells) {
+                const int lo = (int)min((int64_t)nch, cell_c0(ci) / 128);
+                n = tab[row][min(nch, lo + cell_cols(ci) / 128)] - tab[row][lo];
+            }
+            int32_t incl = n;
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) {
+                const int32_t v = __shfl_up(incl, off, 16);
+                if (row >= off) incl += v;
+            }
+            start[ci][row] = incl - n;
+            if (row == 15) start[ci][16] = incl;
+        }
+        __syncthreads();
+        for (int ci = 0; ci < ncells; ci++) {
+            const int words = cell_words(ci), cap = words - kCellHdrWords, total = start[ci][16];
+            uint32_t *rec = cell_rec(ci);
+            const int64_t c0 = cell_c0(ci);
+            const int ch0 = (int)min((int64_t)nch, c0 / 128);
+            for (int i = tid; i < words; i += kPlanRowsNT) {
+                uint32_t w = 0u;
+                if (i >= kCellHdrWords) {
+                    const int s = i - kCellHdrWords;
+                    w = 0xffffu;
+                    if (s < total) {
+                        int row = 0;  // the row whose run holds slot s
+#pragma unroll
+                        for (int step = 8; step > 0; step >>= 1)
+                            if (start[ci][row + step] <= s) row += step;
+                        const int32_t j = rs[row] + tab[row][ch0] + (s - start[ci][row]);
+                        w = (uint32_t)(col(j) - (int32_t)c0) | (val(j) << 16);
+                    }
+                } else if (i == 0) {
+                    w = cell_tag(ci);
+                } else if (i == 1) {
+                    w = (uint32_t)(total > cap ? total - cap : 0);
+                } else if (i < 18) {
+                    w = (uint32_t)min(start[ci][i - 2], cap) | ((uint32_t)min(start[ci][i - 1], cap) << 16);
+                }
+                rec[i] = w;
             }
         }
+        return;
+    }
+    // unsorted rows: the table as a walk meets the boundaries (read only where
+    // the rows ascend), and each cell's entries in CSR order
+    if (p.chunks && tid < 16 && g * 16 + tid < a.N) {
+        uint16_t *crow = p.chunks + (g * 16 + tid) * (int64_t)(nch + 1);
+        int cnext = 0;
+        for (int32_t j = rs[tid]; j < re[tid]; j++)
+            for (; cnext <= nch && (int64_t)cnext * 128 <= (int64_t)col(j); cnext++)
+                crow[cnext] = (uint16_t)min(j - rs[tid], 65535);
+        for (; cnext <= nch; cnext++) crow[cnext] = (uint16_t)min(re[tid] - rs[tid], 65535);
+    }
+    {
+        const int ci = r, row = l;
+        int32_t n = 0;
+        const int64_t c0 = cell_c0(ci), c1 = min(c0 + cell_cols(ci), a.K);
+        if (ci < ncells)
+            for (int32_t j = rs[row]; j < re[row]; j++) n += col(j) >= c0 && col(j) < c1 ? 1 : 0;
+        int32_t incl = n;
+#pragma unroll
+        for (int off = 1; off < 16; off <<= 1) {
+            const int32_t v = __shfl_up(incl, off, 16);
+            if (row >= off) incl += v;
+        }
+        start[ci][row] = incl - n;
+        if (row == 15) start[ci][16] = incl;
+        __syncthreads();
+        if (ci >= ncells) return;
+        const int cap = cell_words(ci) - kCellHdrWords;
+        uint32_t *rec = cell_rec(ci);
+        const int total = start[ci][16];
+        if (row == 0) {
+            rec[0] = cell_tag(ci);
+            rec[1] = (uint32_t)(total > cap ? total - cap : 0);
+            rec[18] = rec[19] = 0u;
+        }
+        rec[2 + row] = (uint32_t)min(incl - n, cap) | ((uint32_t)min(incl, cap) << 16);
+        int32_t w = incl - n;
+        for (int32_t j = rs[row]; j < re[row]; j++)
+            if (col(j) >= c0 && col(j) < c1) {
+                if (w < cap) rec[kCellHdrWords + w] = (uint32_t)(col(j) - (int32_t)c0) | (val(j) << 16);
+                w++;
+            }
+        for (int i = total + row; i < cap; i += 16) rec[kCellHdrWords + i] = 0xffffu;
     }
 }
 
@@ -330,23 +498,19 @@ hipError_t launch_plan_build(const ForwardArgs &a, void *plan, hipStream_t strea
     const int swords = plan_srec_words(a.N, a.K, a.nnz);
     hipLaunchKernelGGL(plan_init_kernel, dim3(1), dim3(64), 0, stream, h, nblocks, nksteps, a.N,
                        a.K, a.nnz, qwords, swords);
-    const size_t lds = ((size_t)nksteps * kPlanBN + 256) * sizeof(int32_t);
-    uint16_t *chunks = plan_chunks_bytes(a.N, a.K)
-                           ? reinterpret_cast<uint16_t *>(static_cast<char *>(plan) + plan_chunks_at(a.N, a.K, a.nnz))
-                           : nullptr;
-    hipLaunchKernelGGL(plan_build_kernel, dim3(nblocks), dim3(256), lds, stream, a, h, offsets,
-                       entries, chunks, nksteps);
-    const unsigned ngroups = (unsigned)((a.N + 15) / 16);
-    if (qwords > 0) {
-        uint32_t *qrec = reinterpret_cast<uint32_t *>(static_cast<char *>(plan) + plan_rec_at(a.N, a.K, a.nnz));
-        hipLaunchKernelGGL(plan_cell_kernel, dim3(ngroups * 4), dim3(64), 0, stream, a, qrec, qwords, 4,
-                           decode_chunks_per_wave(a.K) * 128, kCellQuarter);
-    }
-    if (swords > 0) {
-        const int nslices = (int)((a.K + 1023) / 1024);
-        uint32_t *srec = reinterpret_cast<uint32_t *>(static_cast<char *>(plan) + plan_srec_at(a.N, a.K, a.nnz));
-        hipLaunchKernelGGL(plan_cell_kernel, dim3(ngroups * (unsigned)nslices), dim3(64), 0, stream, a, srec,
-                           swords, nslices, 1024, kCellSlice);
+    const size_t lds = (size_t)nksteps * kPlanBN * sizeof(int32_t);
+    hipLaunchKernelGGL(plan_build_kernel, dim3(nblocks), dim3(kPlanNT), lds, stream, a, h, offsets, entries, nksteps);
+    if (plan_chunks_bytes(a.N, a.K)) {
+        char *base = static_cast<char *>(plan);
+        PlanRowsArgs p;
+        p.chunks = reinterpret_cast<uint16_t *>(base + plan_chunks_at(a.N, a.K, a.nnz));
+        p.qrec = qwords > 0 ? reinterpret_cast<uint32_t *>(base + plan_rec_at(a.N, a.K, a.nnz)) : nullptr;
+        p.srec = swords > 0 ? reinterpret_cast<uint32_t *>(base + plan_srec_at(a.N, a.K, a.nnz)) : nullptr;
+        p.qwords = qwords;
+        p.swords = swords;
+        p.nslices = (int)((a.K + 1023) / 1024);
+        p.qcols = decode_chunks_per_wave(a.K) * 128;
+        hipLaunchKernelGGL(plan_rows_kernel, dim3((unsigned)((a.N + 15) / 16)), dim3(kPlanRowsNT), 0, stream, a, p);
     }
     return hipGetLastError();
 }
@@ -367,9 +531,8 @@ hipError_t launch_plan_build_prefill(const ForwardArgs &a, void *plan, hipStream
     uint32_t *entries = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(offsets) +
                                                      plan_offsets_bytes(a.N, a.K));
     hipLaunchKernelGGL(plan_init_kernel, dim3(1), dim3(64), 0, stream, h, nblocks, nksteps, a.N, a.K, a.nnz, 0, 0);
-    const size_t lds = ((size_t)nksteps * kPlanBN + 256) * sizeof(int32_t);
-    hipLaunchKernelGGL(plan_build_kernel, dim3(nblocks), dim3(256), lds, stream, a, h, offsets, entries,
-                       static_cast<uint16_t *>(nullptr), nksteps);
+    const size_t lds = (size_t)nksteps * kPlanBN * sizeof(int32_t);
+    hipLaunchKernelGGL(plan_build_kernel, dim3(nblocks), dim3(kPlanNT), lds, stream, a, h, offsets, entries, nksteps);
     return hipGetLastError();
 }
 

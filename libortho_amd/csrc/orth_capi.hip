@@ -64,6 +64,7 @@ hipError_t launch_split_group(const ForwardArgs *as, const void *const *plans, i
                               hipStream_t stream);
 hipError_t launch_mid(const ForwardArgs &a, const void *plan, int cus, hipStream_t stream);
 bool skinny_supported(const ForwardArgs &a);
+bool skinny_wide_k_preferred(const ForwardArgs &a, int cus);
 int64_t skinny_workspace_bytes(const ForwardArgs &a, int cus);
 hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float *part, hipStream_t stream);
 hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, void *w_base, int ieee_div,
@@ -402,11 +403,12 @@ int pick_kernel(const ForwardArgs &a, const void *plan, int policy, int cus, int
             // BF16 with 512-word records): c5 down_proj M=32 23.7 against
             // 35.5 us for the split-K kernel
             else if (sp_ok && a.M > 16) *kernel = KERNEL_SPLIT;
-            // 33..64 tokens at K > 4096: the prefill kernel with K split
-            // over the grid (c5 down_proj, K = 11008: 35-37 against 44-53
-            // us on the split-K kernel at 33-64 tokens; at K = 4096 the
-            // split-K kernel is level or ahead: c2 M=48 35.8 against 42.4)
-            else if (pre_ok && a.M > 32 && a.K > 4096 && prefill_split(a, plan, cus) > 1) *kernel = KERNEL_PREFILL;
+            // 33..64 tokens at K > 4096: the prefill kernel with K split over
+            // the grid, unless the split-K kernel is faster there (at K = 4096
+            // it is level or ahead: c2 M=48 26.5 against 41.6)
+            else if (pre_ok && a.M > 32 && a.K > 4096 && prefill_split(a, plan, cus) > 1 &&
+                     !(sk_ok && skinny_wide_k_preferred(a, cus)))
+                *kernel = KERNEL_PREFILL;
             else if (sk_pref) *kernel = KERNEL_SKINNY;
             else if (dec_ok) *kernel = KERNEL_DECODE;
             // (the 256 x 128 kernel where it splits K: c3 at 512 or 1024

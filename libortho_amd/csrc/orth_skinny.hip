@@ -25,11 +25,19 @@
 //    loads two of every eight entries, DPP quad broadcasts hand all eight to
 //    the four, each multiplies them with four tokens' staged activations
 //    (two up to 8 tokens: tokens past M are padding of the tile), and the
-//    sums reach the MFMA lanes through LDS.  From 17 tokens (more
-//    registers, and an LDS exchange would cost the second workgroup per CU)
-//    each lane takes the row and tokens of its own MFMA output and reads the
-//    row's entries itself.  Sums are formed in CSR order: the result does not
-//    depend on scheduling.
+//    sums reach the MFMA lanes through LDS.  Sums are formed in CSR order: the
+//    result does not depend on scheduling.
+//  * From 17 tokens, where K is split, the ortho term is a slice of its own:
+//    workgroups at the head of the grid (skinny_sparse) keep all columns of 8,
+//    4 or 2 tokens in LDS, [column][token], walk the CSR of a run of rows, 16
+//    lanes a row, one LDS read per entry for all the tokens, and write
+//    alpha * sum as one more partial; they run beside the dense workgroups.
+//    (Each lane reading its own MFMA output's entries, one two-byte LDS read
+//    per entry and token, cost as much as the dense term: 4096 -> 11008 at 48
+//    tokens, 1 %, 36.6 us against 18.6 at alpha = 0; now 26.8.)  It needs no
+//    plan.
+//    Without a K split (or where the extra partial would not fit the
+//    no-allocation scratch array) each lane still reads its own entries.
 //  * With the plan's slice records (one token tile, 8-chunk slices,
 //    K % 1024 == 0) each wave instead loads its 16 rows' record of the slice
 //    at entry (packed column | value words at an address that needs no other
@@ -102,7 +110,184 @@ struct SkinnyArgs {
     int lds_sr;          // SPK >= 3: per-wave record regions
     const void *bias;  // [N] added after rounding (out_f16), or null
     int bias_dtype;
+    // SPK 7: the ortho term's workgroups (a multiple of 8, ids first), the
+    // tokens each keeps (8, 4 or 2) and the number of token tiles
+    int sp_wgs, sp_tt, sp_tiles;
 };
+
+// ---- the ortho term of 17 .. 64 tokens as a slice of its own
+
+constexpr int kSsRows = 16;                // rows per unit (one wave's)
+constexpr int kSsLdsMax = 150 * 1024;
+
+// LDS byte offset of column c's TT tokens: 16 bytes of padding after every 8
+// columns (the staging lanes' writes spread over the banks).
+template <int TT>
+__device__ __forceinline__ int ss_col(int c) { return c * (2 * TT) + (c >> 3) * 16; }
+
+static int ss_lds(int64_t K, int tt) {
+    return (int)(K * 2 * tt + K / 8 * 16 + 16 + (kSkNT / 64) * kSsRows * tt * 4);
+}
+
+// Tokens per workgroup (0: K is too large).  As many as fit: every token tile
+// reads all of the CSR, which costs more than the second workgroup per CU
+// that a smaller tile would leave room for (8192 -> 4096 at 48 tokens: 24.7 us
+// with 8 tokens, 26.1 with 4).
+static int ss_tokens(int64_t K) {
+    for (int tt = 8; tt >= 2; tt /= 2)
+        if (K <= 65536 && ss_lds(K, tt) <= kSsLdsMax) return tt;
+    return 0;
+}
+
+template <int TT, bool XB>
+__device__ void skinny_sparse(const SkinnyArgs &a, unsigned char *smem) {
+    constexpr int U = 3;                               // batches of 16 entries of a row in flight
+    constexpr int PL = (TT * kSsRows + 63) / 64;       // outputs per lane of a unit
+    constexpr int W = TT / 2;                          // words of a column's tokens
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K = a.K;
+    const int m0 = (int)(blockIdx.x % (unsigned)a.sp_tiles) * TT;
+    const int wg = (int)(blockIdx.x / (unsigned)a.sp_tiles);
+    const int wgs = (a.sp_wgs + a.sp_tiles - 1 - (int)(blockIdx.x % (unsigned)a.sp_tiles)) / a.sp_tiles;  // of this tile
+    float *sums = reinterpret_cast<float *>(smem + ss_col<TT>(K) + 16) + wave * TT * kSsRows;  // [TT][16]
+    if (tid == 0) *reinterpret_cast<u32x4 *>(smem + ss_col<TT>(K)) = u32x4{0u, 0u, 0u, 0u};  // a zero column
+
+    // staging: a thread takes 8 columns of every token and turns them
+    for (int c8 = tid; c8 < K / 8; c8 += kSkNT) {
+        u32x4 x[TT];
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+            x[t] = *reinterpret_cast<const u32x4 *>(a.x + (int64_t)min(m0 + t, a.M - 1) * K + 8 * c8);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            uint32_t w[W];
+#pragma unroll
+            for (int u = 0; u < W; u++)
+                w[u] = __builtin_amdgcn_perm(x[2 * u + 1][j >> 1], x[2 * u][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+            unsigned char *dst = smem + ss_col<TT>(8 * c8 + j);
+            if constexpr (W == 4) *reinterpret_cast<u32x4 *>(dst) = u32x4{w[0], w[1], w[2], w[3]};
+            else if constexpr (W == 2) *reinterpret_cast<uint2 *>(dst) = uint2{w[0], w[1]};
+            else *reinterpret_cast<uint32_t *>(dst) = w[0];
+        }
+    }
+    __syncthreads();
+
+    const int sub = lane >> 4, l16 = lane & 15;  // row of a pass, lane of the row
+    const int64_t units = (a.N + kSsRows - 1) / kSsRows;
+    float *part = a.part + (int64_t)a.S * a.M * a.N;
+    // two units ahead: the row pointers; one ahead: the entries (a unit's
+    // loads would otherwise wait, one after the other, behind the dense
+    // workgroups' weights)
+    struct Unit {
+        int32_t js[4], je[4], c[4][U];
+        uint32_t v[4][U];
+    };
+    const int64_t step = (int64_t)wgs * (kSkNT / 64);
+    auto load = [&](int32_t je, int32_t jb, int32_t (&cc)[U], uint32_t (&vv)[U]) {
+        const int32_t last = min(max(je - 1, 0), a.nnz - 1);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int32_t j = min(jb + 16 * u + l16, last);
+            cc[u] = a.col[j];
+            vv[u] = __builtin_bit_cast(uint16_t, a.vals[j]);
+        }
+    };
+    auto pointers = [&](int64_t un) -> int32_t { return a.row_ptr[min(min(un, units - 1) * kSsRows + min(lane, kSsRows), a.N)]; };
+    auto begin = [&](int64_t un, int32_t rp, Unit &q) {
+        const int64_t r0 = min(un, units - 1) * kSsRows;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {  // (clamped as csr_row_range does)
+            q.js[p] = min(max(__shfl(rp, 4 * p + sub), 0), a.nnz);
+            q.je[p] = min(max(__shfl(rp, 4 * p + sub + 1), q.js[p]), a.nnz);
+            if (r0 + 4 * p + sub >= a.N) q.je[p] = q.js[p];
+        }
+#pragma unroll
+        for (int p = 0; p < 4; p++) load(q.je[p], q.js[p], q.c[p], q.v[p]);
+    };
+    int64_t un = (int64_t)wg * (kSkNT / 64) + wave;
+    Unit cur, nxt;
+    begin(un, pointers(un), nxt);
+    int32_t rp = pointers(un + step);
+    for (; un < units; un += step) {
+        cur = nxt;
+        begin(un + step, rp, nxt);
+        rp = pointers(un + 2 * step);
+        const int64_t r0 = un * kSsRows;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            float acc[TT];
+#pragma unroll
+            for (int t = 0; t < TT; t++) acc[t] = 0.f;
+            auto use = [&](int32_t jb, const int32_t (&cc)[U], const uint32_t (&vv)[U]) {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    // (an empty slot: the zero column past the last one, no branch)
+                    const bool ok = jb + 16 * u + l16 < cur.je[p] && cc[u] >= 0 && cc[u] < K;
+                    if (u > 0 && !__any(ok)) continue;  // (uniform)
+                    const float val = ok ? (float)__builtin_bit_cast(f16, (uint16_t)vv[u]) : 0.f;
+                    const unsigned char *src = smem + ss_col<TT>(ok ? cc[u] : K);
+                    uint32_t w[W];
+                    if constexpr (W == 4) {
+                        const u32x4 q = *reinterpret_cast<const u32x4 *>(src);
+                        w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+                    } else if constexpr (W == 2) {
+                        const uint2 q = *reinterpret_cast<const uint2 *>(src);
+                        w[0] = q.x; w[1] = q.y;
+                    } else {
+                        w[0] = *reinterpret_cast<const uint32_t *>(src);
+                    }
+#pragma unroll
+                    for (int t = 0; t < TT; t++)
+                        acc[t] = __builtin_fmaf(val, x16_to_f32<XB>(__builtin_bit_cast(f16, (uint16_t)(w[t >> 1] >> (16 * (t & 1))))), acc[t]);
+                }
+            };
+            use(cur.js[p], cur.c[p], cur.v[p]);
+            for (int32_t jb = cur.js[p] + 16 * U; jb < cur.je[p]; jb += 16 * U) {
+                int32_t c2[U];
+                uint32_t v2[U];
+                load(cur.je[p], jb, c2, v2);
+                use(jb, c2, v2);
+            }
+            // sums over the row's 16 lanes, halving the tokens a lane keeps as
+            // it goes (partners: lane ^ 8, 7 - lane of each 8, lane ^ 2, lane ^ 1)
+            if constexpr (TT == 8) {
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float keep = (l16 & 8) ? acc[t + 4] : acc[t], give = (l16 & 8) ? acc[t] : acc[t + 4];
+                    acc[t] = keep + dpp_f32<0x128>(give);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < TT; t++) acc[t] += dpp_f32<0x128>(acc[t]);
+            }
+            if constexpr (TT >= 4) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const float keep = (l16 & 4) ? acc[t + 2] : acc[t], give = (l16 & 4) ? acc[t] : acc[t + 2];
+                    acc[t] = keep + dpp_f32<0x141>(give);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < TT; t++) acc[t] += dpp_f32<0x141>(acc[t]);
+            }
+            const float keep = (l16 & 2) ? acc[1] : acc[0], give = (l16 & 2) ? acc[0] : acc[1];
+            float one = keep + dpp_f32<0x4E>(give);
+            one += dpp_f32<0xB1>(one);
+            const int tok = (TT == 8 ? (l16 >> 3) * 4 : 0) + (TT >= 4 ? ((l16 >> 2) & 1) * 2 : 0) + ((l16 >> 1) & 1);
+            if ((l16 & 1) == 0) sums[tok * kSsRows + 4 * p + sub] = one;  // (lanes of one token agree bit for bit or, below
+                                                                          // 8 tokens, were summed in mirrored order)
+        }
+        __builtin_amdgcn_wave_barrier();  // (same wave: LDS keeps the order)
+#pragma unroll
+        for (int i = 0; i < PL; i++) {
+            const int t = sub + 4 * i;
+            if (t < TT && m0 + t < a.M && r0 + l16 < a.N)
+                part[(int64_t)(m0 + t) * a.N + r0 + l16] = a.alpha * sums[t * kSsRows + l16];
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
 
 // GMODE: 0 per-row scale (G == K); 1 G = 128, scales read as aligned pairs;
 // 2 any G = 128 * 2^j; 3 (one token tile) G = 128 with every slice exactly CPS = 8 chunks
@@ -113,16 +298,17 @@ struct SkinnyArgs {
 // 1 ortho term, 2 ortho term for at most 8 tokens (one tile: the four lanes
 // of a row gather two tokens each, not four); 3 .. 6 (one tile, GMODE 3) the
 // same from the plan's slice records instead of the CSR: 3 / 4 records of
-// 256 words (4: at most 8 tokens), 5 / 6 of 512 words.
+// 256 words (4: at most 8 tokens), 5 / 6 of 512 words; 7 (two and more tiles)
+// the ortho term in workgroups and a partial of its own.
 // (4 waves per SIMD up to two token tiles; BF16 with two tiles needs the
 // registers of 2: at 4 one instantiation spilled 8 bytes)
 template <int NTT, int GMODE, int CPS, int SPK, bool XB>
 __global__ void __launch_bounds__(kSkNT) __attribute__((amdgpu_waves_per_eu(NTT == 1 || (NTT == 2 && !XB) ? 4 : 2)))
 skinny_kernel(SkinnyArgs a) {
-    constexpr bool SPARSE = SPK != 0;
-    constexpr bool SREC = SPK >= 3;                  // slice records: each wave reads its 16 rows' record
+    constexpr bool SPARSE = SPK != 0 && SPK != 7;
+    constexpr bool SREC = SPK >= 3 && SPK != 7;                  // slice records: each wave reads its 16 rows' record
     constexpr bool HALF = SPK == 2 || SPK == 4 || SPK == 6;
-    constexpr int RQ = SPK >= 5 ? 2 : 1;             // record loads per lane (256 words each per wave)
+    constexpr int RQ = SPK == 5 || SPK == 6 ? 2 : 1;             // record loads per lane (256 words each per wave)
     constexpr int MP = NTT * 16;                     // padded tokens
     constexpr int XP = (MP * CPS * 16 + kSkNT - 1) / kSkNT;  // 16-byte pieces per thread
     constexpr int SW = (CPS + 7) / 8;
@@ -164,8 +350,18 @@ skinny_kernel(SkinnyArgs a) {
     // block blk run on XCD blk % 8, as does the reduction workgroup of blk,
     // so a block's partials are written and read through one L2.  The grid
     // is padded to 8 * ceil(nblocks / 8) * S.
-    const int q = (int)(blockIdx.x >> 3);
-    const int blk = (int)(blockIdx.x & 7) + 8 * (q / a.S), slice = q - (q / a.S) * a.S;
+    int bid = (int)blockIdx.x;
+    if constexpr (SPK == 7) {
+        if (bid < a.sp_wgs) {  // (uniform)
+            if (a.sp_tt == 8) skinny_sparse<8, XB>(a, smem);
+            else if (a.sp_tt == 4) skinny_sparse<4, XB>(a, smem);
+            else skinny_sparse<2, XB>(a, smem);
+            return;
+        }
+        bid -= a.sp_wgs;
+    }
+    const int q = bid >> 3;
+    const int blk = (bid & 7) + 8 * (q / a.S), slice = q - (q / a.S) * a.S;
     if (blk >= a.nblocks) return;
     const int64_t n0 = (int64_t)blk * kSkRows;
     const int kc0 = slice * a.cps;                               // first chunk of the slice
@@ -652,6 +848,7 @@ __global__ void __launch_bounds__(256) skinny_reduce_kernel(const float *part, f
 struct SkinnyShape {
     int ntt, cps, S, nblocks, xstride;
     int lds_cr, lds_xs, lds_sp, lds_bytes;
+    int sp_wgs, sp_tt, sp_tiles;  // the ortho term's own workgroups (0: none)
 };
 
 static bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
@@ -677,6 +874,19 @@ static bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
     sh.lds_sp = off;
     off += a.has_ortho && ntt == 1 ? kSkRows * mp * 4 : 0;  // the kernel's QUAD exchange
     sh.lds_bytes = off;
+    sh.sp_wgs = sh.sp_tt = sh.sp_tiles = 0;
+    if (a.has_ortho && ntt > 1 && S > 1 && ss_tokens(a.K) > 0 &&
+        (int64_t)(S + 1) * a.M * a.N * 4 <= (int64_t)ORTH_NOALLOC_SCRATCH_BYTES) {
+        sh.sp_tt = ss_tokens(a.K);
+        sh.sp_tiles = (int)((a.M + sh.sp_tt - 1) / sh.sp_tt);
+        // three workgroups to four CUs, beside the dense ones (4096 -> 11008 at
+        // 48 tokens, 1 %: 128 workgroups 30.3 us, 192 26.8, 256 28.8), each
+        // wave with at least one unit of rows; whole rows of the XCD map
+        const int64_t units = (a.N + kSsRows - 1) / kSsRows;
+        const int64_t per = std::max<int64_t>(1, std::min<int64_t>((units + 7) / 8, cus * 3 / 4 / sh.sp_tiles));
+        sh.sp_wgs = (int)((per * sh.sp_tiles + 7) / 8 * 8);
+        sh.lds_bytes = std::max(off, ss_lds(a.K, sh.sp_tt));
+    }
     return off <= 150 * 1024;
 }
 
@@ -727,6 +937,8 @@ static hipError_t skinny_launch_g(const SkinnyArgs &d, bool sparse, int blocks, 
                             : skinny_launch_t<NTT, GMODE, C, 5, XB>(d, blocks, lds, s);
             }
         }
+        if constexpr (NTT > 1)
+            if (d.sp_wgs > 0) return skinny_launch_t<NTT, GMODE, C, 7, XB>(d, blocks, lds, s);
         if (NTT == 1 && d.M <= 8) return skinny_launch_t<NTT, GMODE, C, (NTT == 1 ? 2 : 1), XB>(d, blocks, lds, s);
         return skinny_launch_t<NTT, GMODE, C, 1, XB>(d, blocks, lds, s);
     }
@@ -760,7 +972,22 @@ static hipError_t skinny_launch_x(const SkinnyArgs &d, int ntt, int gmode, bool 
 int64_t skinny_workspace_bytes(const ForwardArgs &a, int cus) {
     SkinnyShape sh;
     skinny_shape(a, cus, sh);
-    return sh.S > 1 ? (int64_t)sh.S * a.M * a.N * 4 : 0;
+    return sh.S > 1 ? (int64_t)(sh.S + (sh.sp_wgs > 0 ? 1 : 0)) * a.M * a.N * 4 : 0;
+}
+
+// 33 .. 64 tokens at K > 4096 (the dispatcher's choice between this kernel and
+// the prefill kernel with K split).  us, this / prefill: without an ortho term
+// 11008 -> 4096 at 33 tokens 16.6 / 29.7, at 64 22.1 / 31.5, 8192 -> 2048 at 64
+// 11.6 / 22.9; with one, where a workgroup of its own keeps 8 tokens (K up to
+// 8250) and it is not too large (entries x tokens): 5120 -> 5120 at 64, 1 % (17
+// million) 25.0 / 27.7, 2 % (34) 31.3 / 28.2, 8192 -> 2048 at 64, 2 % (21)
+// 21.1 / 26.7, 8192 -> 8192 at 40, 1 % (27) 43.3 / 45.7; 11008 -> 4096 at 64, 2 %
+// 56.7 / 35.7.  Its partials must fit the no-allocation scratch array, as the
+// prefill kernel's always do.
+bool skinny_wide_k_preferred(const ForwardArgs &a, int cus) {
+    SkinnyShape sh;
+    if (!skinny_shape(a, cus, sh) || skinny_workspace_bytes(a, cus) > (int64_t)ORTH_NOALLOC_SCRATCH_BYTES) return false;
+    return !a.has_ortho || (sh.sp_tt == 8 && a.nnz * a.M <= 27000000);
 }
 
 // plan: the ortho plan (optional: its chunk table locates the slice's CSR
@@ -823,7 +1050,10 @@ hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float 
         d.swords = sw;
         lds += 8 * sw * 4;
     }
-    const int blocks = ((sh.nblocks + 7) / 8) * 8 * sh.S;  // padded: see skinny_kernel
+    d.sp_wgs = sh.sp_wgs;
+    d.sp_tt = sh.sp_tt;
+    d.sp_tiles = sh.sp_tiles;
+    const int blocks = sh.sp_wgs + ((sh.nblocks + 7) / 8) * 8 * sh.S;  // padded: see skinny_kernel
     const bool xb = a.io_dtype == ORTH_DT_BF16;
     const hipError_t e = xb ? skinny_launch_x<true>(d, sh.ntt, gmode, sparse, blocks, lds, stream)
                             : skinny_launch_x<false>(d, sh.ntt, gmode, sparse, blocks, lds, stream);
@@ -832,7 +1062,7 @@ hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float 
     const int R = skinny_reduce_parts((int)a.M, vec4);
     const unsigned rblocks = (unsigned)(((sh.nblocks + 7) / 8) * 8 * R);
     hipLaunchKernelGGL(skinny_reduce_kernel, dim3(rblocks), dim3(256), 0, stream, part, static_cast<f16 *>(a.y),
-                       (int)a.M, a.N, sh.S, vec4, sh.nblocks, R, a.bias, a.bias_dtype, xb ? 1 : 0);
+                       (int)a.M, a.N, sh.S + (sh.sp_wgs > 0 ? 1 : 0), vec4, sh.nblocks, R, a.bias, a.bias_dtype, xb ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -22,11 +22,11 @@
 //    when the rows' columns ascend; otherwise (or without a plan) each row's
 //    whole range is read and filtered by column, in batches of eight
 //    entries.  Up to 16 tokens, four consecutive lanes share a row: each
-//    loads two of every eight entries, DPP quad broadcasts hand all eight to
-//    the four, each multiplies them with four tokens' staged activations
-//    (two up to 8 tokens: tokens past M are padding of the tile), and the
-//    sums reach the MFMA lanes through LDS.  Sums are formed in CSR order: the
-//    result does not depend on scheduling.
+//    takes two of every eight entries and multiplies them with all tokens,
+//    read from a second, transposed copy of the staged activations (one
+//    16-byte read per entry and 8 tokens), and the quad's sums reach the MFMA
+//    lanes through LDS.  Sums are formed in a fixed order: the result does
+//    not depend on scheduling.
 //  * From 17 tokens, where K is split, the ortho term is a slice of its own:
 //    workgroups at the head of the grid (skinny_sparse) keep all columns of 8,
 //    4 or 2 tokens in LDS, [column][token], walk the CSR of a run of rows, 16
@@ -67,11 +67,6 @@ constexpr int kSkRows = 128;          // rows per workgroup (= ortho plan block)
 constexpr int kSkMaxCPS = 8;          // chunks per slice (compile-time bound)
 constexpr int kSkEB = 8;              // CSR entries of a row per batch
 
-// x from lane s of each group of four lanes (DPP quad_perm)
-template <int S>
-__device__ __forceinline__ int quad_bcast(int x) {
-    return __builtin_amdgcn_update_dpp(0, x, S | (S << 2) | (S << 4) | (S << 6), 0xf, 0xf, false);
-}
 constexpr uint32_t kSkPlanMagic = 0x504f5254u;
 constexpr uint32_t kSkPlanVersion = 5;
 constexpr uint32_t kSkPlanUnsorted = 4u;  // plan flag: the chunk table does not locate ranges
@@ -102,6 +97,7 @@ struct SkinnyArgs {
     int nblocks;         // 128-row blocks
     int xstride;         // LDS row stride of the staged activations, in halves
     int lds_cr, lds_xs, lds_sp;  // byte offsets of the LDS regions
+    int lds_xt;          // one token tile, ortho term: the slice's activations [column][token]
     float alpha;
     float *part;         // [S][M][N] partials (S > 1)
     const uint32_t *srec;  // plan slice records (SPK >= 3), swords words each
@@ -295,8 +291,8 @@ __device__ void skinny_sparse(const SkinnyArgs &a, unsigned char *smem) {
 // term is straight-line code over chunk pairs (two MFMA chains interleaved)
 // and the weight loads run four chunks ahead instead of all at entry.
 // NTT: 16-token tiles.  CPS: chunk bound per slice.  SPK: 0 no ortho term,
-// 1 ortho term, 2 ortho term for at most 8 tokens (one tile: the four lanes
-// of a row gather two tokens each, not four); 3 .. 6 (one tile, GMODE 3) the
+// 1 ortho term, 2 ortho term for at most 8 tokens (one tile: 8 tokens a
+// column in the transposed copy, not 16); 3 .. 6 (one tile, GMODE 3) the
 // same from the plan's slice records instead of the CSR: 3 / 4 records of
 // 256 words (4: at most 8 tokens), 5 / 6 of 512 words; 7 (two and more tiles)
 // the ortho term in workgroups and a partial of its own.
@@ -336,11 +332,16 @@ skinny_kernel(SkinnyArgs a) {
                                                           c, 0, 0, 0);
     };
     constexpr int EL = QUAD ? kSkEB / 4 : kSkEB;  // entries a lane loads per batch
+    constexpr int XTT = HALF ? 8 : 16;  // QUAD: tokens of a column in the transposed copy
+    // byte offset of a column's tokens (16 bytes of padding after every 8
+    // columns); column CPS * 128 holds zeros, for empty entries
+    auto xt_at = [](int c) -> int { return c * (2 * XTT) + (c >> 3) * 16; };
 
     extern __shared__ __align__(16) unsigned char smem[];
     float *cr = reinterpret_cast<float *>(smem + a.lds_cr);     // [cps][MP] bias sums
     f16 *xs = reinterpret_cast<f16 *>(smem + a.lds_xs);         // [MP][xstride] activations
     float *sp = reinterpret_cast<float *>(smem + a.lds_sp);     // QUAD: [128][MP] sparse sums
+    unsigned char *xt = smem + a.lds_xt;                        // QUAD: transposed activations
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -459,6 +460,24 @@ skinny_kernel(SkinnyArgs a) {
             *reinterpret_cast<u32x4 *>(xs + (m * a.xstride + c * 128 + (p & 15) * 8)) = permute_x8(v);
             if ((p & 15) == 0) cr[c * MP + m] = b;
         }
+        if (SPARSE && QUAD) xreg[i] = v;
+    }
+    if constexpr (SPARSE && QUAD) {
+        // the thread's tokens tid / 128 + 4 i of its 8 columns, turned: token m
+        // at place (m % 4) * (XTT / 4) + m / 4 of its column
+        static_assert(XP == 4 && CPS == 8, "one token tile: 8 columns of four tokens per thread");
+        const int c = (tid / 16) % CPS, j = tid & 15, mq = tid / 128;
+        if (c < a.cps) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+                const uint32_t w0 = __builtin_amdgcn_perm(xreg[1][e >> 1], xreg[0][e >> 1], sel);
+                unsigned char *dst = xt + xt_at(c * 128 + 8 * j + e) + mq * (XTT / 2);
+                if constexpr (HALF) *reinterpret_cast<uint32_t *>(dst) = w0;
+                else *reinterpret_cast<uint2 *>(dst) = uint2{w0, __builtin_amdgcn_perm(xreg[3][e >> 1], xreg[2][e >> 1], sel)};
+            }
+        }
+        if (tid < XTT / 2) *reinterpret_cast<uint32_t *>(xt + xt_at(CPS * 128) + 4 * tid) = 0u;
     }
     if (SREC) {
         uint32_t *wr = reinterpret_cast<uint32_t *>(smem + a.lds_sr) + wave * a.swords;
@@ -506,7 +525,37 @@ skinny_kernel(SkinnyArgs a) {
     // ---- SREC: the sparse sums from the record, before the dense term:
     //      the remaining weight loads are issued first, so the stream does
     //      not pause while the sums are formed
-    constexpr int TQ = QUAD ? (HALF ? 2 : MP / 4) : NTT * 4;  // tokens per lane
+    constexpr int TQ = QUAD ? XTT : NTT * 4;  // tokens per lane (QUAD: all of the lane's own entries)
+    // QUAD: a lane's entry (its column in the slice, or none) times all tokens
+    auto quad_fma = [&](bool ok, int32_t cl, uint32_t vbits, float (&acc)[QUAD ? XTT : 1]) {
+        if constexpr (QUAD) {
+            const float val = ok ? (float)__builtin_bit_cast(f16, (uint16_t)(vbits & 0xffffu)) : 0.f;
+            const u32x4 *src = reinterpret_cast<const u32x4 *>(xt + xt_at(ok ? cl : CPS * 128));
+            u32x4 w[XTT / 8];
+#pragma unroll
+            for (int i = 0; i < XTT / 8; i++) w[i] = src[i];
+#pragma unroll
+            for (int t = 0; t < XTT; t++)
+                acc[t] = __builtin_fmaf(val, x16_to_f32<XB>(__builtin_bit_cast(f16, (uint16_t)(w[t >> 3][(t >> 1) & 3] >> (16 * (t & 1))))), acc[t]);
+        }
+    };
+    // QUAD: the quad's sums (halving the tokens a lane keeps: partners lane ^
+    // 2, lane ^ 1) to sp
+    auto quad_out = [&](float (&acc)[QUAD ? XTT : 1]) {
+        if constexpr (QUAD) {
+#pragma unroll
+            for (int t = 0; t < XTT / 2; t++) {
+                const float keep = (tg & 2) ? acc[t + XTT / 2] : acc[t], give = (tg & 2) ? acc[t] : acc[t + XTT / 2];
+                acc[t] = keep + dpp_f32<0x4E>(give);
+            }
+#pragma unroll
+            for (int t = 0; t < XTT / 4; t++) {
+                const float keep = (tg & 1) ? acc[t + XTT / 4] : acc[t], give = (tg & 1) ? acc[t] : acc[t + XTT / 4];
+                // place (tg / 2) XTT / 2 + (tg % 2) XTT / 4 + t holds token tg + 4 t
+                sp[sr * MP + ((tg >> 1) * 2 + (tg & 1)) + 4 * t] = keep + dpp_f32<0xB1>(give);
+            }
+        }
+    };
     float sacc_e[SREC ? TQ : 1];
     if constexpr (SREC) {
 #pragma unroll
@@ -516,35 +565,11 @@ skinny_kernel(SkinnyArgs a) {
 #pragma unroll
         for (int t = 0; t < TQ; t++) sacc_e[t] = 0.f;
         const int32_t c0 = kc0 * 128, cw = nci * 128;
-        const int xstride = a.xstride;
         auto fma_batch = [&](int32_t j0, const int32_t (&c)[EL], const uint32_t (&v)[EL]) {
 #pragma unroll
-            for (int e = 0; e < kSkEB; e++) {
-                int32_t ce;
-                uint32_t ve;
-                if (QUAD) {  // entry j0 + e sits in lane e % 4 of the quad, slot e / 4
-                    const int slot = e >> 2;
-                    switch (e & 3) {
-                        case 0: ce = quad_bcast<0>(c[slot]); ve = (uint32_t)quad_bcast<0>((int)v[slot]); break;
-                        case 1: ce = quad_bcast<1>(c[slot]); ve = (uint32_t)quad_bcast<1>((int)v[slot]); break;
-                        case 2: ce = quad_bcast<2>(c[slot]); ve = (uint32_t)quad_bcast<2>((int)v[slot]); break;
-                        default: ce = quad_bcast<3>(c[slot]); ve = (uint32_t)quad_bcast<3>((int)v[slot]); break;
-                    }
-                } else {
-                    ce = c[e % EL];
-                    ve = v[e % EL];
-                }
-                const int32_t cl = ce - c0;
-                const bool ok = (j0 + e < hi) & (cl >= 0) & (cl < cw);
-                const int cc = ok ? cl : 0;
-                const float val = (float)__builtin_bit_cast(f16, (uint16_t)(ve & 0xffffu));
-                const int xi = (cc & ~7) | interleaved_pos(cc & 7);
-#pragma unroll
-                for (int t = 0; t < TQ; t++) {
-                    const int m = QUAD ? tg + 4 * t : 16 * (t >> 2) + 4 * g + (t & 3);
-                    const float pr = val * x16_to_f32<XB>(xs[m * xstride + xi]);
-                    sacc_e[t] += ok ? pr : 0.f;
-                }
+            for (int u = 0; u < EL; u++) {
+                const int32_t cl = c[u] - c0;
+                quad_fma((j0 + tg + 4 * u < hi) & (cl >= 0) & (cl < cw), cl, v[u], sacc_e);
             }
         };
         const uint32_t *wr = reinterpret_cast<const uint32_t *>(smem + a.lds_sr) + wave * a.swords;
@@ -580,10 +605,7 @@ skinny_kernel(SkinnyArgs a) {
                 fma_batch(j0, c2, v2);
             }
         }
-        if (QUAD) {
-#pragma unroll
-            for (int t = 0; t < TQ; t++) sp[sr * MP + tg + 4 * t] = sacc_e[t];
-        }
+        quad_out(sacc_e);
     }
     // ---- dense term: wave w, rows 16 w + nl, token tiles tt
     f32x4 acc[NTT];
@@ -685,31 +707,21 @@ skinny_kernel(SkinnyArgs a) {
         const int xstride = a.xstride;
         auto fma_batch = [&](int32_t j0, const int32_t (&c)[EL], const uint32_t (&v)[EL]) {
 #pragma unroll
-            for (int e = 0; e < kSkEB; e++) {
-                int32_t ce;
-                uint32_t ve;
-                if (QUAD) {  // entry j0 + e sits in lane e % 4 of the quad, slot e / 4
-                    const int slot = e >> 2;
-                    switch (e & 3) {
-                        case 0: ce = quad_bcast<0>(c[slot]); ve = (uint32_t)quad_bcast<0>((int)v[slot]); break;
-                        case 1: ce = quad_bcast<1>(c[slot]); ve = (uint32_t)quad_bcast<1>((int)v[slot]); break;
-                        case 2: ce = quad_bcast<2>(c[slot]); ve = (uint32_t)quad_bcast<2>((int)v[slot]); break;
-                        default: ce = quad_bcast<3>(c[slot]); ve = (uint32_t)quad_bcast<3>((int)v[slot]); break;
-                    }
+            for (int e = 0; e < EL; e++) {
+                const int32_t cl = c[e] - c0;
+                if constexpr (QUAD) {
+                    quad_fma((j0 + tg + 4 * e < hi) & (cl >= 0) & (cl < cw), cl, v[e], sacc);
                 } else {
-                    ce = c[e % EL];
-                    ve = v[e % EL];
-                }
-                const int32_t cl = ce - c0;
-                const bool ok = (j0 + e < hi) & (cl >= 0) & (cl < cw);
-                const int cc = ok ? cl : 0;
-                const float val = (float)__builtin_bit_cast(f16, (uint16_t)(ve & 0xffffu));
-                const int xi = (cc & ~7) | interleaved_pos(cc & 7);
+                    const bool ok = (j0 + e < hi) & (cl >= 0) & (cl < cw);
+                    const int cc = ok ? cl : 0;
+                    const float val = (float)__builtin_bit_cast(f16, (uint16_t)(v[e] & 0xffffu));
+                    const int xi = (cc & ~7) | interleaved_pos(cc & 7);
 #pragma unroll
-                for (int t = 0; t < TQ; t++) {
-                    const int m = QUAD ? tg + 4 * t : 16 * (t >> 2) + 4 * g + (t & 3);
-                    const float pr = val * x16_to_f32<XB>(xs[m * xstride + xi]);
-                    sacc[t] += ok ? pr : 0.f;
+                    for (int t = 0; t < TQ; t++) {
+                        const int m = 16 * (t >> 2) + 4 * g + (t & 3);
+                        const float pr = val * x16_to_f32<XB>(xs[m * xstride + xi]);
+                        sacc[t] += ok ? pr : 0.f;
+                    }
                 }
             }
         };
@@ -723,10 +735,7 @@ skinny_kernel(SkinnyArgs a) {
             load_batch(j0, c2, v2);
             fma_batch(j0, c2, v2);
         }
-        if (QUAD) {
-#pragma unroll
-            for (int t = 0; t < TQ; t++) sp[sr * MP + tg + 4 * t] = sacc[t];
-        }
+        if constexpr (QUAD) quad_out(sacc);
     }
     if (SPARSE && QUAD) __syncthreads();  // the sums reach the MFMA lanes
 
@@ -847,7 +856,7 @@ __global__ void __launch_bounds__(256) skinny_reduce_kernel(const float *part, f
 
 struct SkinnyShape {
     int ntt, cps, S, nblocks, xstride;
-    int lds_cr, lds_xs, lds_sp, lds_bytes;
+    int lds_cr, lds_xs, lds_sp, lds_xt, lds_bytes;
     int sp_wgs, sp_tt, sp_tiles;  // the ortho term's own workgroups (0: none)
 };
 
@@ -873,6 +882,8 @@ static bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
     off += ((mp * sh.xstride * 2) + 15) & ~15;
     sh.lds_sp = off;
     off += a.has_ortho && ntt == 1 ? kSkRows * mp * 4 : 0;  // the kernel's QUAD exchange
+    sh.lds_xt = off;  // the transposed activations: 8 or 16 tokens a column, a zero column after the last
+    if (a.has_ortho && ntt == 1) off += (kSkMaxCPS * 128 + 1) * (a.M <= 8 ? 16 : 32) + (kSkMaxCPS * 128 / 8) * 16;
     sh.lds_bytes = off;
     sh.sp_wgs = sh.sp_tt = sh.sp_tiles = 0;
     if (a.has_ortho && ntt > 1 && S > 1 && ss_tokens(a.K) > 0 &&
@@ -1027,6 +1038,7 @@ hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float 
     d.lds_cr = sh.lds_cr;
     d.lds_xs = sh.lds_xs;
     d.lds_sp = sh.lds_sp;
+    d.lds_xt = sh.lds_xt;
     d.alpha = a.alpha;
     d.part = part;
     // pairs of group-128 scales are read as aligned 32-bit words when every

@@ -79,6 +79,25 @@ def test_skinny_slice_odd_csr_infinities_and_bias(gpu, oracle_mod):
     check(oracle_mod, lay, x, 1.0, torch.float16, y)
 
 
+@pytest.mark.parametrize("K,N,M,density,dtype,plan", [
+    (2048, 600, 5, 0.02, torch.float16, True), (1152, 600, 8, 0.1, torch.bfloat16, False),
+    (11008, 300, 9, 0.02, torch.bfloat16, True), (2048, 600, 16, 0.05, torch.float16, False)])
+def test_one_token_tile_transposed_copy(gpu, oracle_mod, K, N, M, density, dtype, plan):
+    """5 .. 16 tokens, 8 or 16 a column, slices of fewer than 8 chunks and a
+    narrower last one, from the records and from the CSR: parity, and an
+    infinity or a NaN (also under an empty entry's column) stays with its token."""
+    lay = W.make_layer(K, N, 128, density, 9200 + K)
+    x = torch.from_numpy(W.make_x(M, K, 9201 + M)).to(dtype).float().numpy()
+    y, k = run(lay, x, 1.0, dtype, plan=plan)
+    assert k == "skinny"
+    check(oracle_mod, lay, x, 1.0, dtype, y)
+    bad = x.copy()
+    bad[1, 0], bad[M - 1, K - 1] = np.inf, np.nan
+    z, _ = run(lay, bad, 1.0, dtype, plan=plan)
+    keep = [m for m in range(M) if m not in (1, M - 1)]
+    assert torch.equal(z[keep], y[keep]) and torch.isnan(z[M - 1]).all()
+
+
 @pytest.mark.parametrize("K,N,M,density,alpha,kernel", [
     (8192, 1024, 33, 0.01, 1.0, "skinny"), (8320, 1024, 33, 0.01, 1.0, "prefill"),
     (8192, 2048, 64, 0.03, 1.0, "prefill"),          # entries x tokens past 27 million

@@ -25,11 +25,13 @@
 //  * float_ortho_kernel, the sparse term (alpha > 0): y += alpha * sum v x.
 //    A workgroup keeps all columns of up to 8 tokens in LDS, [column][token],
 //    so that an entry costs one 16-byte LDS read per 4 tokens, and walks the
-//    CSR of a range of rows, 16 lanes a row.  y is FP32, so adding to it in
-//    a second launch rounds as adding in registers would.  Bound by the LDS
-//    reads (4 bytes a product) with their bank conflicts: 28 us at 512 tokens
-//    of 4096 -> 4096 at 1 %.  (Folding the values into the weight tile, as the
-//    16-bit prefill does, would need two more bfloat16 parts per weight.)
+//    CSR of a range of rows, 16 lanes a row, a lane its own entries (two lanes
+//    sharing each, with a branch around an empty slot: 28 us against 23 at 512
+//    tokens of 4096 -> 4096 at 1 %).  y is FP32, so adding to it in a second
+//    launch rounds as adding in registers would.  Bound by its LDS reads (4
+//    bytes a product) and vector ALU work.  (Folding the values into the
+//    weight tile, as the 16-bit prefill does, would need two more bfloat16
+//    parts per weight.)
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -261,16 +263,15 @@ struct FloatOrthoArgs {
 // U batches of entries of all four loaded before the first is used.
 template <int TT, bool VH>
 __global__ void __launch_bounds__(kFoNT) float_ortho_kernel(FloatOrthoArgs a) {
-    constexpr int V = TT < 4 ? TT : 4;   // tokens per lane
-    constexpr int LPE = TT / V;          // lanes per entry
-    constexpr int U = LPE == 2 ? 3 : 4;  // batches of 16 entries of a row in flight
+    constexpr int U = 3;                 // batches of 16 entries of a row in flight
     constexpr int PL = (TT * kFoRows + 63) / 64;  // outputs per lane of a unit
     extern __shared__ __align__(16) unsigned char smem[];
-    float *xs = reinterpret_cast<float *>(smem);          // [K][TT]
+    float *xs = reinterpret_cast<float *>(smem);          // [K + 1][TT], the last column zero (for empty entries)
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    float *sums = xs + a.K * TT + wave * (TT * kFoRows);  // the wave's [TT][16]
+    float *sums = xs + (a.K + 1) * TT + wave * (TT * kFoRows);  // the wave's [TT][16]
+    if (tid < TT) xs[a.K * TT + tid] = 0.f;
     const int64_t m0 = (int64_t)(blockIdx.x % (unsigned)a.ntm) * TT;
     const int wg = (int)(blockIdx.x / (unsigned)a.ntm);
 
@@ -298,7 +299,6 @@ __global__ void __launch_bounds__(kFoNT) float_ortho_kernel(FloatOrthoArgs a) {
         else return static_cast<const float *>(a.vals)[j];
     };
     const int sub = lane >> 4, l16 = lane & 15;           // row of a pass, lane of the row
-    const int tv = (l16 % LPE) * V;                       // the lane's first token
     const int64_t units = (a.N + kFoRows - 1) / kFoRows;
     for (int64_t un = (int64_t)wg * kFoW + wave; un < units; un += (int64_t)a.wgs * kFoW) {
         const int64_t r0 = un * kFoRows;
@@ -331,28 +331,31 @@ __global__ void __launch_bounds__(kFoNT) float_ortho_kernel(FloatOrthoArgs a) {
         for (int p = 0; p < 4; p++) load(p, js[p], c[p], v[p]);
 #pragma unroll
         for (int p = 0; p < 4; p++) {
-            float acc[V];
+            float acc[TT];
 #pragma unroll
-            for (int i = 0; i < V; i++) acc[i] = 0.f;
-            auto one = [&](int32_t j, int32_t cc, float vv) {
-                if (j < je[p] && cc >= 0 && cc < a.K) {
-                    const float *xc = xs + (int64_t)cc * TT + tv;
-#pragma unroll
-                    for (int i = 0; i < V; i++) acc[i] = __builtin_fmaf(vv, xc[i], acc[i]);
-                }
-            };
+            for (int t = 0; t < TT; t++) acc[t] = 0.f;
+            // a lane takes its own entries, all tokens of each
             auto use = [&](int32_t jb, const int32_t (&cc)[U], const float (&vv)[U]) {
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int32_t j = jb + 16 * u + l16;
-                    if constexpr (LPE == 2) {
-                        // the pair's two entries in turn (quad_perm 0022, 1133), half the tokens each
-                        const int32_t j0 = jb + 16 * u + (l16 & ~1);
-                        one(j0, __builtin_amdgcn_update_dpp(0, cc[u], 0xA0, 0xf, 0xf, false), dpp_f32<0xA0>(vv[u]));
-                        one(j0 + 1, __builtin_amdgcn_update_dpp(0, cc[u], 0xF5, 0xf, 0xf, false), dpp_f32<0xF5>(vv[u]));
+                    const bool ok = jb + 16 * u + l16 < je[p] && cc[u] >= 0 && cc[u] < a.K;
+                    if (u > 0 && !__any(ok)) continue;  // (uniform)
+                    const float val = ok ? vv[u] : 0.f;
+                    const float *xc = xs + (ok ? (int64_t)cc[u] : a.K) * TT;
+                    float x[TT];
+                    if constexpr (TT >= 4) {
+#pragma unroll
+                        for (int i = 0; i < TT / 4; i++) {
+                            const f32x4 q = reinterpret_cast<const f32x4 *>(xc)[i];
+#pragma unroll
+                            for (int e = 0; e < 4; e++) x[4 * i + e] = q[e];
+                        }
                     } else {
-                        one(j, cc[u], vv[u]);
+#pragma unroll
+                        for (int t = 0; t < TT; t++) x[t] = xc[t];
                     }
+#pragma unroll
+                    for (int t = 0; t < TT; t++) acc[t] = __builtin_fmaf(val, x[t], acc[t]);
                 }
             };
             use(js[p], c[p], v[p]);
@@ -362,20 +365,28 @@ __global__ void __launch_bounds__(kFoNT) float_ortho_kernel(FloatOrthoArgs a) {
                 load(p, jb, c2, v2);
                 use(jb, c2, v2);
             }
-            // sums over the row's lanes of equal l16 % LPE (rotations within 16 lanes)
+            // sums over the row's 16 lanes, halving the tokens a lane keeps as
+            // it goes (partners: lane ^ 8, 7 - lane of each 8, lane ^ 2, lane ^ 1)
+            auto fold = [&](auto ctrl_c, int bit, auto n_c) {
+                constexpr int CTRL = decltype(ctrl_c)::value, NV = decltype(n_c)::value;  // NV values: halve, 0: keep all
+                if constexpr (NV > 0) {
 #pragma unroll
-            for (int i = 0; i < V; i++) {
-                float s = acc[i];
-                s += dpp_f32<0x128>(s);
-                s += dpp_f32<0x124>(s);
-                s += dpp_f32<0x122>(s);
-                if (LPE == 1) s += dpp_f32<0x121>(s);
-                acc[i] = s;
-            }
-            if (l16 < LPE) {
+                    for (int t = 0; t < NV / 2; t++) {
+                        const float keep = (l16 & bit) ? acc[t + NV / 2] : acc[t], give = (l16 & bit) ? acc[t] : acc[t + NV / 2];
+                        acc[t] = keep + dpp_f32<CTRL>(give);
+                    }
+                } else {
 #pragma unroll
-                for (int i = 0; i < V; i++) sums[(tv + i) * kFoRows + 4 * p + sub] = acc[i];
-            }
+                    for (int t = 0; t < TT; t++) acc[t] += dpp_f32<CTRL>(acc[t]);
+                }
+            };
+            fold(std::integral_constant<int, 0x128>{}, 8, std::integral_constant<int, TT == 8 ? 8 : 0>{});
+            fold(std::integral_constant<int, 0x141>{}, 4, std::integral_constant<int, TT >= 4 ? 4 : 0>{});
+            fold(std::integral_constant<int, 0x4E>{}, 2, std::integral_constant<int, TT >= 2 ? 2 : 0>{});
+            const float one = acc[0] + dpp_f32<0xB1>(acc[0]);
+            const int tok = (TT == 8 ? (l16 >> 3) * 4 : 0) + (TT >= 4 ? ((l16 >> 2) & 1) * 2 : 0) + (TT >= 2 ? (l16 >> 1) & 1 : 0);
+            // (the lanes of one token hold the same bits: partners add the same two values)
+            if ((l16 & 1) == 0) sums[tok * kFoRows + 4 * p + sub] = one;
         }
         __builtin_amdgcn_wave_barrier();  // (same wave: LDS keeps the order)
         const int64_t n = r0 + l16;
@@ -399,7 +410,7 @@ static const int64_t kFoLdsMax = 160 * 1024;
 // Tokens a sparse-term workgroup keeps in LDS (0: K is too large).
 static int float_ortho_tokens(int64_t K) {
     for (int tt = 8; tt >= 1; tt /= 2)
-        if ((K + kFoRows * kFoW) * tt * 4 <= kFoLdsMax) return tt;
+        if ((K + 1 + kFoRows * kFoW) * tt * 4 <= kFoLdsMax) return tt;
     return 0;
 }
 
@@ -445,7 +456,7 @@ static hipError_t launch_float_ortho(FloatOrthoArgs o, int cus, hipStream_t stre
     // about one workgroup per CU (its LDS holds one), each wave with work
     o.ntm = (int)ntm;
     o.wgs = (int)std::max<int64_t>(1, std::min<int64_t>((units + kFoW - 1) / kFoW, cus / ntm));
-    const uint32_t lds = (uint32_t)((o.K + kFoRows * kFoW) * TT * 4);
+    const uint32_t lds = (uint32_t)((o.K + 1 + kFoRows * kFoW) * TT * 4);
     hipLaunchKernelGGL((float_ortho_kernel<TT, VH>), dim3((unsigned)(ntm * o.wgs)), dim3(kFoNT), lds, stream, o);
     return hipGetLastError();
 }

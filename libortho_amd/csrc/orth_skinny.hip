@@ -271,8 +271,8 @@ __device__ void skinny_sparse(const SkinnyArgs &a, unsigned char *smem) {
             float one = keep + dpp_f32<0x4E>(give);
             one += dpp_f32<0xB1>(one);
             const int tok = (TT == 8 ? (l16 >> 3) * 4 : 0) + (TT >= 4 ? ((l16 >> 2) & 1) * 2 : 0) + ((l16 >> 1) & 1);
-            if ((l16 & 1) == 0) sums[tok * kSsRows + 4 * p + sub] = one;  // (lanes of one token agree bit for bit or, below
-                                                                          // 8 tokens, were summed in mirrored order)
+            // (the lanes of one token hold the same bits: partners add the same two values)
+            if ((l16 & 1) == 0) sums[tok * kSsRows + 4 * p + sub] = one;
         }
         __builtin_amdgcn_wave_barrier();  // (same wave: LDS keeps the order)
 #pragma unroll

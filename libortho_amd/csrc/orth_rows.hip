@@ -20,13 +20,17 @@
 //    every product is exact and every sum FP32; the scale multiplies a
 //    chunk's (or 32 columns') partial.
 //  * Sparse term: each wave takes 2 RB rows; a row's entries are loaded 64 at
-//    a time, one per lane, before the staging's barrier, and handed to the
-//    lanes (entry, token) in turn, which gather from the staged activations.
+//    a time, one per lane, before the staging's barrier, with the place of the
+//    activation in a staged row (empty slots: a zero past its end), and handed
+//    to the lanes (entry, token) in turn, which gather there.  This follows
+//    the dense term, whose weights were asked for first: 4000 -> 11008, 16
+//    FP16 tokens at 1 %, 21.7 -> 18.9 us against taking it first with a test
+//    per entry; the dense term alone 12.2.
 //  * The waves' partials meet in LDS (deterministic) and are rounded once.
 //
 // What bounds it: the latency chain (staging, the weights' first bytes, the
 // reduction) at few tokens, the LDS reads of the sparse term at 16 (4000 ->
-// 11008, 16 FP16 tokens at 1 %: 139 us on the general kernel, 21 here).
+// 11008, 16 FP16 tokens at 1 %: 139 us on the general kernel, 18.9 here).
 #include <algorithm>
 #include <atomic>
 
@@ -116,8 +120,8 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
         }
     };
     // ---- entries of the wave's rows: row i's bounds and its first 64
-    //      entries, one per lane (column | value bits << 16; column 0xffff:
-    //      none)
+    //      entries, one per lane (place of its activation in a token's row |
+    //      value bits << 16; none: the zero place past the last column, 0)
     auto row_of = [&](int ps, int i) -> int64_t { return (int64_t)ps * RB * 16 + wave * NR + i; };
     int32_t js[NR], je[NR];
     uint32_t ent[NR];
@@ -125,7 +129,8 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
         const int32_t j = (int32_t)min(jb + lane, (int64_t)max(end - 1, 0));
         const uint32_t c = (uint32_t)a.col[j];
         const uint32_t v = __builtin_bit_cast(uint16_t, a.vals[j]);
-        return (c < (uint32_t)K && jb + lane < end) ? (c | (v << 16)) : 0xffffu;
+        const uint32_t at = F16 ? (c & ~7u) | (uint32_t)interleaved_pos(c & 7) : c;
+        return (c < (uint32_t)K && jb + lane < end) ? (at | (v << 16)) : (uint32_t)(a.nch * 128);
     };
     auto bounds = [&](int ps) {
 #pragma unroll
@@ -150,6 +155,8 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
         if (k >= K) v = u32x4{0u, 0u, 0u, 0u};
         *reinterpret_cast<u32x4 *>(xs + t * xst + k) = F16 ? permute_x8(v) : v;
     };
+    for (int t = tid; t < live; t += kRwNT)  // the zero place (and its row's padding)
+        *reinterpret_cast<u32x4 *>(xs + t * xst + a.nch * 128) = u32x4{0u, 0u, 0u, 0u};
     const int span = kRwNT * kRwXB;
     int p0 = tid;
     u32x4 xr[kRwXB];
@@ -176,53 +183,6 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
 
     const X *xa = xs + min(nl, live - 1) * xst;  // the lane's token (padding tokens repeat the last one)
     for (;;) {
-        // ---- sparse sums: lane (entry lane / tl of a round, token lane % tl)
-        if (a.sparse) {
-            const int tl = a.tl, tok = min(lane & (tl - 1), live - 1), e0 = lane / tl, epi = 64 / tl;
-            const X *xt = xs + tok * xst;
-            auto product = [&](uint32_t w) -> float {
-                const bool ok = (w & 0xffffu) != 0xffffu;
-                const uint32_t c = ok ? w & 0xffffu : 0u;
-                const float v = (float)__builtin_bit_cast(f16, (uint16_t)(w >> 16));
-                float xv;
-                if constexpr (F32) xv = xt[c];
-                else if constexpr (F16) xv = (float)__builtin_bit_cast(f16, xt[(c & ~7u) | interleaved_pos(c & 7)]);
-                else xv = bf16_bits_to_f32(xt[c]);
-                return ok ? v * xv : 0.f;
-            };
-            // every row's first 64 entries in step (a row that ends earlier
-            // holds empty ones): the rows' LDS round trips overlap
-            float s[NR];
-            int32_t top = 0;
-#pragma unroll
-            for (int i = 0; i < NR; i++) {
-                s[i] = 0.f;
-                top = max(top, je[i] - js[i]);
-            }
-            top = min(top, 64);
-            for (int r = 0; r < top; r += epi) {
-                uint32_t w[NR];
-#pragma unroll
-                for (int i = 0; i < NR; i++) w[i] = __shfl(ent[i], r + e0);  // (r + e0 < 64)
-#pragma unroll
-                for (int i = 0; i < NR; i++) s[i] += product(w[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < NR; i++) {  // longer rows
-                for (int64_t jb = (int64_t)js[i] + 64; jb < je[i]; jb += 64) {
-                    const uint32_t en = entries(jb, je[i]);
-                    for (int r = 0; r < 64; r += epi) s[i] += product(__shfl(en, r + e0));
-                }
-            }
-            for (int off = 32; off >= tl; off >>= 1)
-#pragma unroll
-                for (int i = 0; i < NR; i++) s[i] += __shfl_xor(s[i], off, 64);
-            if (lane < live) {
-#pragma unroll
-                for (int i = 0; i < NR; i++) sp[(wave * NR + i) * kRwRS + lane] = s[i];
-            }
-        }
-
         // ---- dense term
         f32x4 acc[RB];
 #pragma unroll
@@ -271,6 +231,54 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
             for (int d = 0; d < kRwD; d++) {
                 if (c + d < c1) chunk(c + d, buf[d]);  // (uniform)
                 issue(ps, c + d + kRwD, buf[d]);
+            }
+        }
+
+        // ---- sparse sums: lane (entry lane / tl of a round, token lane % tl).
+        //      After the dense term: the entries' loads were issued after the
+        //      weights'
+        if (a.sparse) {
+            const int tl = a.tl, tok = min(lane & (tl - 1), live - 1), e0 = lane / tl, epi = 64 / tl;
+            const X *xt = xs + tok * xst;
+            auto product = [&](uint32_t w, float s) -> float {
+                const float v = (float)__builtin_bit_cast(f16, (uint16_t)(w >> 16));
+                const X x = xt[w & 0xffffu];
+                float xv;
+                if constexpr (F32) xv = x;
+                else if constexpr (F16) xv = (float)__builtin_bit_cast(f16, x);
+                else xv = bf16_bits_to_f32(x);
+                return __builtin_fmaf(v, xv, s);
+            };
+            // every row's first 64 entries in step (a row that ends earlier
+            // holds empty ones): the rows' LDS round trips overlap
+            float s[NR];
+            int32_t top = 0;
+#pragma unroll
+            for (int i = 0; i < NR; i++) {
+                s[i] = 0.f;
+                top = max(top, je[i] - js[i]);
+            }
+            top = min(top, 64);
+            for (int r = 0; r < top; r += epi) {
+                uint32_t w[NR];
+#pragma unroll
+                for (int i = 0; i < NR; i++) w[i] = __shfl(ent[i], r + e0);  // (r + e0 < 64)
+#pragma unroll
+                for (int i = 0; i < NR; i++) s[i] = product(w[i], s[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < NR; i++) {  // longer rows
+                for (int64_t jb = (int64_t)js[i] + 64; jb < je[i]; jb += 64) {
+                    const uint32_t en = entries(jb, je[i]);
+                    for (int r = 0; r < 64; r += epi) s[i] = product(__shfl(en, r + e0), s[i]);
+                }
+            }
+            for (int off = 32; off >= tl; off >>= 1)
+#pragma unroll
+                for (int i = 0; i < NR; i++) s[i] += __shfl_xor(s[i], off, 64);
+            if (lane < live) {
+#pragma unroll
+                for (int i = 0; i < NR; i++) sp[(wave * NR + i) * kRwRS + lane] = s[i];
             }
         }
 
@@ -327,7 +335,8 @@ struct RowsShape {
 };
 
 static bool rows_shape(const ForwardArgs &a, int cus, RowsShape &sh) {
-    if (a.K % 8 != 0 || a.K < 32 || a.K > 65528 || a.N >= ((int64_t)1 << 31)) return false;
+    if (a.K % 8 != 0 || a.K < 32 || a.N >= ((int64_t)1 << 31)) return false;
+    if (a.K > 65408) return false;  // an entry holds its activation's place, at most K rounded up to 128, in 16 bits
     if (a.scale_dtype != ORTH_DT_F16 || (a.has_ortho && a.val_dtype != ORTH_DT_F16)) return false;
     if (a.ngroups != 1 && a.G % 32 != 0) return false;
     if ((reinterpret_cast<uintptr_t>(a.x) & 15) || (reinterpret_cast<uintptr_t>(a.q) & 3)) return false;
@@ -370,10 +379,10 @@ static bool rows_shape(const ForwardArgs &a, int cus, RowsShape &sh) {
 // Whether this kernel takes the call: its shape, and enough outputs to pay
 // for the staging and its barrier.  The general kernel's time grows with
 // M * N, this one's hardly below 16 tokens (us, general / this): FP32 4096 ->
-// 4096 at 2 tokens 10.2 / 11.4, at 4 14.6 / 12.0, 4096 -> 11008 at 1 18.8 /
-// 22.3, at 2 25.0 / 22.8, at 8 66 / 26; FP16 4000 -> 4096 at 1 10.8 / 11.2,
-// 4000 -> 11008 at 1 20.3 / 14.0, at 16 139 / 21; narrow rows (2720 -> 4096,
-// group 32) at 4 12.9 / 13.9, at 16 37.8 / 16.4.
+// 4096 at 2 tokens 10.2 / 11.4, at 4 14.6 / 12.3, 4096 -> 11008 at 1 18.8 /
+// 22.3, at 2 25.0 / 22.0, at 8 66 / 24.9; FP16 4000 -> 4096 at 1 10.8 / 11.2,
+// 4000 -> 11008 at 1 20.3 / 13.5, at 16 139 / 18.5; narrow rows (2720 -> 4096,
+// group 32) at 4 12.9 / 12.4, at 16 37.8 / 16.4.
 bool rows_preferred(const ForwardArgs &a, int cus) {
     RowsShape sh;
     if (!rows_shape(a, cus, sh)) return false;

@@ -20,9 +20,10 @@
 #include <vector>
 
 #include "orth_common.h"
+#include "orth_skinny_shape.h"
 
 namespace orth {
-hipError_t launch_general(const ForwardArgs &a, int cus, hipStream_t stream);
+hipError_t launch_general(const ForwardArgs &a, hipStream_t stream);
 hipError_t launch_dequant(const ForwardArgs &a, float *out, hipStream_t stream);
 hipError_t launch_pack_base(const void *w, int wdt, int64_t N, int64_t K, int64_t G, const void *s_in,
                             int sdt, uint8_t *q, void *s_out, hipStream_t stream);
@@ -64,7 +65,6 @@ hipError_t launch_split_group(const ForwardArgs *as, const void *const *plans, i
                               hipStream_t stream);
 hipError_t launch_mid(const ForwardArgs &a, const void *plan, int cus, hipStream_t stream);
 bool skinny_supported(const ForwardArgs &a);
-bool skinny_wide_k_preferred(const ForwardArgs &a, int cus);
 int64_t skinny_workspace_bytes(const ForwardArgs &a, int cus);
 hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float *part, hipStream_t stream);
 hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, void *w_base, int ieee_div,
@@ -72,7 +72,6 @@ hipError_t launch_sieve_quantize(const void *w, int dt, int64_t N, int64_t K, vo
 hipError_t launch_sieve_split(const void *w, int dt, int64_t N, int64_t K, const void *h, int hdt, int64_t h_stride,
                               int score_dt, int use_rank, int64_t rank, float thresh, void *w_base, void *w_ortho,
                               float *score, void *sel, int ieee_div, hipStream_t stream);
-int64_t sieve_select_bytes();
 int64_t sieve_hdiag_slices(int64_t n);
 hipError_t launch_sieve_hdiag(const void *x, int dt, int64_t n, int64_t K, float *partial, void *out, int ieee_div,
                               hipStream_t stream);
@@ -575,7 +574,9 @@ int launch_kernel(const ForwardArgs &a, const void *plan, int kernel, int dev, h
             e = pf(a.has_ortho ? plan : nullptr);
         }
     } else {
-        e = launch_general(a, g_dev[dev].cus, stream);
+        ForwardArgs g = a;
+        g.cus = g_dev[dev].cus;
+        e = launch_general(g, stream);
     }
     if (e != hipSuccess) return fail_hip(e, "kernel launch");
     return rc;
@@ -878,7 +879,7 @@ int orth_sieve_quantize_hip(const void *w, int32_t w_dtype, int64_t out_features
     return ORTH_OK;
 }
 
-int64_t orth_sieve_select_bytes(void) { return sieve_select_bytes(); }
+int64_t orth_sieve_select_bytes(void) { return (int64_t)sizeof(SieveSel); }
 
 int orth_sieve_split_hip(const void *w, int32_t w_dtype, int64_t out_features, int64_t in_features,
                          const void *h_inv, int32_t h_dtype, int64_t h_stride, int32_t score_dtype,

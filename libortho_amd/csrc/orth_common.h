@@ -57,6 +57,21 @@ struct ForwardArgs {
     int has_ortho;           // alpha > 0 && nnz > 0 (/root/reference/src/ortho.c:343)
     const void *bias = nullptr;  // [N] added to y after rounding, or null
     int bias_dtype = 0;
+    int cus = 256;           // compute units of the device
+};
+
+// ------------------------------------------------------ the sieve's select
+
+// Radix-select state: a histogram per level (a few copies, each added to by
+// every fourth workgroup, so that fewer atomics meet on one counter), the
+// bins found so far with the rank left within them, and the collected
+// scores per workgroup of the second pass (-1: too many for its part of the
+// buffer).
+constexpr int kSelBins = 2048, kSelCopies = 4, kSelWgs = 1024;
+struct SieveSel {
+    uint32_t hist[3][kSelCopies][kSelBins];
+    uint32_t bin[2], left[2];
+    int32_t count[kSelWgs];
 };
 
 // ---------------------------------------------------------------- scalars
@@ -210,9 +225,13 @@ __device__ __forceinline__ void int4x8_to_bf16_biased(uint32_t w, uint32_t out[4
     out[3] = ((w >> 12) & 0x000F000Fu) ^ 0x43084308u;  // (3,7)
 }
 
-// Exact BF16 integers q in natural order, word i holding weights 2 i and
-// 2 i + 1: the nibble XOR 8 as a byte, converted to FP32 minus 8 (exact), the
-// high halves packed (an integer of magnitude at most 8 fits them).
+// Exact BF16 values q / 1024 in natural order, word i holding weights 2 i and
+// 2 i + 1: the nibble XOR 8 as a byte, converted to FP32, (byte - 8) / 1024 in
+// one exact FMA, the high halves packed (an integer of magnitude at most 8
+// times a power of two fits them).  The divisor keeps the sum of up to 128
+// products with any finite activations finite; the caller's scales carry
+// kBf16Q.
+constexpr float kBf16Q = 1024.0f;
 __device__ __forceinline__ void int4x8_to_bf16_exact(uint32_t w, uint32_t out[4]) {
     const uint32_t u = w ^ 0x88888888u;
     const uint32_t lo = u & 0x0F0F0F0Fu, hi = (u >> 4) & 0x0F0F0F0Fu;

@@ -166,7 +166,8 @@ hipError_t launch_float(const ForwardArgs &a, int cus, hipStream_t stream);
 bool rows_preferred(const ForwardArgs &a, int cus);  // orth_rows.hip
 hipError_t launch_rows(const ForwardArgs &a, int cus, hipStream_t stream);
 
-hipError_t launch_general(const ForwardArgs &a, int cus, hipStream_t stream) {
+hipError_t launch_general(const ForwardArgs &a, hipStream_t stream) {
+    const int cus = a.cus;
     // FP32 activations, large batches: the tile kernels (orth_float.hip) take
     // the same time for any batch of one round of their grid (~1 us per 64
     // columns), the rows kernel's grows with M * N.  us, rows / float, alpha = 1:

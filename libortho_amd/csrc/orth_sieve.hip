@@ -79,23 +79,10 @@ __device__ __forceinline__ float sieve_scalar_div(float v, float d, int ieee_div
     return ieee_div ? v / d : v * (1.0f / d);
 }
 
-// Radix-select state: a histogram per level (a few copies, each added to by
-// every fourth workgroup, so that fewer atomics meet on one counter), the
-// bins found so far with the rank left within them, and the collected
-// scores per workgroup of the second pass (-1: too many for its part of the
-// buffer).
-constexpr int kSelBins = 2048, kSelCopies = 4, kSelWgs = 1024;
-struct SieveSel {
-    uint32_t hist[3][kSelCopies][kSelBins];
-    uint32_t bin[2], left[2];
-    int32_t count[kSelWgs];
-};
 constexpr int kSvNT = 512;                      // threads of the split's passes
 constexpr int kSvLdsCols = 16384;               // columns of h + 1e-6 a workgroup keeps in LDS
 constexpr int kSvCache = 4;                     // vectors of a row per thread kept in registers
 constexpr int kSvLanes = 4;                     // LDS histograms, by lane
-
-int64_t sieve_select_bytes() { return (int64_t)sizeof(SieveSel); }
 
 __global__ void __launch_bounds__(256) sieve_sel_init_kernel(SieveSel *st) {
     const int i = blockIdx.x * 256 + threadIdx.x;

@@ -107,7 +107,7 @@ int orth_layer_check_hip(const orth_hip_layer_t *layer, const void *input, void 
  * term), the slice-split kernel (17..32 at the other K % 128 == 0, a plan
  * or no ortho term), the split-K mid-batch kernel (other batches up to 64;
  * 33..64 at K > 4096 with a plan or no ortho term: the prefill kernel with
- * K split over the grid),
+ * K split over the grid where it is the faster one),
  * the MFMA prefill kernels above (256 x 128 tiles with K split over the
  * grid and a reduction launch where the tiles alone leave CUs idle and a
  * plan or no ortho term is given; else the wide kernel where its 256 x 352
@@ -120,7 +120,7 @@ int orth_layer_check_hip(const orth_hip_layer_t *layer, const void *input, void 
  * kernel for 5..16 (both K = 4096 with a plan or no ortho term), the
  * slice-split kernel for 17..32 (K % 128 == 0, a plan or no ortho term),
  * the split-K mid-batch kernel for the other batches up to 64
- * (K % 128 == 0), the prefill kernel above; FP32 I/O the general kernel.  Kernels
+ * (K % 128 == 0), the prefill kernel above; FP32 I/O the general kernels.  Kernels
  * that need scratch memory (split-K partials, a prefill plan when none is
  * given) take it from a per-stream workspace or stream-ordered allocations.
  * Replaces orth_layer_forward_cuda, /root/reference/include/ortho.h:141-144

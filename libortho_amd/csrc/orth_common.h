@@ -248,7 +248,8 @@ __device__ __forceinline__ void int4x8_to_bf16_exact(uint32_t w, uint32_t out[4]
     asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(o[3]) : "v"(hi));
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        out[i] = __builtin_amdgcn_perm(__float_as_uint(o[i] - 8.0f), __float_as_uint(e[i] - 8.0f), 0x07060302u);
+        out[i] = __builtin_amdgcn_perm(__float_as_uint(__builtin_fmaf(o[i], 1.0f / kBf16Q, -8.0f / kBf16Q)),
+                                       __float_as_uint(__builtin_fmaf(e[i], 1.0f / kBf16Q, -8.0f / kBf16Q)), 0x07060302u);
 }
 
 // Eight FP32 values as three bfloat16 vectors with v = p0 + p1 + p2 exactly

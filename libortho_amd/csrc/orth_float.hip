@@ -6,8 +6,8 @@
 //
 //  * float_kernel, the dense term.  An FP32 value is the exact sum of three
 //    bfloat16 values (its significand cut in three runs of 8 bits, by
-//    truncation, so nothing rounds or overflows), and an INT4 weight is an
-//    exact bfloat16 integer, so three v_mfma_f32_16x16x32_bf16 passes form
+//    truncation, so nothing rounds or overflows), and an INT4 weight / 1024
+//    is an exact bfloat16 value, so three v_mfma_f32_16x16x32_bf16 passes form
 //    x * q with exact products and FP32 sums; the group scale multiplies the
 //    group's FP32 partial.  That is three passes at the bfloat16 matrix rate
 //    (2.5 PFLOP/s dense) against one at the FP32 matrix rate (157 TFLOP/s).
@@ -114,7 +114,8 @@ __global__ void __launch_bounds__(kFlNT) float_kernel(FloatArgs a) {
     load(1, r1);
     for (int i = tid; i < kFlBN * a.ngroups; i += kFlNT) {
         const int row = i / a.ngroups, gi = i - row * a.ngroups;
-        sl[gi * kFlBN + row] = load_as_f32(a.scales, a.scale_dtype, min(n0 + row, a.N - 1) * a.ngroups + gi);
+        sl[gi * kFlBN + row] =
+            kBf16Q * load_as_f32(a.scales, a.scale_dtype, min(n0 + row, a.N - 1) * a.ngroups + gi);
     }
     store(0, r0);
     load(2, r0);

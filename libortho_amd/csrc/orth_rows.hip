@@ -15,7 +15,7 @@
 //    covers 32 consecutive columns and takes its own group's scale (groups
 //    that are multiples of 32, rows of any multiple of 4 bytes).  Four chunks
 //    of loads are in flight, issued before the staging waits for its own.
-//  * The weights become exact FP16 or bfloat16 integers; FP32 activations
+//  * The weights become exact FP16 integers or bfloat16 q / 1024; FP32 activations
 //    are cut into three bfloat16 parts without rounding (split_bf16x3), so
 //    every product is exact and every sum FP32; the scale multiplies a
 //    chunk's (or 32 columns') partial.
@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
                     part[r] = mfma(av[0], bv, first ? zero : part[r]);
                     if constexpr (F32) low[r] = mfma(av[1], bv, mfma(av[2], bv, first ? zero : low[r]));
                     if (!WIDE || j == 3) {
-                        const float s = (float)b.s[r][WIDE ? 0 : j];
+                        const float s = (float)b.s[r][WIDE ? 0 : j] * (F16 ? 1.0f : kBf16Q);
 #pragma unroll
                         for (int i = 0; i < 4; i++)
                             acc[r][i] = __builtin_fmaf(s, F32 ? part[r][i] + low[F32 ? r : 0][i] : part[r][i], acc[r][i]);

@@ -72,6 +72,19 @@ def test_float_small_and_large_activations_keep_their_bits(oracle_mod):
     assert (np.abs(run(lay, x, 1.0) - ref) <= bound(lay, x, 1.0)).all()
 
 
+@pytest.mark.parametrize("M,K,N,G", [(130, 512, 2400, 128), (3, 512, 8200, None), (20, 480, 2400, 32)])
+def test_float_products_past_the_range_times_a_scale_within_it(oracle_mod, M, K, N, G):
+    """|q x| up to 4.8e38 overflows FP32, scale * q * x does not (tile kernel,
+    rows kernel with wide and narrow rows)."""
+    lay = W.make_layer(K, N, G, 0.02, 7300)
+    x = np.zeros((M, K), np.float32)
+    x[:, ::32] = np.random.Generator(np.random.PCG64(2)).uniform(-6e37, 6e37, (M, K // 32))
+    ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 0.0)
+    assert np.abs(ref).max() < 3e38
+    y = run(lay, x, 0.0)
+    assert np.isfinite(y).all() and (np.abs(y - ref) <= bound(lay, x, 0.0)).all()
+
+
 def test_float_infinities_and_nan_stay_with_their_token():
     K, N, M = 256, 4400, 70
     lay = W.make_layer(K, N, 128, 0.02, 7200)

@@ -283,6 +283,8 @@ int orth_sieve_quantize_hip(const void *w, int32_t w_dtype, int64_t out_features
  * `score`, FP32 [out_features * in_features], holding values of score_dtype,
  * the promotion of w's and h's dtypes).  h: element k at h_inv[k * h_stride]
  * (the diagonal of a matrix H_inv: its two strides summed; a vector: 1).
+ * w_base and w_ortho may be w's own buffer (in place); buffers that overlap at
+ * an offset give unspecified values.
  * use_rank: t = the rank-th largest score (torch.topk(...).values[-1], NaN
  * largest; rank 0 keeps nothing), found by a radix select in select_state
  * (orth_sieve_select_bytes() bytes of device memory); else t = threshold. */

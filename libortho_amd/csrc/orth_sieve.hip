@@ -69,6 +69,8 @@ struct SieveArgs {
     int score_dt;       // dtype of the score (torch's promotion of w's and H's)
     int ieee_div;       // 1: division by a host scalar as IEEE division (CPU
                         // tensors), 0: as a product with its FP32 reciprocal
+    int keep;           // the first pass stores the residual in w_ortho (else the
+                        // last one forms it again from w and w_base)
     struct SieveSel *sel;  // radix select, or null: the threshold below
     uint32_t rank;
     float thresh;
@@ -267,12 +269,13 @@ __global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4)))
                 }
                 sieve_store<DT, V>(a.w_base, base + k, wb);
                 if (a.score) {
+                    float rr[V];
 #pragma unroll
                     for (int e = 0; e < V; e++) {
-                        float rr;
-                        sc[e] = sieve_score<DT, S32>(w[j][e], wb[e], sieve_h<HL>(a, hs, k + e), s16, rr);
+                        sc[e] = sieve_score<DT, S32>(w[j][e], wb[e], sieve_h<HL>(a, hs, k + e), s16, rr[e]);
                         if (count) atomicAdd(&mine[sieve_key(sc[e]) >> 21], 1u);
                     }
+                    if (a.keep) sieve_store<DT, V>(a.w_ortho, base + k, rr);
                     sieve_store<ORTH_DT_F32, V>(a.score, base + k, sc);
                 }
                 __builtin_amdgcn_sched_barrier(0);  // one vector's divisions at a time: registers
@@ -362,10 +365,18 @@ __global__ void __launch_bounds__(kSvNT) sieve_refine_kernel(const float *score,
         if (h[i]) atomicAdd(&st->hist[2][blockIdx.x % kSelCopies][i], h[i]);
 }
 
-// w_ortho = residual * (score > t): t the selected k-th largest score or the
-// caller's threshold rounded to the score's dtype (torch compares a tensor
-// with a host scalar in the tensor's dtype); NaN compares false.  Both are
-// formed again from w and w_base: the residual is not stored in between.
+// The threshold: the selected k-th largest score, or the caller's rounded to
+// the score's dtype (torch compares a tensor with a host scalar in the
+// tensor's dtype).
+__device__ __forceinline__ float sieve_threshold(const SieveArgs &a) {
+    if (!a.sel) return round_as(a.score_dt, a.thresh);
+    uint32_t bin, left;
+    sieve_pick(a.sel, 2, a.sel->left[1], bin, left);
+    return sieve_unkey((a.sel->bin[0] << 21) | (a.sel->bin[1] << 10) | bin);
+}
+
+// w_ortho = residual * (score > t); NaN compares false.  Both are formed again
+// from w and w_base: the residual is not stored in between.
 template <int DT, int V, bool HL, bool S32>
 __global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4))) sieve_mask_kernel(SieveArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -373,12 +384,7 @@ __global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4)))
     const int tid = threadIdx.x;
     sieve_stage_h<HL>(a, hs);
     const bool s16 = a.score_dt == ORTH_DT_F16;
-    float t = round_as(a.score_dt, a.thresh);
-    if (a.sel) {
-        uint32_t bin, left;
-        sieve_pick(a.sel, 2, a.sel->left[1], bin, left);
-        t = sieve_unkey((a.sel->bin[0] << 21) | (a.sel->bin[1] << 10) | bin);
-    }
+    const float t = sieve_threshold(a);
     __syncthreads();
     for (int64_t r = blockIdx.x; r < a.N; r += gridDim.x) {
         const int64_t base = r * a.K;
@@ -405,6 +411,21 @@ __global__ void __launch_bounds__(kSvNT) __attribute__((amdgpu_waves_per_eu(4)))
                 __builtin_amdgcn_sched_barrier(0);  // (as above)
             }
         }
+    }
+}
+
+// The same from the residual stored in w_ortho and the scores (a.keep).
+template <int DT, int V>
+__global__ void __launch_bounds__(kSvNT) sieve_apply_kernel(SieveArgs a) {
+    const float t = sieve_threshold(a);
+    const int64_t n = a.N * a.K, step = (int64_t)gridDim.x * kSvNT * V;
+    for (int64_t i = ((int64_t)blockIdx.x * kSvNT + threadIdx.x) * V; i < n; i += step) {
+        float r[V], sc[V];
+        sieve_load<DT, V>(a.w_ortho, i, r);
+        sieve_load<ORTH_DT_F32, V>(a.score, i, sc);
+#pragma unroll
+        for (int e = 0; e < V; e++) r[e] = sieve_mul(r[e], sc[e] > t ? 1.f : 0.f);
+        sieve_store<DT, V>(a.w_ortho, i, r);
     }
 }
 
@@ -473,11 +494,12 @@ static hipError_t sieve_launch_t(const SieveArgs &a, hipStream_t stream) {
     if (!a.w_ortho) return hipGetLastError();
     if (a.sel) {
         // segments of whole vectors; their keys' list is the w_ortho buffer,
-        // which the last pass overwrites
+        // which the last pass overwrites (none where it holds the residual)
         const int64_t seg = ((n + kSelWgs - 1) / kSelWgs + 3) & ~int64_t(3);
         const unsigned wgs = (unsigned)((n + seg - 1) / seg);
         uint32_t *list = static_cast<uint32_t *>(a.w_ortho);
-        const int64_t cap = reinterpret_cast<uintptr_t>(a.w_ortho) % 4 == 0 ? n * (DT == ORTH_DT_F32 ? 4 : 2) / 4 / kSelWgs : 0;
+        const int64_t cap = !a.keep && reinterpret_cast<uintptr_t>(a.w_ortho) % 4 == 0
+                                ? n * (DT == ORTH_DT_F32 ? 4 : 2) / 4 / kSelWgs : 0;
         if (n % 4 == 0 && reinterpret_cast<uintptr_t>(a.score) % 16 == 0)
             hipLaunchKernelGGL((sieve_collect_kernel<4>), dim3(wgs), dim3(kSvNT), 0, stream, a.score, n, seg, a.sel,
                                a.rank, list, cap);
@@ -486,8 +508,27 @@ static hipError_t sieve_launch_t(const SieveArgs &a, hipStream_t stream) {
                                a.rank, list, cap);
         hipLaunchKernelGGL(sieve_refine_kernel, dim3(wgs), dim3(kSvNT), 0, stream, a.score, n, seg, a.sel, list, cap);
     }
-    hipLaunchKernelGGL((sieve_mask_kernel<DT, V, HL, S32>), dim3(rows), dim3(kSvNT), hb, stream, a);
+    if (a.keep) {
+        const int64_t wgs = (n + (int64_t)kSvNT * V - 1) / ((int64_t)kSvNT * V);
+        hipLaunchKernelGGL((sieve_apply_kernel<DT, V>), dim3((unsigned)(wgs < 4096 ? wgs : 4096)), dim3(kSvNT), 0,
+                           stream, a);
+    } else {
+        hipLaunchKernelGGL((sieve_mask_kernel<DT, V, HL, S32>), dim3(rows), dim3(kSvNT), hb, stream, a);
+    }
     return hipGetLastError();
+}
+
+// Whether two of the four buffers of a split share memory.
+static bool sieve_overlap(const SieveArgs &a, int dt) {
+    const int64_t n = a.N * a.K, e = dt == ORTH_DT_F32 ? 4 : 2;
+    const void *p[4] = {a.w, a.w_base, a.w_ortho, a.score};
+    const int64_t bytes[4] = {n * e, n * e, n * e, n * 4};
+    for (int i = 0; i < 4; i++)
+        for (int j = 0; j < i; j++) {
+            const char *b0 = static_cast<const char *>(p[i]), *b1 = static_cast<const char *>(p[j]);
+            if (b0 < b1 + bytes[j] && b1 < b0 + bytes[i]) return true;
+        }
+    return false;
 }
 
 template <int DT, bool S32>
@@ -538,6 +579,9 @@ hipError_t launch_sieve_split(const void *w, int dt, int64_t N, int64_t K, const
     a.rank = (uint32_t)rank;
     // rank 0: the reference keeps nothing (threshold max + 1)
     a.thresh = use_rank ? __builtin_nanf("") : thresh;
+    // in place (w_base or w_ortho is w): w is read in the first pass only,
+    // each element before it is written
+    a.keep = sieve_overlap(a, dt);
     return sieve_launch(a, dt, stream);
 }
 

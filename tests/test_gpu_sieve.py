@@ -121,6 +121,37 @@ def test_hessian_sieve_select_edges(gpu, dt, hdt, N, K, target, tied):
     assert bits_equal(wo, torch.from_numpy(wo_o))
 
 
+@pytest.mark.parametrize("dt,N,K,in_place", [
+    ("f32", 40, 260, "w_base"), ("f16", 30, 1027, "w_base"), ("bf16", 12, 8196, "w_base"),
+    ("f32", 1100, 260, "w_ortho"), ("f16", 30, 8196, "w_ortho"), ("bf16", 30, 1027, "w_ortho"),
+    ("f32", 30, 520, "score")])
+@pytest.mark.parametrize("rank", [0, 77, None])
+def test_split_in_place(gpu, dt, N, K, in_place, rank):
+    """orth_sieve_split_hip with an output that is w's own buffer gives the
+    results of separate buffers (rank None: a threshold)."""
+    from libortho_amd import _lib
+    w0 = make_w(dt, N, K, seed=9, device=gpu)
+    h = (torch.rand(K, generator=torch.Generator().manual_seed(8)) + 0.1).to(gpu)
+    L = _lib.lib()
+    code = {"f16": _lib.DT_F16, "bf16": _lib.DT_BF16, "f32": _lib.DT_F32}[dt]
+
+    def split(shared):
+        buf = {"w": w0.clone(), "w_base": torch.empty_like(w0), "w_ortho": torch.empty_like(w0),
+               "score": torch.empty(N, K, device=gpu)}
+        if shared:
+            buf[shared] = buf["w"]
+        sel = torch.empty(L.orth_sieve_select_bytes(), dtype=torch.uint8, device=gpu)
+        _lib.check(L.orth_sieve_split_hip(buf["w"].data_ptr(), code, N, K, h.data_ptr(), _lib.DT_F32, 1, _lib.DT_F32,
+                                          int(rank is not None), rank or 0, 1e-3, buf["w_base"].data_ptr(),
+                                          buf["w_ortho"].data_ptr(), buf["score"].data_ptr(), sel.data_ptr(), 0,
+                                          torch.cuda.current_stream().cuda_stream))
+        return buf
+    want, got = split(None), split(in_place)
+    assert want["w_ortho"].count_nonzero() > 0 or rank == 0
+    for name in ("w_base", "w_ortho", "score"):
+        assert bits_equal(got[name], want[name]), name
+
+
 def test_hessian_sieve_matrix_h_and_ties(gpu):
     """H_inv given as a matrix (its diagonal is used) and a score with many
     exact ties at the threshold (the k-th largest value is the same whatever

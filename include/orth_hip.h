@@ -74,7 +74,7 @@ typedef struct {
     const void *values;
     int32_t value_dtype;     /* orth_dtype_t: ORTH_DT_F16 or ORTH_DT_F32 */
     int32_t reserved;
-    int64_t count;           /* nnz */
+    int64_t count;           /* nnz, at most 2^31 - 4096 */
 } orth_hip_ortho_t;
 
 /* The dual-manifold layer.  Mirrors orth_layer_t,

@@ -115,6 +115,11 @@ int fail_hip(hipError_t e, const char *what) {
     return fail(ORTH_ERR_HIP, "%s: %s (%d)", what, hipGetErrorString(e), (int)e);
 }
 
+// The kernels step through a row's entries in int32, up to a few hundred past
+// its end before the comparison that stops them: the last counts of the int32
+// range would wrap there and read in front of the arrays.
+constexpr int64_t kMaxEntries = ((int64_t)1 << 31) - 4096;
+
 bool valid_dtype(int32_t d) { return d == ORTH_DT_F16 || d == ORTH_DT_BF16 || d == ORTH_DT_F32; }
 int64_t dtype_size(int32_t d) { return d == ORTH_DT_F32 ? 4 : 2; }
 
@@ -143,8 +148,9 @@ int resolve(const orth_hip_layer_t *L, const void *input, void *output, int64_t 
     if (b.scale_dtype != ORTH_DT_F16 && b.scale_dtype != ORTH_DT_F32)
         return fail(ORTH_ERR_INVALID_ARGUMENT, "scale_dtype must be F16 or F32 (got %d)", b.scale_dtype);
     if (o.count < 0) return fail(ORTH_ERR_INVALID_ARGUMENT, "ortho.count is negative");
-    if (o.count >= ((int64_t)1 << 31))
-        return fail(ORTH_ERR_UNSUPPORTED, "ortho.count exceeds the int32 CSR index range");
+    if (o.count > kMaxEntries)
+        return fail(ORTH_ERR_UNSUPPORTED, "ortho.count exceeds the int32 CSR index range (at most %lld entries)",
+                    (long long)kMaxEntries);
     if (o.count > 0) {
         if (!o.row_ptr || !o.col_indices || !o.values)
             return fail(ORTH_ERR_INVALID_ARGUMENT, "ortho has %lld entries but a NULL CSR buffer",

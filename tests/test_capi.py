@@ -122,6 +122,14 @@ def test_layer_validation_errors(L, mutate, status, needle):
     assert needle in _lib.last_error()
 
 
+def test_entry_counts_the_kernels_index_arithmetic_cannot_step_past(L):
+    """A row's loop runs up to a few hundred int32 indices past the row's end
+    before it stops: the last 4095 counts of the int32 range are refused."""
+    assert check(L, fake_layer(nnz=(1 << 31) - 4096)) == _lib.OK
+    assert check(L, fake_layer(nnz=(1 << 31) - 4095)) == _lib.ERR_UNSUPPORTED and "int32" in _lib.last_error()
+    assert check(L, fake_layer(nnz=(1 << 31) - 1)) == _lib.ERR_UNSUPPORTED
+
+
 def test_io_validation_errors(L):
     assert check(L, None) == _lib.ERR_INVALID_ARGUMENT and "NULL" in _lib.last_error()
     assert check(L, fake_layer(), M=-1) == _lib.ERR_INVALID_ARGUMENT

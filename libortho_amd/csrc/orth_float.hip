@@ -112,14 +112,26 @@ __global__ void __launch_bounds__(kFlNT) float_kernel(FloatArgs a) {
     Regs r0, r1;
     load(0, r0);
     load(1, r1);
-    for (int i = tid; i < kFlBN * a.ngroups; i += kFlNT) {
-        const int row = i / a.ngroups, gi = i - row * a.ngroups;
-        sl[gi * kFlBN + row] =
-            kBf16Q * load_as_f32(a.scales, a.scale_dtype, min(n0 + row, a.N - 1) * a.ngroups + gi);
-    }
+    // the weights' divisor goes into the scales, or (FP32 scales too large for
+    // that somewhere in the tile) multiplies the finished sums
+    auto scales = [&](float f) -> int {
+        int over = 0;
+        for (int i = tid; i < kFlBN * a.ngroups; i += kFlNT) {
+            const int row = i / a.ngroups, gi = i - row * a.ngroups;
+            const float v = load_as_f32(a.scales, a.scale_dtype, min(n0 + row, a.N - 1) * a.ngroups + gi);
+            sl[gi * kFlBN + row] = f * v;
+            over |= !__builtin_isfinite(f * v) && __builtin_isfinite(v) ? 1 : 0;
+        }
+        return over;
+    };
+    const int over = scales(kBf16Q);
     store(0, r0);
     load(2, r0);
-    __syncthreads();
+    const bool late = __syncthreads_or(over) != 0;  // (uniform)
+    if (late) {
+        scales(1.0f);
+        __syncthreads();
+    }
 
     f32x4 acc[2][4], part[2][4];
 #pragma unroll
@@ -227,7 +239,7 @@ __global__ void __launch_bounds__(kFlNT) float_kernel(FloatArgs a) {
         const float b = a.bias ? load_as_f32(a.bias, a.bias_dtype, n) : 0.f;
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            const f32x4 v = acc[u][j] + mine[(u * 4 + j) * 64];
+            const f32x4 v = (acc[u][j] + mine[(u * 4 + j) * 64]) * (late ? kBf16Q : 1.0f);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int64_t m = m0 + wm * 32 + 16 * u + 4 * g + i;
@@ -426,12 +438,12 @@ bool float_supported(const ForwardArgs &a) {
 
 // More than 64 KB of dynamic LDS must be allowed once per device and kernel
 // (the attribute call is idempotent, so two threads racing is harmless).
-static hipError_t float_allow_lds(const void *fn, std::atomic<int> *allowed) {
+static hipError_t float_allow_lds(const void *fn, int bytes, std::atomic<int> *allowed) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 64 || allowed[dev].load(std::memory_order_acquire)) return hipSuccess;
-    e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFoLdsMax);
+    e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e == hipSuccess) allowed[dev].store(1, std::memory_order_release);
     return e;
 }
@@ -439,7 +451,7 @@ static hipError_t float_allow_lds(const void *fn, std::atomic<int> *allowed) {
 template <int SPF>
 static hipError_t launch_float_dense(const FloatArgs &d, int64_t N, hipStream_t stream) {
     static std::atomic<int> allowed[64];
-    hipError_t e = float_allow_lds(reinterpret_cast<const void *>(float_kernel<SPF>), allowed);
+    hipError_t e = float_allow_lds(reinterpret_cast<const void *>(float_kernel<SPF>), 2 * kFlStage + kFlMaxGroups * kFlBN * 4, allowed);
     if (e != hipSuccess) return e;
     const uint32_t lds = 2 * kFlStage + (uint32_t)d.ngroups * kFlBN * 4;
     const unsigned blocks = (unsigned)(d.ntm * ((N + kFlBN - 1) / kFlBN));
@@ -450,7 +462,7 @@ static hipError_t launch_float_dense(const FloatArgs &d, int64_t N, hipStream_t 
 template <int TT, bool VH>
 static hipError_t launch_float_ortho(FloatOrthoArgs o, int cus, hipStream_t stream) {
     static std::atomic<int> allowed[64];
-    hipError_t e = float_allow_lds(reinterpret_cast<const void *>(float_ortho_kernel<TT, VH>), allowed);
+    hipError_t e = float_allow_lds(reinterpret_cast<const void *>(float_ortho_kernel<TT, VH>), (int)kFoLdsMax, allowed);
     if (e != hipSuccess) return e;
     const int64_t ntm = (o.M + TT - 1) / TT;
     const int64_t units = (o.N + kFoRows - 1) / kFoRows;

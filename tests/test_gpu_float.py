@@ -85,6 +85,27 @@ def test_float_products_past_the_range_times_a_scale_within_it(oracle_mod, M, K,
     assert np.isfinite(y).all() and (np.abs(y - ref) <= bound(lay, x, 0.0)).all()
 
 
+@pytest.mark.parametrize("K,N,M,G", [(256, 4400, 70, 128), (64, 2100, 130, None)])
+def test_float_scales_near_the_top_of_the_range(oracle_mod, K, N, M, G):
+    """FP32 scales past FLT_MAX / 1024 beside ordinary ones, in
+    some of the row tiles."""
+    lay = W.make_layer(K, N, G, 0.0, 7400)
+    x = W.make_x(M, K, 7401).astype(np.float32)
+    d = W.to_device(lay)
+    s = d["scales"].float()
+    big = torch.arange(0, N - 300, 37)
+    s[big.cuda()] *= 2.0 ** 123
+    y = torch.empty(M, N, dtype=torch.float32, device="cuda")
+    _C_ops.forward_planned(d["q"], s, d["vals"].float(), d["col"], d["row_ptr"], torch.from_numpy(x).cuda(), y, 1.0, None)
+    y = y.cpu().numpy()
+    ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 1.0)
+    err = bound(lay, x, 1.0)
+    f = np.ones(N)
+    f[big] = 2.0 ** 123
+    assert np.abs(s.cpu().numpy()).max() > 3.4e35 and np.abs(ref * f).max() < 3.4e38
+    assert np.isfinite(y).all() and (np.abs(y - ref * f) <= err * f).all()
+
+
 def test_float_infinities_and_nan_stay_with_their_token():
     K, N, M = 256, 4400, 70
     lay = W.make_layer(K, N, 128, 0.02, 7200)

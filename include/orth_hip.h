@@ -321,7 +321,7 @@ typedef struct {
 int orth_hip_device_info(int device, orth_hip_device_info_t *info);
 
 /* Kernel choice override for benchmarking and tests: 0 = automatic (the
- * default), 1 = decode, 2 = prefill, 3 = general, 4 = split-K mid-batch
+ * default), 1 = decode, 2 = prefill, 3 = general (the wave-per-row kernel), 4 = split-K mid-batch
  * (5..64 tokens), 5 = one-launch mid-batch (5..16 tokens), 6 = K quarters
  * over the grid (17..32 tokens, K = 4096), 7 = 1024-column slices over the
  * grid (1..32 tokens), 8 = the wide prefill kernel (any batch; its 256 x
@@ -339,6 +339,11 @@ int orth_hip_get_kernel_policy(void);
  * grid, 9 the same for a group of layers in one launch, 10 the wide
  * prefill kernel (256 x 352 or 256 x 128 tiles), 0 none. */
 int orth_hip_last_kernel(void);
+
+/* Of the kernels reported as 3 (general), the one that call launched: 1 the
+ * wave-per-row kernel (takes every call), 2 the rows kernel, 3 the FP32 tile
+ * kernel; 0 where the call took another kernel. */
+int orth_hip_last_variant(void);
 
 /* Device clock stamp for timing stream-ordered work (benchmarks; no
  * counterpart in the reference): launches ORTH_CLOCK_GROUPS workgroups on

@@ -43,7 +43,7 @@ _DT = {torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16, torch.float32: 
 # forward_layer and make_layer (descriptor reuse for OrthoLinear) stay internal;
 # forward_group takes make_layer descriptors (OrthoLinear.forward_group wraps it)
 __all__ = ["forward", "forward_planned", "forward_group", "build_plan", "dequant", "pack_base", "pack_csr", "sieve_quantize",
-           "sieve_split", "sieve_hdiag", "last_kernel", "set_kernel_policy", "get_kernel_policy", "device_info",
+           "sieve_split", "sieve_hdiag", "last_kernel", "last_variant", "set_kernel_policy", "get_kernel_policy", "device_info",
            "plan_cache_clear", "plan_cache_limit", "plan_cache_info"]
 
 
@@ -597,6 +597,12 @@ def last_kernel() -> str:
     tokens), prefill, general, or decode_group (one decode launch for the
     layers of a :func:`forward_group` call)."""
     return _lib.last_kernel()
+
+
+def last_variant() -> str:
+    """Of the kernels reported as ``general``, the one this thread's last
+    forward used: wave, rows or tiles (empty: it used another kernel)."""
+    return _lib.last_variant()
 
 
 set_kernel_policy = _lib.set_kernel_policy

@@ -23,6 +23,7 @@ STATUS_NAMES = {OK: "ORTH_OK", ERR_INVALID_ARGUMENT: "ORTH_ERR_INVALID_ARGUMENT"
 # kernel ids (orth_hip_last_kernel) and policies (orth_hip_set_kernel_policy)
 KERNEL_NAMES = {0: "none", 1: "decode", 2: "prefill", 3: "general", 4: "skinny", 5: "decode_group", 6: "mid", 7: "quarter",
                 8: "split", 9: "split_group", 10: "prefill_wide"}
+VARIANT_NAMES = {0: "", 1: "wave", 2: "rows", 3: "tiles"}  # of "general" (orth_hip_last_variant)
 GROUP_MAX = 4
 POLICIES = {"auto": 0, "decode": 1, "prefill": 2, "general": 3, "skinny": 4, "mid": 5, "quarter": 6, "split": 7, "prefill_wide": 8}
 
@@ -82,6 +83,7 @@ SIGNATURES = {
     "orth_hip_set_kernel_policy": (ctypes.c_int, [ctypes.c_int]),
     "orth_hip_get_kernel_policy": (ctypes.c_int, []),
     "orth_hip_last_kernel": (ctypes.c_int, []),
+    "orth_hip_last_variant": (ctypes.c_int, []),
     "orth_hip_last_error": (ctypes.c_char_p, []),
     "orth_hip_abi_version": (ctypes.c_int, []),
     "orth_hip_clock_stamp": (ctypes.c_int, [_P, _P]),
@@ -157,6 +159,10 @@ def last_error() -> str:
 
 def last_kernel() -> str:
     return KERNEL_NAMES.get(lib().orth_hip_last_kernel(), "?")
+
+
+def last_variant() -> str:
+    return VARIANT_NAMES.get(lib().orth_hip_last_variant(), "?")
 
 
 def set_kernel_policy(policy: str) -> None:

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "orth_common.h"
+#include "orth_general_shape.h"
 #include "orth_skinny_shape.h"
 
 namespace orth {
@@ -84,6 +85,7 @@ namespace {
 
 thread_local std::string t_error;
 thread_local int t_last_kernel = KERNEL_NONE;
+thread_local int t_last_variant = 0;
 
 int policy_from_env() {
     const char *e = std::getenv("ORTH_KERNEL_POLICY");
@@ -445,6 +447,7 @@ int forward_impl(const orth_hip_layer_t *layer, const void *plan, int64_t plan_b
                     (long long)plan_bytes, (long long)plan_bytes_for(a.N, a.K, a.nnz));
     if (batch == 0) {
         t_last_kernel = KERNEL_NONE;
+        t_last_variant = 0;
         return ORTH_OK;
     }
     int dev = 0;
@@ -453,8 +456,12 @@ int forward_impl(const orth_hip_layer_t *layer, const void *plan, int64_t plan_b
     hipStream_t stream = static_cast<hipStream_t>(stream_v);
 
     int kernel = KERNEL_NONE;
-    rc = pick_kernel(a, plan, g_policy.load(std::memory_order_relaxed), g_dev[dev].cus, &kernel);
+    const int policy = g_policy.load(std::memory_order_relaxed);
+    a.cus = g_dev[dev].cus;
+    rc = pick_kernel(a, plan, policy, a.cus, &kernel);
     if (rc != ORTH_OK) return rc;
+    // (policy 3 forces the wave-per-row kernel, which takes every call)
+    if (kernel == KERNEL_GENERAL) a.variant = policy == 3 ? (int)GENERAL_WAVE : general_variant(a, a.cus);
 
     // No-allocation calls share the device's scratch array: a call on a
     // stream other than the last one's first waits for that call (its
@@ -490,6 +497,7 @@ int forward_impl(const orth_hip_layer_t *layer, const void *plan, int64_t plan_b
     }
     if (rc != ORTH_OK) return rc;
     t_last_kernel = kernel;
+    t_last_variant = a.variant;
     return ORTH_OK;
 }
 
@@ -580,9 +588,7 @@ int launch_kernel(const ForwardArgs &a, const void *plan, int kernel, int dev, h
             e = pf(a.has_ortho ? plan : nullptr);
         }
     } else {
-        ForwardArgs g = a;
-        g.cus = g_dev[dev].cus;
-        e = launch_general(g, stream);
+        e = launch_general(a, stream);
     }
     if (e != hipSuccess) return fail_hip(e, "kernel launch");
     return rc;
@@ -623,6 +629,7 @@ int group_forward_impl(const orth_hip_layer_t *const *layers, const void *const 
     }
     if (batch == 0) {
         t_last_kernel = KERNEL_NONE;
+        t_last_variant = 0;
         return ORTH_OK;
     }
     int dev = 0;
@@ -640,6 +647,7 @@ int group_forward_impl(const orth_hip_layer_t *const *layers, const void *const 
         hipError_t e = launch_decode_group(as, pl, count, g_dev[dev].cus, static_cast<hipStream_t>(stream_v));
         if (e != hipSuccess) return fail_hip(e, "kernel launch");
         t_last_kernel = KERNEL_DECODE_GROUP;
+        t_last_variant = 0;
         return ORTH_OK;
     }
     // 17..32 tokens: one slice-split launch (and one reduction) for layers
@@ -666,6 +674,7 @@ int group_forward_impl(const orth_hip_layer_t *const *layers, const void *const 
             hipError_t e = launch_split_group(as, spl, count, part, stream);
             if (e != hipSuccess) return fail_hip(e, "kernel launch");
             t_last_kernel = KERNEL_SPLIT_GROUP;
+            t_last_variant = 0;
             return ORTH_OK;
         }
     }
@@ -970,6 +979,8 @@ int orth_hip_set_kernel_policy(int policy) {
 int orth_hip_get_kernel_policy(void) { return g_policy.load(); }
 
 int orth_hip_last_kernel(void) { return t_last_kernel; }
+
+int orth_hip_last_variant(void) { return t_last_variant; }
 
 const char *orth_hip_last_error(void) { return t_error.c_str(); }
 

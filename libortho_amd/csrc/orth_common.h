@@ -58,6 +58,7 @@ struct ForwardArgs {
     const void *bias = nullptr;  // [N] added to y after rounding, or null
     int bias_dtype = 0;
     int cus = 256;           // compute units of the device
+    int variant = 0;         // of KERNEL_GENERAL: a GeneralVariant
 };
 
 // ------------------------------------------------------ the sieve's select

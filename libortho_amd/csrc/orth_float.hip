@@ -37,15 +37,14 @@
 #include <type_traits>
 
 #include "orth_common.h"
+#include "orth_general_shape.h"
 
 namespace orth {
 
-constexpr int kFlBM = 64, kFlBN = 128, kFlBK = 64;
 constexpr int kFlNT = 512;
 constexpr int kFlPlane = kFlBM * kFlBK * 2;           // one bfloat16 part of the activations' stage
 constexpr int kFlW = kFlBN * kFlBK * 2;               // the weights' stage
 constexpr int kFlStage = 3 * kFlPlane + kFlW;         // 40 KB
-constexpr int kFlMaxGroups = 128;                     // scale groups the tile's LDS holds (64 KB)
 
 struct FloatArgs {
     const uint8_t *q;
@@ -251,10 +250,6 @@ __global__ void __launch_bounds__(kFlNT) float_kernel(FloatArgs a) {
 
 // ------------------------------------------------------------- sparse term
 
-constexpr int kFoNT = 1024;
-constexpr int kFoW = kFoNT / 64;
-constexpr int kFoRows = 16;                // rows per unit (one wave's)
-
 struct FloatOrthoArgs {
     const int32_t *row_ptr;
     const int32_t *col;
@@ -418,24 +413,6 @@ __global__ void __launch_bounds__(kFoNT) float_ortho_kernel(FloatOrthoArgs a) {
 
 // ------------------------------------------------------------------ host
 
-static const int64_t kFoLdsMax = 160 * 1024;
-
-// Tokens a sparse-term workgroup keeps in LDS (0: K is too large).
-static int float_ortho_tokens(int64_t K) {
-    for (int tt = 8; tt >= 1; tt /= 2)
-        if ((K + 1 + kFoRows * kFoW) * tt * 4 <= kFoLdsMax) return tt;
-    return 0;
-}
-
-bool float_supported(const ForwardArgs &a) {
-    if (a.io_dtype != ORTH_DT_F32 || a.K % kFlBK != 0) return false;
-    if (a.ngroups != 1 && (a.G % kFlBK != 0 || a.ngroups > kFlMaxGroups)) return false;
-    if (reinterpret_cast<uintptr_t>(a.x) & 15 || reinterpret_cast<uintptr_t>(a.q) & 7) return false;
-    if (a.has_ortho && float_ortho_tokens(a.K) == 0) return false;
-    const int64_t tiles = ((a.M + kFlBM - 1) / kFlBM) * ((a.N + kFlBN - 1) / kFlBN);
-    return a.M + a.N < ((int64_t)1 << 31) && tiles < ((int64_t)1 << 31);
-}
-
 // More than 64 KB of dynamic LDS must be allowed once per device and kernel
 // (the attribute call is idempotent, so two threads racing is harmless).
 static hipError_t float_allow_lds(const void *fn, int bytes, std::atomic<int> *allowed) {
@@ -465,10 +442,8 @@ static hipError_t launch_float_ortho(FloatOrthoArgs o, int cus, hipStream_t stre
     hipError_t e = float_allow_lds(reinterpret_cast<const void *>(float_ortho_kernel<TT, VH>), (int)kFoLdsMax, allowed);
     if (e != hipSuccess) return e;
     const int64_t ntm = (o.M + TT - 1) / TT;
-    const int64_t units = (o.N + kFoRows - 1) / kFoRows;
-    // about one workgroup per CU (its LDS holds one), each wave with work
     o.ntm = (int)ntm;
-    o.wgs = (int)std::max<int64_t>(1, std::min<int64_t>((units + kFoW - 1) / kFoW, cus / ntm));
+    o.wgs = (int)float_ortho_wgs(o.N, ntm, cus);
     const uint32_t lds = (uint32_t)((o.K + 1 + kFoRows * kFoW) * TT * 4);
     hipLaunchKernelGGL((float_ortho_kernel<TT, VH>), dim3((unsigned)(ntm * o.wgs)), dim3(kFoNT), lds, stream, o);
     return hipGetLastError();
@@ -476,10 +451,10 @@ static hipError_t launch_float_ortho(FloatOrthoArgs o, int cus, hipStream_t stre
 
 template <bool VH>
 static hipError_t launch_float_ortho_v(const FloatOrthoArgs &o, int cus, hipStream_t stream) {
-    const int tt = (int)std::min<int64_t>(float_ortho_tokens(o.K), o.M);
-    if (tt >= 8) return launch_float_ortho<8, VH>(o, cus, stream);
-    if (tt >= 4) return launch_float_ortho<4, VH>(o, cus, stream);
-    if (tt >= 2) return launch_float_ortho<2, VH>(o, cus, stream);
+    const int tt = float_ortho_tile(o.K, o.M);
+    if (tt == 8) return launch_float_ortho<8, VH>(o, cus, stream);
+    if (tt == 4) return launch_float_ortho<4, VH>(o, cus, stream);
+    if (tt == 2) return launch_float_ortho<2, VH>(o, cus, stream);
     return launch_float_ortho<1, VH>(o, cus, stream);
 }
 

@@ -15,6 +15,7 @@
 // when the activations are 16-byte aligned; otherwise a byte (2 nibbles) per
 // lane, as the shapes allow.
 #include "orth_common.h"
+#include "orth_general_shape.h"
 
 namespace orth {
 
@@ -161,26 +162,14 @@ static hipError_t launch_general_io(const ForwardArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-bool float_supported(const ForwardArgs &a);  // orth_float.hip
-hipError_t launch_float(const ForwardArgs &a, int cus, hipStream_t stream);
-bool rows_preferred(const ForwardArgs &a, int cus);  // orth_rows.hip
-hipError_t launch_rows(const ForwardArgs &a, int cus, hipStream_t stream);
+hipError_t launch_float(const ForwardArgs &a, int cus, hipStream_t stream);  // orth_float.hip
+hipError_t launch_rows(const ForwardArgs &a, int cus, hipStream_t stream);   // orth_rows.hip
 
+// a.variant: which of them (general_variant, or the wave-per-row kernel
+// where the policy forces it)
 hipError_t launch_general(const ForwardArgs &a, hipStream_t stream) {
-    const int cus = a.cus;
-    // FP32 activations, large batches: the tile kernels (orth_float.hip) take
-    // the same time for any batch of one round of their grid (~1 us per 64
-    // columns), the rows kernel's grows with M * N.  us, rows / float, alpha = 1:
-    // 4096 -> 4096 at 64 tokens 52 / 74, at 80 81 / 76, at 128 100 / 76; 4096 ->
-    // 11008 at 32 78 / 76; 1024 -> 4096 at 64 20 / 28, at 128 37 / 29; where
-    // only 4 tokens' columns fit the rows kernel's LDS, 8192 -> 1024 at 128
-    // 83 / 132, at 256 159 / 133, 11008 -> 4096 at 32 150 / 175, at 48 186 / 180.
-    // Without the rows kernel (FP32 scales or values) they cross the general
-    // kernel near 2^17: 4096 -> 4096 at 24 tokens 61 (general) / 72, at 32 80 / 72.
-    const bool rows = rows_preferred(a, cus);
-    const int64_t from = !rows ? 1 << 17 : a.K >= 8192 ? 200000 : 300000;
-    if (a.M * a.N >= from && float_supported(a)) return launch_float(a, cus, stream);
-    if (rows) return launch_rows(a, cus, stream);
+    if (a.variant == GENERAL_TILES) return launch_float(a, a.cus, stream);
+    if (a.variant == GENERAL_ROWS) return launch_rows(a, a.cus, stream);
     if (a.io_dtype == ORTH_DT_F32) return launch_general_io<ORTH_DT_F32>(a, stream);
     if (a.io_dtype == ORTH_DT_BF16) return launch_general_io<ORTH_DT_BF16>(a, stream);
     return launch_general_io<ORTH_DT_F16>(a, stream);

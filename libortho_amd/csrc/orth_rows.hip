@@ -35,16 +35,13 @@
 #include <atomic>
 
 #include "orth_common.h"
+#include "orth_general_shape.h"
 
 namespace orth {
 
-constexpr int kRwW = 8;            // waves
 constexpr int kRwNT = 64 * kRwW;
 constexpr int kRwD = 4;            // chunks of weights in flight
 constexpr int kRwXB = 8;           // 16-byte activation loads in flight per thread
-constexpr int kRwRS = 20;          // row stride of the partials in LDS, in floats
-constexpr int kRwMaxRB = 4;
-static const int64_t kRwLdsMax = 160 * 1024;
 
 struct RowsArgs {
     const uint8_t *q;
@@ -328,66 +325,6 @@ __global__ void __launch_bounds__(kRwNT) rows_kernel(RowsArgs a) {
 }
 
 // ------------------------------------------------------------------ host
-
-struct RowsShape {
-    int rb, mt, tl, tiles, lds, gx, npass;
-    bool wide;
-};
-
-static bool rows_shape(const ForwardArgs &a, int cus, RowsShape &sh) {
-    if (a.K % 8 != 0 || a.K < 32 || a.N >= ((int64_t)1 << 31)) return false;
-    if (a.K > 65408) return false;  // an entry holds its activation's place, at most K rounded up to 128, in 16 bits
-    if (a.scale_dtype != ORTH_DT_F16 || (a.has_ortho && a.val_dtype != ORTH_DT_F16)) return false;
-    if (a.ngroups != 1 && a.G % 32 != 0) return false;
-    if ((reinterpret_cast<uintptr_t>(a.x) & 15) || (reinterpret_cast<uintptr_t>(a.q) & 3)) return false;
-    sh.wide = a.K % 32 == 0 && (reinterpret_cast<uintptr_t>(a.q) & 15) == 0 && (a.ngroups == 1 || a.G % 128 == 0);
-    const int64_t kp = (a.K + 127) / 128 * 128;
-    const int64_t tok = a.io_dtype == ORTH_DT_F32 ? (kp + 4) * 4 : (kp + 8) * 2;  // LDS bytes of a token
-    const int64_t nblk = (a.N + 15) / 16;
-    // one workgroup per CU where the rows allow it, each looping over its
-    // passes with the activations staged once.  More blocks per pass share
-    // the reading (and cutting) of the activations and the pass's barriers:
-    // a pass costs about 1.5 blocks beside its own (narrow rows: registers
-    // for 3 blocks, with FP32 activations 2)
-    int64_t best = 0;
-    const int max_rb = sh.wide ? kRwMaxRB : a.io_dtype == ORTH_DT_F32 ? 2 : 3;
-    for (int rb = 1; rb <= max_rb; rb++) {
-        const int64_t red = (int64_t)5 * rb * 16 * kRwRS * 4 + 16;
-        const int64_t fit = std::min<int64_t>(16, (kRwLdsMax - red) / tok);
-        if (fit < 1) break;
-        const int64_t tiles = (a.M + fit - 1) / fit;
-        if (tiles > 65535) break;
-        const int64_t npass = (nblk + rb - 1) / rb;
-        const int64_t gx = std::min<int64_t>(npass, std::max<int64_t>(1, cus / tiles));
-        const int64_t rounds = (tiles * gx + cus - 1) / cus;
-        const int64_t cost = rounds * ((npass + gx - 1) / gx) * (2 * rb + 3);
-        if (best && cost >= best) continue;
-        best = cost;
-        sh.rb = rb;
-        sh.tiles = (int)tiles;
-        sh.mt = (int)((a.M + tiles - 1) / tiles);
-        sh.lds = (int)(((sh.mt * tok + 15) & ~int64_t(15)) + red);
-        sh.npass = (int)npass;
-        sh.gx = (int)gx;
-    }
-    if (!best) return false;
-    sh.tl = 1;
-    while (sh.tl < sh.mt) sh.tl *= 2;
-    return true;
-}
-
-// Whether this kernel takes the call: its shape, and enough outputs to pay
-// for the staging and its barrier.  The general kernel's time grows with
-// M * N, this one's hardly below 16 tokens (us, general / this): FP32 4096 ->
-// 4096 at 2 tokens 10.2 / 11.4, at 4 14.6 / 12.3, 4096 -> 11008 at 1 18.8 /
-// 22.3, at 2 25.0 / 22.0, at 8 66 / 24.9; FP16 4000 -> 4096 at 1 10.8 / 11.2,
-// 4000 -> 11008 at 1 20.3 / 13.5, at 16 139 / 18.5; narrow rows (2720 -> 4096,
-// group 32) at 4 12.9 / 12.4, at 16 37.8 / 16.4.
-bool rows_preferred(const ForwardArgs &a, int cus) {
-    RowsShape sh;
-    if (!rows_shape(a, cus, sh)) return false;
-    return a.M * a.N >= (!sh.wide ? 24576 : a.io_dtype == ORTH_DT_F32 ? 16384 : 8192);
-}
 
 template <int IO, int RB, bool WIDE>
 static hipError_t rows_launch_t(const RowsArgs &d, const RowsShape &sh, hipStream_t stream) {

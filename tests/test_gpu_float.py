@@ -6,20 +6,24 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
-from libortho_amd import _C_ops  # noqa: E402
+from libortho_amd import _C_ops, _lib  # noqa: E402
 from libortho_amd import workloads as W  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
 
-def run(lay, x, alpha, bias=None, wide=False):
+def run(lay, x, alpha, bias=None, wide=False, variant="tiles", policy="auto"):
     d = W.to_device(lay)
     if wide:  # FP32 scales and values
         d["scales"], d["vals"] = d["scales"].float(), d["vals"].float()
     xd = torch.from_numpy(x).cuda()
     y = torch.empty(x.shape[0], lay.N, dtype=torch.float32, device="cuda")
-    _C_ops.forward_planned(d["q"], d["scales"], d["vals"], d["col"], d["row_ptr"], xd, y, alpha, None, bias=bias)
-    assert _C_ops.last_kernel() == "general"
+    _lib.set_kernel_policy(policy)
+    try:
+        _C_ops.forward_planned(d["q"], d["scales"], d["vals"], d["col"], d["row_ptr"], xd, y, alpha, None, bias=bias)
+    finally:
+        _lib.set_kernel_policy("auto")
+    assert (_C_ops.last_kernel(), _C_ops.last_variant()) == ("general", variant)
     return y.cpu().numpy()
 
 
@@ -55,7 +59,7 @@ def bound(lay, x, alpha):
 def test_float_parity(oracle_mod, K, N, group, M, density, alpha, wide):
     lay = W.make_layer(K, N, group, density, 7000 + K + M)
     x = np.random.Generator(np.random.PCG64(M)).normal(0, 1, (M, K)).astype(np.float32)
-    y = run(lay, x, alpha, wide=wide)
+    y = run(lay, x, alpha, wide=wide, variant="wave" if wide and M * N < 1 << 17 else "tiles")
     ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, alpha)
     assert np.isfinite(y).all()
     assert (np.abs(y - ref) <= bound(lay, x, alpha)).all()
@@ -81,7 +85,7 @@ def test_float_products_past_the_range_times_a_scale_within_it(oracle_mod, M, K,
     x[:, ::32] = np.random.Generator(np.random.PCG64(2)).uniform(-6e37, 6e37, (M, K // 32))
     ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 0.0)
     assert np.abs(ref).max() < 3e38
-    y = run(lay, x, 0.0)
+    y = run(lay, x, 0.0, variant="tiles" if M == 130 else "rows")
     assert np.isfinite(y).all() and (np.abs(y - ref) <= bound(lay, x, 0.0)).all()
 
 
@@ -97,6 +101,7 @@ def test_float_scales_near_the_top_of_the_range(oracle_mod, K, N, M, G):
     s[big.cuda()] *= 2.0 ** 123
     y = torch.empty(M, N, dtype=torch.float32, device="cuda")
     _C_ops.forward_planned(d["q"], s, d["vals"].float(), d["col"], d["row_ptr"], torch.from_numpy(x).cuda(), y, 1.0, None)
+    assert _C_ops.last_variant() == "tiles"
     y = y.cpu().numpy()
     ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 1.0)
     err = bound(lay, x, 1.0)
@@ -151,3 +156,16 @@ def test_float_odd_csr_and_bias(oracle_mod):
     y = run(lay, x, 1.0)
     lay.col[~keep] = 0
     assert (np.abs(y - x.astype(np.float64) @ w.T) <= bound(lay, x, 1.0)).all()
+
+
+@pytest.mark.parametrize("K,N,M,variant", [(512, 2400, 130, "tiles"), (2048, 4096, 12, "rows")])
+def test_the_general_policy_forces_the_wave_per_row_kernel(oracle_mod, K, N, M, variant):
+    """Policy "general" takes the kernel that takes every call, also where the
+    automatic choice is another of those reported as general."""
+    lay = W.make_layer(K, N, 128, 0.02, 7500)
+    x = W.make_x(M, K, 7501).astype(np.float32)
+    a = run(lay, x, 1.0, variant=variant)
+    b = run(lay, x, 1.0, variant="wave", policy="general")
+    ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 1.0)
+    for y in (a, b):
+        assert (np.abs(y - ref) <= bound(lay, x, 1.0)).all()

@@ -27,7 +27,7 @@ def run(lay, x, alpha, dtype, bias=None):
     xd = torch.from_numpy(x).cuda().to(dtype)
     y = torch.empty(x.shape[0], lay.N, dtype=dtype, device="cuda")
     _C_ops.forward_planned(d["q"], d["scales"], d["vals"], d["col"], d["row_ptr"], xd, y, alpha, None, bias=bias)
-    assert _C_ops.last_kernel() == "general"
+    assert (_C_ops.last_kernel(), _C_ops.last_variant()) == ("general", "rows")
     return y
 
 

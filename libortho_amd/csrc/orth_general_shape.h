@@ -108,30 +108,82 @@ inline bool float_supported(const ForwardArgs &a) {
 }
 
 // ----------------------------------------------------------------- choice
+//
+// The kernels' times in microseconds, from the shapes of their loops.  The
+// constants are a least-squares fit to MI355X times of calls whose weights
+// come from HBM: 14,255 wave-per-row, 13,934 rows and 4,761 tile calls over K
+// 256 .. 30000, N 512 .. 28672, 1 .. 256 tokens, 0 .. 20 % ortho, FP16 and
+// FP32 activations; they are off by 10, 8 and 6 % (rms).
 
-// The general kernel a call takes.  FP32 activations, large batches: the tile
-// kernel takes the same time for any batch of one round of its grid (~1 us per
-// 64 columns), the rows kernel's grows with M * N.  us, rows / tiles, alpha = 1:
-// 4096 -> 4096 at 64 tokens 52 / 74, at 80 81 / 76, at 128 100 / 76; 4096 ->
-// 11008 at 32 78 / 76; 1024 -> 4096 at 64 20 / 28, at 128 37 / 29; where
-// only 4 tokens' columns fit the rows kernel's LDS, 8192 -> 1024 at 128
-// 83 / 132, at 256 159 / 133, 11008 -> 4096 at 32 150 / 175, at 48 186 / 180.
-// Without the rows kernel (FP32 scales or values) they cross the wave-per-row
-// kernel near 2^17: 4096 -> 4096 at 24 tokens 61 (wave) / 72, at 32 80 / 72.
-// The rows kernel needs enough outputs to pay for the staging and its barrier:
-// the wave-per-row kernel's time grows with M * N, its hardly below 16 tokens
-// (us, wave / rows): FP32 4096 -> 4096 at 2 tokens 10.2 / 11.4, at 4 14.6 /
-// 12.3, 4096 -> 11008 at 1 18.8 / 22.3, at 2 25.0 / 22.0, at 8 66 / 24.9; FP16
-// 4000 -> 4096 at 1 10.8 / 11.2, 4000 -> 11008 at 1 20.3 / 13.5, at 16 139 /
-// 18.5; narrow rows (2720 -> 4096, group 32) at 4 12.9 / 12.4, at 16 37.8 /
-// 16.4.
+inline double ceil_div(double a, double b) { return std::ceil(a / b); }
+
+// A wave per row and token tile: its own steps (512 columns, 64 entries) one
+// after the other, beside those of all waves.
+inline double wave_us(const ForwardArgs &a, int cus) {
+    static const double step[3] = {0.55, 0.78, 1.0}, steps[3] = {1.1, 1.9, 2.9}, row[3] = {0.43, 0.64, 1.9},
+                        ent[3] = {0.49, 1.2, 2.4};
+    const int k = a.M <= 1 ? 0 : a.M == 2 ? 1 : 2;  // tiles of 1, 2 and 4 tokens
+    const double waves = (double)a.N * ceil_div((double)a.M, 1 << k) * 1e-4, rows = a.N * 1e-4;
+    const double it = ceil_div((double)a.K, 512), se = a.has_ortho ? ceil_div((double)a.nnz, 64.0 * a.N) : 0;
+    const double one = it * step[k] + 0.9 * se;
+    const double all = (waves * (it * steps[k] + row[k] + se * ent[k]) + rows * (0.9 * it + 1.8 * se)) * 256 / cus;
+    return 2.8 + std::sqrt(one * one + all * all);
+}
+
+// Staging once per workgroup, then its passes: chunks (wide rows' loads go four
+// at a time, also where a wave has fewer; narrow rows of several groups load
+// and place four scales a chunk) and entries.
+inline double rows_us(const ForwardArgs &a, const RowsShape &sh, int cus) {
+    const bool f32 = a.io_dtype == ORTH_DT_F32;
+    const double rounds = ceil_div((double)sh.tiles * sh.gx, cus), passes = ceil_div(sh.npass, sh.gx);
+    const double nch = ceil_div((double)a.K, 128), cpw = ceil_div(nch, kRwW);
+    const double busy = ceil_div(nch, cpw) / kRwW;  // waves with chunks
+    const double chunks = sh.wide ? 0.074 * cpw + 1.4 * ceil_div(cpw, 4) * busy : (a.ngroups > 1 ? 1.6 : 0.59) * cpw;
+    const double dense = sh.rb * chunks + (f32 ? 0.65 * cpw : 0);
+    const double sparse = !a.has_ortho ? 0 : sh.rb * (0.0023 * (double)a.nnz / a.N * sh.tl + 1.3 * ceil_div((double)a.nnz, 64.0 * a.N));
+    const double start = 3.0 + sh.rb * (sh.wide ? 1.1 : 3.8) + 1.5 * sh.mt * (double)a.K * (f32 ? 4 : 2) / 65536;
+    const double pass = 3.0 + (sh.wide ? 0 : 2.3 * sh.rb);
+    return rounds * (start + passes * (dense + sparse) + (passes - 1) * pass) +
+           0.058e-6 * sh.tiles * (double)a.N * a.K / 2;
+}
+
+// Rounds of the tile grid, and of the sparse launch: its staging, then a
+// wave's units of 16 rows, 48 entries of a row at a time.
+inline double tiles_us(const ForwardArgs &a, int cus) {
+    const double tiles = ceil_div((double)a.M, kFlBM) * ceil_div((double)a.N, kFlBN);
+    double t = ceil_div(tiles, cus) * (6.1 + 0.89 * (double)(a.K / kFlBK));
+    if (!a.has_ortho) return t;
+    const int tt = float_ortho_tile(a.K, a.M);
+    const int64_t ntm = (a.M + tt - 1) / tt, wgs = float_ortho_wgs(a.N, ntm, cus);
+    const double units = ceil_div(ceil_div((double)a.N, kFoRows), (double)wgs * kFoW);
+    const double unit = 0.0023 * (double)a.nnz / a.N * tt + 2.2 * ceil_div((double)a.nnz, 48.0 * a.N) + 2.0;
+    return t + ceil_div((double)ntm * wgs, cus) * (3.5 * (double)a.K * tt * 4 / 65536 + units * unit);
+}
+
+// The general kernel a call takes: the one with the smallest of these times
+// (the wave-per-row one within 3 %, at one token 20 %: it gains more from
+// weights in cache, FP32 4096 -> 4096 at 1 token 10.9 / 12.1 then).
+// us, wave / rows / tiles, at 1 % unless said: FP32 4096 -> 4096, 1 token 12.8 /
+// 12.5 / 67, 4 tokens 20.5 / 13.4 / 70, 64 tokens 173 / 57 / 73, 128 tokens 348 /
+// 106 / 74; FP32 4096 -> 11008, 1 token 24.8 / 24.3; FP32 8192 -> 1024, 128
+// tokens 194 / 88 / 133, 256 tokens 355 / 165 / 133; FP32 28672 -> 1024 without
+// ortho, 24 tokens 101 / 155; FP32 1024 -> 1024 at 20 %, 16 tokens 11.7 / 20.3;
+// FP16 4000 -> 11008, 1 token 25.2 / 17.6, 16 tokens 140 / 20.7; FP16 1344 ->
+// 11008 in groups of 96 without ortho, 4 tokens 22.6 / 25.8, 16 tokens 54 / 26.
+// (Lines at a fixed M * N sent calls with more entries, more columns or
+// narrower rows than the ones they were drawn from to a kernel up to 4.8 times
+// slower; by these times the chosen one is 0.5 % off the best on average, and
+// in 0.5 % of the calls above more than 10 % slower than the wave-per-row one.)
 inline int general_variant(const ForwardArgs &a, int cus) {
+    int v = GENERAL_WAVE;
+    double best = wave_us(a, cus) / (a.M == 1 ? 1.2 : 1.03);
     RowsShape sh;
-    const bool rows = rows_shape(a, cus, sh) &&
-                      a.M * a.N >= (!sh.wide ? 24576 : a.io_dtype == ORTH_DT_F32 ? 16384 : 8192);
-    const int64_t from = !rows ? 1 << 17 : a.K >= 8192 ? 200000 : 300000;
-    if (a.M * a.N >= from && float_supported(a)) return GENERAL_TILES;
-    return rows ? GENERAL_ROWS : GENERAL_WAVE;
+    if (rows_shape(a, cus, sh)) {
+        const double t = rows_us(a, sh, cus);
+        if (t < best) best = t, v = GENERAL_ROWS;
+    }
+    if (float_supported(a) && tiles_us(a, cus) < 1.03 * best) v = GENERAL_TILES;  // (the surer estimate)
+    return v;
 }
 
 }  // namespace orth

@@ -45,21 +45,20 @@ def bound(lay, x, alpha):
     return adds * 2.0 ** -23 * (np.abs(x).astype(np.float64) @ w.T) + 1e-30
 
 
-# the dispatch's edges (M * N = 2^17 with FP32 scales, else 200,000 or
-# 300,000), ragged token and row tiles, one K step, odd and even steps per
+# ragged token and row tiles, one K step, odd and even steps per
 # scale group, one scale per row over an odd number of steps, 8 / 4 / 2 tokens
 # per sparse workgroup (K = 4096, 9216, 11008), more entries per row than one
 # batch of loads holds, FP32 scales and values
 @pytest.mark.parametrize("K,N,group,M,density,alpha,wide", [
     (4096, 1024, 128, 127, 0.01, 1.0, True), (4096, 1024, 128, 128, 0.01, 1.0, True),
-    (4096, 1200, 128, 250, 0.01, 1.0, False), (64, 4650, 64, 65, 0.05, 1.0, False),
+    (4096, 1200, 128, 378, 0.01, 1.0, False), (64, 4650, 64, 65, 0.05, 1.0, False),
     (192, 2333, 192, 129, 0.05, 0.5, False), (320, 1111, None, 130, 0.2, 1.0, True),
-    (1024, 1600, 256, 191, 0.0, 1.0, False), (9216, 1000, 128, 253, 0.01, 1.0, False),
+    (1024, 1600, 256, 319, 0.0, 1.0, False), (9216, 1000, 128, 253, 0.01, 1.0, False),
     (11008, 1010, 128, 200, 0.02, 1.0, False), (8192, 460, 64, 440, 0.01, 0.0, False)])
 def test_float_parity(oracle_mod, K, N, group, M, density, alpha, wide):
     lay = W.make_layer(K, N, group, density, 7000 + K + M)
     x = np.random.Generator(np.random.PCG64(M)).normal(0, 1, (M, K)).astype(np.float32)
-    y = run(lay, x, alpha, wide=wide, variant="wave" if wide and M * N < 1 << 17 else "tiles")
+    y = run(lay, x, alpha, wide=wide)
     ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, alpha)
     assert np.isfinite(y).all()
     assert (np.abs(y - ref) <= bound(lay, x, alpha)).all()
@@ -76,16 +75,18 @@ def test_float_small_and_large_activations_keep_their_bits(oracle_mod):
     assert (np.abs(run(lay, x, 1.0) - ref) <= bound(lay, x, 1.0)).all()
 
 
-@pytest.mark.parametrize("M,K,N,G", [(130, 512, 2400, 128), (3, 512, 8200, None), (20, 480, 2400, 32)])
-def test_float_products_past_the_range_times_a_scale_within_it(oracle_mod, M, K, N, G):
+@pytest.mark.parametrize("M,K,N,G,variant", [(130, 512, 2400, 128, "tiles"), (3, 512, 8200, None, "wave"),
+                                             (20, 480, 2400, 32, "wave"), (12, 2048, 4096, 128, "rows"),
+                                             (64, 480, 4800, 32, "rows")])
+def test_float_products_past_the_range_times_a_scale_within_it(oracle_mod, M, K, N, G, variant):
     """|q x| up to 4.8e38 overflows FP32, scale * q * x does not (tile kernel,
-    rows kernel with wide and narrow rows)."""
+    rows kernel with wide and narrow rows, wave-per-row kernel)."""
     lay = W.make_layer(K, N, G, 0.02, 7300)
     x = np.zeros((M, K), np.float32)
     x[:, ::32] = np.random.Generator(np.random.PCG64(2)).uniform(-6e37, 6e37, (M, K // 32))
     ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 0.0)
     assert np.abs(ref).max() < 3e38
-    y = run(lay, x, 0.0, variant="tiles" if M == 130 else "rows")
+    y = run(lay, x, 0.0, variant=variant)
     assert np.isfinite(y).all() and (np.abs(y - ref) <= bound(lay, x, 0.0)).all()
 
 

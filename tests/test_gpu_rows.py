@@ -22,12 +22,12 @@ def within(y, ref, sums, dtype):
     return (np.abs(y - ref) <= sums + np.maximum(EPS[dtype] * (np.abs(ref) + sums), TINY[dtype])).all()
 
 
-def run(lay, x, alpha, dtype, bias=None):
+def run(lay, x, alpha, dtype, bias=None, variant="rows"):
     d = W.to_device(lay)
     xd = torch.from_numpy(x).cuda().to(dtype)
     y = torch.empty(x.shape[0], lay.N, dtype=dtype, device="cuda")
     _C_ops.forward_planned(d["q"], d["scales"], d["vals"], d["col"], d["row_ptr"], xd, y, alpha, None, bias=bias)
-    assert (_C_ops.last_kernel(), _C_ops.last_variant()) == ("general", "rows")
+    assert (_C_ops.last_kernel(), _C_ops.last_variant()) == ("general", variant)
     return y
 
 
@@ -44,24 +44,43 @@ def run(lay, x, alpha, dtype, bias=None):
     (960, 2048, 96, 15, 0.02, F16), (448, 13000, 64, 2, 0.02, BF16), (4096, 4096, 128, 4, 0.01, F32),
     (4096, 2100, 128, 16, 0.02, F32), (4096, 8191, None, 17, 0.01, F32), (11008, 4096, 128, 7, 0.01, F32),
     (4000, 4100, None, 9, 0.02, F32), (2720, 4100, 32, 9, 0.02, F32), (1000, 13000, None, 2, 0.02, F32),
+    (2720, 9000, 32, 17, 0.01, BF16), (448, 13000, 64, 16, 0.02, BF16), (1000, 13000, None, 16, 0.02, F32),
     (16384, 1030, 256, 16, 0.005, F32)])
 def test_rows_parity(gpu, oracle_mod, K, N, group, M, density, dtype):
     lay = W.make_layer(K, N, group, density, 7500 + K + M)
     x = torch.from_numpy(W.make_x(M, K, 7501 + M)).to(dtype).float().numpy()
     if dtype == F32:
         x = np.random.Generator(np.random.PCG64(M)).normal(0, 1, (M, K)).astype(np.float32)
+    small = (K, M) in ((448, 2), (1000, 2), (2720, 4))  # (left to the wave-per-row kernel)
     for alpha in (1.0, 0.0):
-        y = run(lay, x, alpha, dtype).float().cpu().numpy()
+        y = run(lay, x, alpha, dtype, variant="wave" if small else "rows").float().cpu().numpy()
         ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, alpha)
         sums = bound(lay, x, alpha)
         assert within(y, ref, sums, dtype)
+
+
+# either side of the choice's lines, in calls whose times are well apart:
+# few and many tokens, entries and columns, wide and narrow rows, FP32 scales
+@pytest.mark.parametrize("K,N,group,M,density,dtype,variant", [
+    (4096, 4096, 128, 4, 0.01, F32, "rows"), (4096, 4096, 128, 64, 0.01, F32, "rows"),
+    (4096, 4096, 128, 128, 0.01, F32, "tiles"), (8192, 1024, 128, 128, 0.01, F32, "rows"),
+    (1024, 1024, 128, 4, 0.01, F32, "wave"), (1024, 1024, 128, 16, 0.2, F32, "wave"),
+    (28672, 1024, 128, 24, 0.0, F32, "wave"), (1344, 11008, 96, 4, 0.0, F16, "wave"),
+    (1344, 11008, 96, 16, 0.0, F16, "rows"), (4000, 11008, None, 1, 0.01, BF16, "rows"),
+    (30000, 1024, None, 48, 0.02, F16, "wave")])
+def test_general_choice(gpu, oracle_mod, K, N, group, M, density, dtype, variant):
+    lay = W.make_layer(K, N, group, density, 7900 + K)
+    x = torch.from_numpy(W.make_x(M, K, 7901)).to(dtype).float().numpy()
+    y = run(lay, x, 1.0, dtype, variant=variant).float().cpu().numpy()
+    ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, 1.0)
+    assert within(y, ref, bound(lay, x, 1.0), dtype)
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16, F32])
 def test_rows_odd_csr_bias_and_infinities(gpu, oracle_mod, dtype):
     """Duplicate, unsorted and out-of-range columns as given; the bias added
     to the rounded output; an infinity or a NaN stays with its token."""
-    K, N, M = 480, 5000, 6
+    K, N, M = 480, 5000, 12
     lay = W.make_layer(K, N, None, 0.05, 7600)
     lay.col[:] = lay.col[::-1].copy()
     lay.col[::7] = lay.col[3]
@@ -77,7 +96,7 @@ def test_rows_odd_csr_bias_and_infinities(gpu, oracle_mod, dtype):
     bad = x.copy()
     bad[1, 5], bad[4, 479] = np.inf, np.nan
     z = run(lay, bad, 1.0, dtype)
-    keep = [0, 2, 3, 5]
+    keep = [m for m in range(M) if m not in (1, 4)]
     assert torch.equal(z[keep], y[keep]) and torch.isnan(z[4]).all() and not torch.isfinite(z[1]).any()
     lay.col[::11] = K + 5
     lay.col[1::11] = -3

@@ -164,13 +164,22 @@ __device__ __forceinline__ uint32_t value_bits_f16(const void *vals, int dtype, 
 constexpr int kPlanNT = 1024;
 constexpr int kPlanWRows = kPlanBN / (kPlanNT / 64);  // rows per wave
 
+// x of lane i (uniform), and of the lane below (lane 0: 0): register moves,
+// where a shuffle is an LDS round trip.  Called with every lane active.
+__device__ __forceinline__ int32_t lane_i32(int32_t x, int i) { return __builtin_amdgcn_readlane(x, i); }
+__device__ __forceinline__ int32_t lane_below(int32_t x) {
+    return __builtin_amdgcn_update_dpp(0, x, 0x138, 0xf, 0xf, false);  // wave_shr:1
+}
+
 // One workgroup per block of kPlanBN output rows.  Counting sort of the
 // block's CSR entries by 64-column step, stable in (row, CSR position).  A
 // wave takes 8 rows, 64 entries of a row at a time: in a row whose columns
 // ascend strictly the entries of a step are consecutive, so an entry's place
-// among them is its distance from the first.  Other rows are walked entry by
-// entry by one lane.  (Each row walked by one thread, three times, with the
-// chunk table on the way: 72 us for 4096 -> 11008 at 1 %.)
+// among them is its distance from the first.  In other rows it is the number of
+// earlier lanes with the step, counted lane by lane (one lane walking the wave's
+// rows in turn: the plan of 4160 -> 4096, columns descending, 262 us at 1 % and
+// 1,212 at 5 %, now 60 and 166).  (Each row walked by one thread, three times, with the chunk
+// table on the way: 72 us for 4096 -> 11008 at 1 %, ascending.)
 __global__ void __launch_bounds__(kPlanNT) plan_build_kernel(ForwardArgs a, PlanHeader *h,
                                                              int32_t *offsets, uint32_t *entries, int nksteps) {
     extern __shared__ __align__(16) int32_t cnt[];  // [nksteps][BN]
@@ -183,53 +192,68 @@ __global__ void __launch_bounds__(kPlanNT) plan_build_kernel(ForwardArgs a, Plan
     for (int i = tid; i < L; i += kPlanNT) cnt[i] = 0;
     if (tid == 0) s_flags = 0;
 
-    // the rows' ranges (row_ptr of rows 8 w .. 8 w + 8 in lanes 0 .. 8) and first 64 columns
+    // the rows' ranges (row_ptr of rows 8 w .. 8 w + 8 in lanes 0 .. 8), first
+    // 64 columns and their values
     const int64_t n0 = b * kPlanBN + wave * kPlanWRows;
     const int32_t rp = a.row_ptr[min(n0 + min(lane, kPlanWRows), a.N)];
     uint32_t myflags = 0;
     int32_t rs[kPlanWRows], re[kPlanWRows], c0[kPlanWRows];
+    uint32_t v0[kPlanWRows];
 #pragma unroll
     for (int i = 0; i < kPlanWRows; i++) {
-        const int32_t ra = __shfl(rp, i), rb = __shfl(rp, i + 1), nnz = (int32_t)a.nnz;
+        const int32_t ra = lane_i32(rp, i), rb = lane_i32(rp, i + 1), nnz = (int32_t)a.nnz;
         const bool live = n0 + i < a.N;
         if (live && (ra < 0 || rb < ra || rb > nnz)) myflags |= kPlanMalformed;
         rs[i] = min(max(ra, 0), nnz);  // (csr_row_range)
         re[i] = live ? min(max(rb, rs[i]), nnz) : rs[i];
-        c0[i] = a.col[min((int64_t)rs[i] + lane, (int64_t)max(re[i] - 1, 0))];
+        const int64_t j = min((int64_t)rs[i] + lane, (int64_t)max(re[i] - 1, 0));
+        c0[i] = a.col[j];
+        v0[i] = value_bits_f16(a.vals, a.val_dtype, j);
         if (re[i] - rs[i] > 65535) myflags |= kPlanUnsorted;  // counts past 16 bits
     }
     __syncthreads();  // the counters are zero
 
-    uint32_t slow = 0;  // rows whose columns do not ascend strictly (uniform)
+    // rows whose columns do not ascend strictly, and rows of more than one
+    // batch (uniform); every row's first batch is taken in straight-line code,
+    // so that the rows' LDS round trips overlap
+    uint32_t slow = 0, more = 0;
 #pragma unroll
     for (int i = 0; i < kPlanWRows; i++) {
-        const int r = wave * kPlanWRows + i;
-        bool bad = false;
-        int32_t last = INT32_MIN;
-        for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
-            const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
-            const int32_t up = __shfl_up(c, 1);
-            if (jb + lane < re[i] && c <= (lane ? up : last) && (lane || jb > rs[i])) bad = true;
-            last = __shfl(c, 63);
-        }
-        if (__ballot(bad)) {
-            slow |= 1u << i;
-            if (lane == 0) {
-                myflags |= kPlanUnsorted;
-                int32_t prev = -1;
-                for (int32_t j = rs[i]; j < re[i]; j++) {
-                    const int32_t c = a.col[j];
-                    if (c >= 0 && c < a.K) {
-                        cnt[(c / kPlanBK) * kPlanBN + r] += 1;
-                        if (c <= prev) myflags |= kPlanNonCanonical;
-                        prev = c;
-                    }
-                }
+        const int32_t c = c0[i], up = lane_below(c);
+        const bool live = lane < re[i] - rs[i];
+        if (__ballot(live && lane && c <= up)) slow |= 1u << i;
+        if (re[i] - rs[i] > 64) more |= 1u << i;
+        if (live && c >= 0 && c < a.K) atomicAdd(&cnt[(c / kPlanBK) * kPlanBN + wave * kPlanWRows + i], 1);
+    }
+    if (more) {
+#pragma unroll
+        for (int i = 0; i < kPlanWRows; i++) {
+            int32_t last = lane_i32(c0[i], 63);
+            bool bad = false;
+            for (int64_t jb = (int64_t)rs[i] + 64; jb < re[i]; jb += 64) {
+                const int32_t c = a.col[min(jb + lane, (int64_t)re[i] - 1)], up = lane_below(c);
+                const bool live = jb + lane < re[i];
+                if (live && c <= (lane ? up : last)) bad = true;
+                last = lane_i32(c, 63);
+                if (live && c >= 0 && c < a.K) atomicAdd(&cnt[(c / kPlanBK) * kPlanBN + wave * kPlanWRows + i], 1);
             }
-        } else {
+            if (__ballot(bad)) slow |= 1u << i;
+        }
+    }
+    if (slow) {
+        if (lane == 0) myflags |= kPlanUnsorted;
+        // columns in range that do not ascend strictly among themselves
+#pragma unroll
+        for (int i = 0; i < kPlanWRows; i++) {
+            if (!(slow & (1u << i))) continue;
+            int32_t prev = -1;  // the last one so far
             for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
                 const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
-                if (jb + lane < re[i] && c >= 0 && c < a.K) atomicAdd(&cnt[(c / kPlanBK) * kPlanBN + r], 1);
+                const bool ok = jb + lane < re[i] && c >= 0 && c < a.K;
+                const uint64_t in = __ballot(ok), below = in & ((1ull << lane) - 1);
+                const int32_t p = __shfl(c, below ? 63 - __builtin_clzll(below) : 0);
+                if (ok && c <= (below ? p : prev)) myflags |= kPlanNonCanonical;
+                if (in) prev = lane_i32(c, 63 - __builtin_clzll(in));
             }
         }
     }
@@ -274,36 +298,68 @@ __global__ void __launch_bounds__(kPlanNT) plan_build_kernel(ForwardArgs a, Plan
         int64_t o = kt < nksteps ? cnt[kt * kPlanBN] : total;
         off[kt] = (int32_t)(base + (fits ? o : 0));
     }
-    __syncthreads();  // the walk of the unsorted rows below advances the same counters
+    __syncthreads();  // the unsorted rows below advance the same counters
     if (fits) {
+        auto put = [&](int i, int32_t pos, int32_t c, uint32_t v) {
+            entries[base + pos] = ((uint32_t)(wave * kPlanWRows + i) << 24) | ((uint32_t)(c & (kPlanBK - 1)) << 16) | v;
+        };
+        // a batch at jb of a row that ascends: the step's first entry is at
+        // `first` where the step `last` goes on (both updated)
+        auto place = [&](int i, int64_t jb, int32_t c, uint32_t v, int64_t &first, int32_t &last) {
+            const bool ok = jb + lane < re[i] && c >= 0 && c < a.K;
+            const int32_t kt = c >> 6;  // (negative or past K: a step of its own, not written)
+            const int32_t up = lane_below(kt);
+            const uint64_t heads = __ballot(kt != (lane ? up : last));
+            const uint64_t below = heads & (~0ull >> (63 - lane));
+            const int64_t f = below ? jb + (63 - __builtin_clzll(below)) : first;
+            if (ok) put(i, cnt[kt * kPlanBN + wave * kPlanWRows + i] + (int32_t)(jb + lane - f), c, v);
+            first = lane_i32((int)(f - rs[i]), 63) + (int64_t)rs[i];
+            last = lane_i32(kt, 63);
+        };
+        int64_t first[kPlanWRows];
+        int32_t last[kPlanWRows];
 #pragma unroll
         for (int i = 0; i < kPlanWRows; i++) {
-            const int r = wave * kPlanWRows + i;
-            auto put = [&](int32_t pos, int32_t c, int64_t j) {
-                entries[base + pos] = ((uint32_t)r << 24) | ((uint32_t)(c & (kPlanBK - 1)) << 16) |
-                                      value_bits_f16(a.vals, a.val_dtype, j);
-            };
-            if (slow & (1u << i)) {
-                if (lane == 0)
-                    for (int32_t j = rs[i]; j < re[i]; j++) {
-                        const int32_t c = a.col[j];
-                        if (c >= 0 && c < a.K) put(cnt[(c / kPlanBK) * kPlanBN + r]++, c, j);
-                    }
-                continue;
+            first[i] = rs[i];
+            last[i] = INT32_MIN;
+            if (!(slow & (1u << i))) place(i, rs[i], c0[i], v0[i], first[i], last[i]);
+        }
+        if (more) {
+#pragma unroll
+            for (int i = 0; i < kPlanWRows; i++) {
+                if (slow & (1u << i)) continue;
+                for (int64_t jb = (int64_t)rs[i] + 64; jb < re[i]; jb += 64) {
+                    const int64_t j = min(jb + lane, (int64_t)re[i] - 1);
+                    place(i, jb, a.col[j], value_bits_f16(a.vals, a.val_dtype, j), first[i], last[i]);
+                }
             }
-            int64_t first = rs[i];       // the first entry of the last step so far
-            int32_t last = INT32_MIN;    // and that step
-            for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
-                const int32_t c = jb == rs[i] ? c0[i] : a.col[min(jb + lane, (int64_t)re[i] - 1)];
-                const bool ok = jb + lane < re[i] && c >= 0 && c < a.K;
-                const int32_t kt = c >> 6;  // (negative or past K: a step of its own, not written)
-                const int32_t up = __shfl_up(kt, 1);
-                const uint64_t heads = __ballot(kt != (lane ? up : last));
-                const uint64_t below = heads & (~0ull >> (63 - lane));
-                const int64_t f = below ? jb + (63 - __builtin_clzll(below)) : first;
-                if (ok) put(cnt[kt * kPlanBN + r] + (int32_t)(jb + lane - f), c, jb + lane);
-                first = __shfl((int)(f - rs[i]), 63) + (int64_t)rs[i];
-                last = __shfl(kt, 63);
+        }
+        if (slow) {
+            // an entry's place: its step's counter (this row's, so this
+            // wave's alone) plus the step's entries in the lanes below
+#pragma unroll
+            for (int i = 0; i < kPlanWRows; i++) {
+                if (!(slow & (1u << i))) continue;
+                for (int64_t jb = rs[i]; jb < re[i]; jb += 64) {
+                    const int64_t j = min(jb + lane, (int64_t)re[i] - 1);
+                    const int32_t c = jb == rs[i] ? c0[i] : a.col[j];
+                    const uint32_t v = jb == rs[i] ? v0[i] : value_bits_f16(a.vals, a.val_dtype, j);
+                    const bool ok = jb + lane < re[i] && c >= 0 && c < a.K;
+                    const int32_t kt = ok ? c / kPlanBK : -1;
+                    int32_t rank = 0, same = 0;
+                    const int live = (int)min((int64_t)64, re[i] - jb);
+                    for (int l = 0; l < live; l++) {
+                        const bool eq = lane_i32(kt, l) == kt;
+                        rank += eq && l < lane ? 1 : 0;
+                        same += eq ? 1 : 0;
+                    }
+                    int32_t *count = cnt + max(kt, 0) * kPlanBN + wave * kPlanWRows + i;
+                    const int32_t at = *count;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (every lane has read its counter)
+                    if (ok) put(i, at + rank, c, v);
+                    if (ok && rank == same - 1) *count = at + same;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
             }
         }
     }
@@ -317,8 +373,8 @@ __global__ void __launch_bounds__(kPlanNT) plan_build_kernel(ForwardArgs a, Plan
 // workgroup each: the group's entries are staged in LDS with coalesced loads;
 // where every row's columns ascend (not necessarily strictly), a chunk's or a
 // cell's entries of a row are a run found by binary search, and the records
-// are written word by word.  Otherwise each row's entries are walked in CSR
-// order by one thread per row and cell.  (A workgroup of 64 per cell, whose
+// are written word by word.  Otherwise each row's entries are taken in CSR
+// order by one wave.  (A workgroup of 64 per cell, whose
 // 16 row threads walked the CSR twice, took 28-35 us for each of the two
 // kinds of record of 4096 -> 11008 at 1 %.)
 constexpr int kPlanRowsNT = 256;
@@ -442,22 +498,62 @@ __global__ void __launch_bounds__(kPlanRowsNT) plan_rows_kernel(ForwardArgs a, P
         }
         return;
     }
-    // unsorted rows: the table as a walk meets the boundaries (read only where
-    // the rows ascend), and each cell's entries in CSR order
-    if (p.chunks && tid < 16 && g * 16 + tid < a.N) {
-        uint16_t *crow = p.chunks + (g * 16 + tid) * (int64_t)(nch + 1);
-        int cnext = 0;
-        for (int32_t j = rs[tid]; j < re[tid]; j++)
-            for (; cnext <= nch && (int64_t)cnext * 128 <= (int64_t)col(j); cnext++)
-                crow[cnext] = (uint16_t)min(j - rs[tid], 65535);
-        for (; cnext <= nch; cnext++) crow[cnext] = (uint16_t)min(re[tid] - rs[tid], 65535);
+    // unsorted rows, a wave four of them, 64 entries at a time.  The table as a
+    // walk meets the boundaries (read only where the rows ascend): the first
+    // entry at or past each, so an entry whose running maximum passes some
+    // records them.  A cell's entries in CSR order: a ballot per cell and batch
+    // counts them (lane ci holds cell ci's), and ranks them when they are
+    // written.  (A thread per row and cell walking the whole row: 11008 -> 4096
+    // at 5 %, descending, 3,402 us for the plan, now 435.)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint64_t under = (1ull << lane) - 1;
+    for (int i = 0; i < 4; i++) {
+        const int row = 4 * wave + i;
+        const int32_t s = lane_i32(rs[row], 0), e = lane_i32(re[row], 0);
+        uint16_t *crow = p.chunks && g * 16 + row < a.N ? p.chunks + (g * 16 + row) * (int64_t)(nch + 1) : nullptr;
+        int32_t n = 0, top = INT32_MIN;
+        for (int64_t jb = s; jb < e; jb += 64) {
+            const bool live = jb + lane < e;
+            const int32_t c = live ? col((int32_t)(jb + lane)) : INT32_MIN;
+            const bool ok = live && c >= 0 && c < a.K;
+            const int qi = ok ? c / p.qcols : -1, si = ok ? c >> 10 : -1;
+            for (int ci = 0; ci < ncq; ci++) {
+                const int m = __builtin_popcountll(__ballot(qi == ci));
+                n += lane == ci ? m : 0;
+            }
+            for (int ci = ncq; ci < ncells; ci++) {
+                const int m = __builtin_popcountll(__ballot(si == ci - ncq));
+                n += lane == ci ? m : 0;
+            }
+            if (crow) {
+                int32_t mx = max(c, top);
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                    const int32_t v = __shfl_up(mx, off);
+                    if (lane >= off) mx = max(mx, v);
+                }
+                // boundaries this batch passes, a lane each: the lanes whose
+                // maximum is below it come before
+                const int hi = min(nch, lane_i32(mx, 63) >> 7);
+                for (int cb0 = max(0, (top >> 7) + 1); cb0 <= hi; cb0 += 64) {
+                    const int cb = cb0 + lane;
+                    int first = 0;
+#pragma unroll
+                    for (int step = 32; step > 0; step >>= 1)
+                        if ((__shfl(mx, first + step - 1) >> 7) < cb) first += step;
+                    if (cb <= hi) crow[cb] = (uint16_t)min(jb + first - s, (int64_t)65535);
+                }
+                top = lane_i32(mx, 63);
+            }
+        }
+        if (crow)
+            for (int cb = max(0, (top >> 7) + 1) + lane; cb <= nch; cb += 64) crow[cb] = (uint16_t)min(e - s, 65535);
+        if (lane < kPlanMaxCells) tab[row][lane] = n;
     }
+    __syncthreads();
     {
         const int ci = r, row = l;
-        int32_t n = 0;
-        const int64_t c0 = cell_c0(ci), c1 = min(c0 + cell_cols(ci), a.K);
-        if (ci < ncells)
-            for (int32_t j = rs[row]; j < re[row]; j++) n += col(j) >= c0 && col(j) < c1 ? 1 : 0;
+        const int32_t n = tab[row][ci];
         int32_t incl = n;
 #pragma unroll
         for (int off = 1; off < 16; off <<= 1) {
@@ -466,24 +562,47 @@ __global__ void __launch_bounds__(kPlanRowsNT) plan_rows_kernel(ForwardArgs a, P
         }
         start[ci][row] = incl - n;
         if (row == 15) start[ci][16] = incl;
-        __syncthreads();
-        if (ci >= ncells) return;
-        const int cap = cell_words(ci) - kCellHdrWords;
+    }
+    __syncthreads();
+    for (int ci = 0; ci < ncells; ci++) {  // headers and empty slots
+        const int words = cell_words(ci), cap = words - kCellHdrWords, total = start[ci][16];
         uint32_t *rec = cell_rec(ci);
-        const int total = start[ci][16];
-        if (row == 0) {
-            rec[0] = cell_tag(ci);
-            rec[1] = (uint32_t)(total > cap ? total - cap : 0);
-            rec[18] = rec[19] = 0u;
+        for (int i = tid; i < words; i += kPlanRowsNT) {
+            if (i == 0) rec[i] = cell_tag(ci);
+            else if (i == 1) rec[i] = (uint32_t)(total > cap ? total - cap : 0);
+            else if (i < 18) rec[i] = (uint32_t)min(start[ci][i - 2], cap) | ((uint32_t)min(start[ci][i - 1], cap) << 16);
+            else if (i < kCellHdrWords) rec[i] = 0u;
+            else if (i - kCellHdrWords >= total) rec[i] = 0xffffu;
         }
-        rec[2 + row] = (uint32_t)min(incl - n, cap) | ((uint32_t)min(incl, cap) << 16);
-        int32_t w = incl - n;
-        for (int32_t j = rs[row]; j < re[row]; j++)
-            if (col(j) >= c0 && col(j) < c1) {
-                if (w < cap) rec[kCellHdrWords + w] = (uint32_t)(col(j) - (int32_t)c0) | (val(j) << 16);
-                w++;
+    }
+    for (int i = 0; i < 4; i++) {
+        const int row = 4 * wave + i;
+        const int32_t s = lane_i32(rs[row], 0), e = lane_i32(re[row], 0);
+        int32_t at = lane < ncells ? start[lane][row] : 0;
+        for (int64_t jb = s; jb < e; jb += 64) {
+            const bool live = jb + lane < e;
+            const int32_t j = (int32_t)min(jb + lane, (int64_t)e - 1), c = live ? col(j) : INT32_MIN;
+            const uint32_t v = val(j) << 16;
+            const bool ok = live && c >= 0 && c < a.K;
+            const int qi = ok ? c / p.qcols : -1, si = ok ? c >> 10 : -1;
+            int qw = 0, sw = 0;  // the entry's slots
+            for (int ci = 0; ci < ncq; ci++) {
+                const uint64_t m = __ballot(qi == ci);
+                const int w = lane_i32(at, ci) + __builtin_popcountll(m & under);
+                qw = qi == ci ? w : qw;
+                at += lane == ci ? __builtin_popcountll(m) : 0;
             }
-        for (int i = total + row; i < cap; i += 16) rec[kCellHdrWords + i] = 0xffffu;
+            for (int ci = ncq; ci < ncells; ci++) {
+                const uint64_t m = __ballot(si == ci - ncq);
+                const int w = lane_i32(at, ci) + __builtin_popcountll(m & under);
+                sw = si == ci - ncq ? w : sw;
+                at += lane == ci ? __builtin_popcountll(m) : 0;
+            }
+            if (ok && ncq && qw < p.qwords - kCellHdrWords)
+                p.qrec[(g * 4 + qi) * (int64_t)p.qwords + kCellHdrWords + qw] = (uint32_t)(c - qi * p.qcols) | v;
+            if (ok && p.srec && sw < p.swords - kCellHdrWords)
+                p.srec[(g * p.nslices + si) * (int64_t)p.swords + kCellHdrWords + sw] = (uint32_t)(c & 1023) | v;
+        }
     }
 }
 

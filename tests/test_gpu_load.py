@@ -1,5 +1,6 @@
 """The load path's kernels byte by byte: the ortho plan against a plain numpy
-form of its layout (orth_prefill.hip)."""
+form of its layout (orth_prefill.hip), the CSR against torch's nonzero and the
+INT4 nibbles against the divisions they round (orth_pack.hip)."""
 import ctypes
 import math
 
@@ -140,3 +141,51 @@ def test_plan_bytes(gpu, K, N, density, heavy, order):
         elif order == "some" and n % 7 == 3 and c.size:
             c[-1], c[0] = K + 3, -2
     check(K, N, row_ptr, col, vals if N % 2 else vals.astype(np.float32))
+
+
+# rows of one and of several 4096-column chunks; sparse and dense chunks, both
+# in one row, a lane's 64 columns full; more rows than one pass of the scan
+@pytest.mark.parametrize("K,N,density,block", [
+    (4096, 70, 0.01, None), (4096, 70, 0.1, None), (8320, 33, 0.5, None), (12288, 20, 0.003, (4100, 4164)),
+    (12288, 20, 0.003, (4096, 8192)), (64, 20000, 0.02, None), (128, 8193, 0.3, None), (4100, 30, 0.03, (0, 90))])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_pack_csr_entries(gpu, K, N, density, block, dtype):
+    from libortho_amd import _C_ops
+    g = torch.Generator().manual_seed(K + N)
+    mask = torch.rand(N, K, generator=g) < density
+    if block:
+        mask[::2, block[0]:block[1]] = True
+    w = torch.where(mask, torch.randn(N, K, generator=g).to(dtype), torch.zeros((), dtype=dtype))
+    row_ptr, col, vals = (t.cpu() for t in _C_ops.pack_csr(w.cuda()))
+    at = torch.nonzero(w)
+    assert torch.equal(row_ptr[1:].long(), torch.bincount(at[:, 0], minlength=N).cumsum(0)) and row_ptr[0] == 0
+    assert torch.equal(col.long(), at[:, 1]) and torch.equal(vals, w[at[:, 0], at[:, 1]])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("group", [None, 128])
+def test_pack_nibbles_at_the_halves(gpu, dtype, group):
+    """Weights at and beside half steps of their scale, where the quotient's
+    last bit decides; scales from the clamp to near the top of the range."""
+    from libortho_amd import _C_ops
+    K, N = 1024, 600
+    g = torch.Generator().manual_seed(3)
+    top = {torch.float16: 12.0, torch.bfloat16: 120.0, torch.float32: 120.0}[dtype]
+    mx = torch.exp2(torch.rand(N, 1, generator=g) * (top + 18) - 18) * (1 + torch.rand(N, 1, generator=g))
+    mx[:7] = torch.tensor([1e-9, 6.9e-6, 7e-6, 7.1e-6, 1.0, 7.0, 14.0])[:, None]
+    mx = mx.to(dtype)
+    s = (mx.float() * torch.tensor(1.0) / 7).to(dtype)
+    w = (s.float() * (torch.randint(-14, 15, (N, K), generator=g) / 2)).to(dtype)
+    step = torch.randint(-2, 3, (N, K), generator=g)
+    bits = w.view(torch.int32 if dtype == torch.float32 else torch.int16)
+    w = torch.where(w != 0, (bits + step.to(bits.dtype)).view(dtype), w)
+    w[:, ::128] = mx
+    wd = w.cuda()
+    cells = wd.float().view(N, -1, group or K)
+    amax = cells.abs().amax(-1, keepdim=True)
+    scale = torch.clamp((amax * torch.tensor(1.0 / 7, device="cuda")).to(dtype), min=1e-6)
+    want = torch.clamp(torch.round((cells / scale.float()).to(dtype).float()), -8, 7).view(N, K).to(torch.int8)
+    q, scales = _C_ops.pack_base(wd, group)
+    got = torch.stack((q & 15, q >> 4), -1).reshape(N, K).to(torch.int8)
+    assert torch.equal((got ^ 8) - 8, want)
+    assert torch.equal(scales.view(N, -1), scale.view(N, -1).half())

@@ -442,6 +442,7 @@ int forward_impl(const orth_hip_layer_t *layer, const void *plan, int64_t plan_b
         return fail(ORTH_ERR_INVALID_ARGUMENT, "bias dtype %d is not F16, BF16 or F32", bias_dtype);
     a.bias = bias;
     a.bias_dtype = bias_dtype;
+    a.planned = plan != nullptr;
     if (plan && plan_bytes < plan_bytes_for(a.N, a.K, a.nnz))
         return fail(ORTH_ERR_INVALID_ARGUMENT, "plan_bytes %lld is smaller than the plan size %lld",
                     (long long)plan_bytes, (long long)plan_bytes_for(a.N, a.K, a.nnz));
@@ -615,6 +616,7 @@ int group_forward_impl(const orth_hip_layer_t *const *layers, const void *const 
         as[l].bias = bias;
         as[l].bias_dtype = bdt;
         pl[l] = plans ? plans[l] : nullptr;
+        as[l].planned = pl[l] != nullptr;
         if (pl[l] && (!plan_bytes || plan_bytes[l] < plan_bytes_for(as[l].N, as[l].K, as[l].nnz)))
             return fail(ORTH_ERR_INVALID_ARGUMENT, "plan %d is smaller than the plan size %lld", l,
                         (long long)plan_bytes_for(as[l].N, as[l].K, as[l].nnz));

@@ -59,6 +59,7 @@ struct ForwardArgs {
     int bias_dtype = 0;
     int cus = 256;           // compute units of the device
     int variant = 0;         // of KERNEL_GENERAL: a GeneralVariant
+    int planned = 0;         // the call has an ortho plan
 };
 
 // ------------------------------------------------------ the sieve's select

@@ -8,7 +8,7 @@ torch = pytest.importorskip("torch")
 
 from libortho_amd import _C_ops  # noqa: E402
 from libortho_amd import workloads as W  # noqa: E402
-from tests.test_gpu_float import bound, dense64  # noqa: E402
+from tests.test_gpu_float import bound, dense64, rms_error  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -57,6 +57,8 @@ def test_rows_parity(gpu, oracle_mod, K, N, group, M, density, dtype):
         ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, alpha)
         sums = bound(lay, x, alpha)
         assert within(y, ref, sums, dtype)
+        if dtype == F32:
+            assert rms_error(y, ref) <= 5e-7
 
 
 # either side of the choice's lines, in calls whose times are well apart:

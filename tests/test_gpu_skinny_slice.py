@@ -38,9 +38,25 @@ def check(oracle_mod, lay, x, alpha, dtype, y):
     assert (err <= sums + np.maximum(EPS[dtype] * (np.abs(ref) + sums), TINY[dtype])).all()
 
 
+def check_ortho(oracle_mod, lay, x, alpha, dtype, **kw):
+    """With scales of zero the output is the ortho term alone (the dense sums
+    are multiplied by 0), its bound that of its own few sums: one entry of a
+    row left out or taken twice is far outside it."""
+    scales = lay.scales.copy()
+    lay.scales[:] = 0
+    y, _ = run(lay, x, alpha, dtype, **kw)
+    ref = oracle_mod.forward_f64(lay.q, lay.scales, lay.row_ptr, lay.col, lay.vals, x, alpha)
+    sums = bound(lay, x, alpha)
+    one = alpha * np.sqrt(np.mean(lay.vals.astype(np.float64) ** 2) * np.mean(x.astype(np.float64) ** 2))
+    assert np.median(sums + EPS[dtype] * np.abs(ref)) < 0.2 * one  # (what one entry adds, rms)
+    err = np.abs(y.float().cpu().numpy() - ref)
+    assert (err <= sums + np.maximum(EPS[dtype] * (np.abs(ref) + sums), TINY[dtype])).all()
+    lay.scales[:] = scales
+
+
 # two, three and four token tiles, the last 8 (4, 2) tokens ragged, rows that
 # end inside a unit, rows with more entries than one batch of loads, tiles of 8
-# tokens (K <= 8250), 4 and 2, one scale per row
+# tokens (K <= 8192), 4 and 2, one scale per row
 @pytest.mark.parametrize("K,N,group,M,density,dtype", [
     (4096, 1000, 128, 17, 0.01, torch.float16), (4096, 3001, 128, 33, 0.02, torch.bfloat16),
     (2048, 2000, None, 48, 0.05, torch.float16), (4096, 1040, 256, 64, 0.005, torch.float16),
@@ -53,7 +69,27 @@ def test_skinny_slice_parity(gpu, oracle_mod, K, N, group, M, density, dtype):
     assert k == "skinny"
     check(oracle_mod, lay, x, 0.5, dtype, y)
     z, _ = run(lay, x, 0.5, dtype, plan=K <= 12288)
-    assert torch.equal(y, z)  # (it reads no plan)
+    if K == 11008:  # (with a plan each lane finds its own entries)
+        check(oracle_mod, lay, x, 0.5, dtype, z)
+        check_ortho(oracle_mod, lay, x, 0.5, dtype, plan=True)
+    else:
+        assert torch.equal(y, z)  # (it reads no plan)
+    check_ortho(oracle_mod, lay, x, 0.5, dtype)
+
+
+@pytest.mark.parametrize("K,N,M,density,dtype", [
+    (4096, 1000, 33, 0.2, torch.float16), (4096, 2100, 64, 0.1, torch.bfloat16), (1152, 9000, 49, 0.2, torch.float16)])
+def test_many_planned_entries(gpu, oracle_mod, K, N, M, density, dtype):
+    """17 .. 64 tokens with a plan and so many entries that each lane finds its
+    own: the same results as from the workgroups that take them without one,
+    to the rounding of sums in another order."""
+    lay = W.make_layer(K, N, 128, density, 9300 + K)
+    x = torch.from_numpy(W.make_x(M, K, 9301 + M)).to(dtype).float().numpy()
+    for plan in (True, False):
+        y, k = run(lay, x, 1.0, dtype, plan=plan)
+        assert k == "skinny"
+        check(oracle_mod, lay, x, 1.0, dtype, y)
+        check_ortho(oracle_mod, lay, x, 1.0, dtype, plan=plan)
 
 
 def test_skinny_slice_odd_csr_infinities_and_bias(gpu, oracle_mod):
@@ -91,6 +127,7 @@ def test_one_token_tile_transposed_copy(gpu, oracle_mod, K, N, M, density, dtype
     y, k = run(lay, x, 1.0, dtype, plan=plan)
     assert k == "skinny"
     check(oracle_mod, lay, x, 1.0, dtype, y)
+    check_ortho(oracle_mod, lay, x, 1.0, dtype, plan=plan)
     bad = x.copy()
     bad[1, 0], bad[M - 1, K - 1] = np.inf, np.nan
     z, _ = run(lay, bad, 1.0, dtype, plan=plan)
@@ -101,6 +138,7 @@ def test_one_token_tile_transposed_copy(gpu, oracle_mod, K, N, M, density, dtype
 @pytest.mark.parametrize("K,N,M,density,alpha,kernel", [
     (8192, 1024, 33, 0.01, 1.0, "skinny"), (8320, 1024, 33, 0.01, 1.0, "prefill"),
     (8192, 2048, 64, 0.03, 1.0, "prefill"),          # entries x tokens past 27 million
+    (5120, 512, 33, 0.03, 1.0, "skinny"), (5120, 512, 33, 0.04, 1.0, "prefill"),  # 1 entry in 32
     (11008, 1024, 64, 0.01, 0.0, "skinny"), (11008, 1024, 64, 0.01, 1.0, "prefill")])
 def test_wide_k_dispatch(gpu, oracle_mod, K, N, M, density, alpha, kernel):
     lay = W.make_layer(K, N, 128, density, 9100 + K)

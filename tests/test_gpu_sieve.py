@@ -152,6 +152,22 @@ def test_split_in_place(gpu, dt, N, K, in_place, rank):
         assert bits_equal(got[name], want[name]), name
 
 
+@pytest.mark.parametrize("dt,N,K", [("f32", 40, 260), ("f16", 30, 1027), ("bf16", 1030, 520), ("f16", 9, 16388)])
+def test_threshold_with_a_matrix_diagonal(gpu, dt, N, K):
+    """A threshold with h a matrix's diagonal (the residual is kept from the first
+    pass): the bits of the same h as a vector."""
+    from libortho_amd.tools.sieve import hessian_sieve
+    w = make_w(dt, N, K, seed=11, device=gpu)
+    h = (torch.rand(K, generator=torch.Generator().manual_seed(12)) + 0.1).to(gpu)
+    a = hessian_sieve(w, h, curvature_thresh=1e-3)
+    # (overlapping rows: every third element is the diagonal, no K x K memory)
+    H = torch.empty(K * 3, device=gpu).as_strided((K, K), (2, 1))
+    torch.diagonal(H).copy_(h)
+    b = hessian_sieve(w, H, curvature_thresh=1e-3)
+    assert a[1].count_nonzero() > 0
+    assert bits_equal(a[0], b[0]) and bits_equal(a[1], b[1])
+
+
 def test_hessian_sieve_matrix_h_and_ties(gpu):
     """H_inv given as a matrix (its diagonal is used) and a score with many
     exact ties at the threshold (the k-th largest value is the same whatever

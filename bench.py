@@ -965,7 +965,7 @@ def main():
                           "us_per_step": round(rr["ms_per_step"] * 1e3, 2), "TFLOP/s": round(tf, 1),
                           "frac_bf16_peak": round(tf / FP16_PEAK_TFLOPS, 4)})
         log(f"  {secondary[-1]}")
-        # the general kernel (one wave per output): FP32 activations and
+        # the kernels reported as general: FP32 activations and
         # output (4 bytes each in the traffic), and an FP16 layer whose K is
         # not a multiple of 128 (per-row scales), which no fast kernel takes
         odd = W.make_layer(4000, 11008, None, 0.01, 4000)

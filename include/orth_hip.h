@@ -107,15 +107,16 @@ int orth_layer_check_hip(const orth_hip_layer_t *layer, const void *input, void 
  * term), the slice-split kernel (17..32 at the other K % 128 == 0, a plan
  * or no ortho term), the split-K mid-batch kernel (other batches up to 64;
  * 33..64 at K > 4096 with a plan or no ortho term: the prefill kernel with
- * K split over the grid where it is the faster one),
+ * K split over the grid where it is the faster one, with more than 1 entry
+ * in 32, many entries times tokens or K > 8192),
  * the MFMA prefill kernels above (256 x 128 tiles with K split over the
  * grid and a reduction launch where the tiles alone leave CUs idle and a
  * plan or no ortho term is given; else the wide kernel where its 256 x 352
  * tile per workgroup needs fewer rounds of the grid than 256 x 128 tiles,
  * as at 4096 -> 11008 with 2048 tokens, or from 1024 tokens with 256 x
- * 128 tiles in 64-column steps; else 256 x 128 tiles), and a general kernel for shapes and
+ * 128 tiles in 64-column steps; else 256 x 128 tiles), and the general kernels for shapes and
  * dtypes the fast kernels do not take (orth_hip_last_kernel() names the
- * choice).  BF16 I/O
+ * choice, orth_hip_last_variant() which of the three general ones).  BF16 I/O
  * takes the decode kernel for 1..4 tokens and the one-launch mid-batch
  * kernel for 5..16 (both K = 4096 with a plan or no ortho term), the
  * slice-split kernel for 17..32 (K % 128 == 0, a plan or no ortho term),

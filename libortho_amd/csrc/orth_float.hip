@@ -1,4 +1,4 @@
-// FP32 activations, batches from a few dozen tokens: the dual GEMM on the
+// FP32 activations, batches from a few dozen tokens (general_variant): the dual GEMM on the
 // matrix cores without giving up an FP32 bit of the activations.
 //
 // Same formula as /root/reference/src/dual_gemm.cu:176-225, whose
@@ -21,7 +21,7 @@
 //    beside 24 MFMAs): the two K halves, which share each SIMD, therefore
 //    take the MFMAs and the staging in opposite order (77 -> 74 us at 512
 //    tokens of 4096 -> 4096, alpha = 0, with the byte conversions written
-//    out; 1,203 us on the general kernel).
+//    out; 1,203 us on the wave-per-row kernel).
 //  * float_ortho_kernel, the sparse term (alpha > 0): y += alpha * sum v x.
 //    A workgroup keeps all columns of up to 8 tokens in LDS, [column][token],
 //    so that an entry costs one 16-byte LDS read per 4 tokens, and walks the
@@ -475,9 +475,9 @@ hipError_t launch_float(const ForwardArgs &a, int cus, hipStream_t stream) {
     d.bias_dtype = a.bias_dtype;
     // The partials are summed into the scaled sums every two steps, also
     // inside a longer group: one chain over all of K would lose more than the
-    // general kernel's lanes do (4096 columns, one scale per row: relative
-    // error against FP64 4.2e-7; flushed every two steps 1.3e-7, the general
-    // kernel 1.6e-7).
+    // wave-per-row kernel's lanes do (4096 columns, one scale per row: relative
+    // error against FP64 4.2e-7; flushed every two steps 1.3e-7, those
+    // lanes 1.6e-7).
     hipError_t e = d.spg % 2 ? launch_float_dense<1>(d, a.N, stream) : launch_float_dense<2>(d, a.N, stream);
     if (e != hipSuccess || !a.has_ortho) return e;
     FloatOrthoArgs o;

@@ -3,7 +3,7 @@
 // scale groups of 32, 64, 96, ... columns.
 //
 // Same formula as /root/reference/src/dual_gemm.cu:176-225.  A wave of the
-// general kernel owns one output row and reads every activation for it (4
+// wave-per-row kernel owns one output row and reads every activation for it (4
 // tokens of 4096 FP32 columns: 64 KB a row, 268 MB over a 4096-row layer); here
 // a workgroup stages the activations of up to 16 tokens in LDS once and takes
 // RB blocks of 16 rows per pass, and the products run on the matrix cores:
@@ -24,13 +24,14 @@
 //    activation in a staged row (empty slots: a zero past its end), and handed
 //    to the lanes (entry, token) in turn, which gather there.  This follows
 //    the dense term, whose weights were asked for first: 4000 -> 11008, 16
-//    FP16 tokens at 1 %, 21.7 -> 18.9 us against taking it first with a test
+//    FP16 tokens at 1 %, weights in cache, 21.7 -> 18.9 us against taking it first with a test
 //    per entry; the dense term alone 12.2.
 //  * The waves' partials meet in LDS (deterministic) and are rounded once.
 //
 // What bounds it: the latency chain (staging, the weights' first bytes, the
 // reduction) at few tokens, the LDS reads of the sparse term at 16 (4000 ->
-// 11008, 16 FP16 tokens at 1 %: 139 us on the general kernel, 18.9 here).
+// 11008, 16 FP16 tokens at 1 %, weights from HBM: 149.8 us on the wave-per-row
+// kernel, 21.8 here; 1 token 26.3 and 18.4).
 #include <algorithm>
 #include <atomic>
 

@@ -36,8 +36,9 @@
 //    per entry and token, cost as much as the dense term: 4096 -> 11008 at 48
 //    tokens, 1 %, 36.6 us against 18.6 at alpha = 0; now 26.8.)  It needs no
 //    plan.
-//    Without a K split (or where the extra partial would not fit the
-//    no-allocation scratch array) each lane still reads its own entries.
+//    Each lane still reads its own entries without a K split, where the extra
+//    partial would not fit the no-allocation scratch array, and where the plan
+//    locates many entries in rows of like length (skinny_shape).
 //  * With the plan's slice records (one token tile, 8-chunk slices,
 //    K % 1024 == 0) each wave instead loads its 16 rows' record of the slice
 //    at entry (packed column | value words at an address that needs no other

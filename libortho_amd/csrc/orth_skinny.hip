@@ -38,7 +38,12 @@
 //    plan.
 //    Each lane still reads its own entries without a K split, where the extra
 //    partial would not fit the no-allocation scratch array, and where the plan
-//    locates many entries in rows of like length (skinny_shape).
+//    locates many entries in rows of like length (skinny_shape).  Whether it
+//    does (columns that ascend) is in the plan's header, on the device: the
+//    workgroups are launched behind the dense ones all the same and end at
+//    once, or take the entries of a plan that does not (4096 -> 1024 at 24
+//    tokens, 20 %, columns descending: 261 us with own entries in whole rows,
+//    now 55).
 //  * With the plan's slice records (one token tile, 8-chunk slices,
 //    K % 1024 == 0) each wave instead loads its 16 rows' record of the slice
 //    at entry (packed column | value words at an address that needs no other
@@ -101,10 +106,20 @@ struct SkinnyArgs {
     int lds_sr;          // SPK >= 3: per-wave record regions
     const void *bias;  // [N] added after rounding (out_f16), or null
     int bias_dtype;
-    // SPK 7: the ortho term's workgroups (a multiple of 8, ids first), the
-    // tokens each keeps (8, 4 or 2) and the number of token tiles
-    int sp_wgs, sp_tt, sp_tiles;
+    // SPK 7, 8: the ortho term's workgroups (a multiple of 8; 7: ids first, 8:
+    // from id sp_first), the tokens each keeps (8, 4 or 2) and the number of
+    // token tiles
+    int sp_wgs, sp_tt, sp_tiles, sp_first;
 };
+
+// Whether a plan header (word(l): its 32-bit word l) is this layer's and its
+// chunk table locates the rows' ranges.
+template <typename Word>
+__device__ __forceinline__ bool skinny_plan_ok(Word word, int64_t N, int64_t K, int64_t nnz) {
+    auto dword = [&](int l) -> int64_t { return (int64_t)(word(l) | ((uint64_t)word(l + 1) << 32)); };
+    return (word(0) == kSkPlanMagic) & (word(1) == kSkPlanVersion) & (dword(6) == N) & (dword(8) == K) &
+           (dword(10) == nnz) & ((word(12) & kSkPlanUnsorted) == 0);
+}
 
 // ---- the ortho term of 17 .. 64 tokens as a slice of its own
 
@@ -113,17 +128,18 @@ struct SkinnyArgs {
 template <int TT>
 __device__ __forceinline__ int ss_col(int c) { return c * (2 * TT) + (c >> 3) * 16; }
 
+// id: of the a.sp_wgs workgroups.
 template <int TT, bool XB>
-__device__ void skinny_sparse(const SkinnyArgs &a, unsigned char *smem) {
+__device__ void skinny_sparse(const SkinnyArgs &a, unsigned id, unsigned char *smem) {
     constexpr int U = 3;                               // batches of 16 entries of a row in flight
     constexpr int PL = (TT * kSsRows + 63) / 64;       // outputs per lane of a unit
     constexpr int W = TT / 2;                          // words of a column's tokens
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = a.K;
-    const int m0 = (int)(blockIdx.x % (unsigned)a.sp_tiles) * TT;
-    const int wg = (int)(blockIdx.x / (unsigned)a.sp_tiles);
-    const int wgs = (a.sp_wgs + a.sp_tiles - 1 - (int)(blockIdx.x % (unsigned)a.sp_tiles)) / a.sp_tiles;  // of this tile
+    const int m0 = (int)(id % (unsigned)a.sp_tiles) * TT;
+    const int wg = (int)(id / (unsigned)a.sp_tiles);
+    const int wgs = (a.sp_wgs + a.sp_tiles - 1 - (int)(id % (unsigned)a.sp_tiles)) / a.sp_tiles;  // of this tile
     float *sums = reinterpret_cast<float *>(smem + ss_col<TT>(K) + 16) + wave * TT * kSsRows;  // [TT][16]
     if (tid == 0) *reinterpret_cast<u32x4 *>(smem + ss_col<TT>(K)) = u32x4{0u, 0u, 0u, 0u};  // a zero column
 
@@ -273,14 +289,15 @@ __device__ void skinny_sparse(const SkinnyArgs &a, unsigned char *smem) {
 // column in the transposed copy, not 16); 3 .. 6 (one tile, GMODE 3) the
 // same from the plan's slice records instead of the CSR: 3 / 4 records of
 // 256 words (4: at most 8 tokens), 5 / 6 of 512 words; 7 (two and more tiles)
-// the ortho term in workgroups and a partial of its own.
+// the ortho term in workgroups and a partial of its own; 8 the same where the
+// plan does not locate the entries, else as 1.
 // (4 waves per SIMD up to two token tiles; BF16 with two tiles needs the
 // registers of 2: at 4 one instantiation spilled 8 bytes)
 template <int NTT, int GMODE, int CPS, int SPK, bool XB>
 __global__ void __launch_bounds__(kSkNT) __attribute__((amdgpu_waves_per_eu(NTT == 1 || (NTT == 2 && !XB) ? 4 : 2)))
 skinny_kernel(SkinnyArgs a) {
     constexpr bool SPARSE = SPK != 0 && SPK != 7;
-    constexpr bool SREC = SPK >= 3 && SPK != 7;                  // slice records: each wave reads its 16 rows' record
+    constexpr bool SREC = SPK >= 3 && SPK < 7;                   // slice records: each wave reads its 16 rows' record
     constexpr bool HALF = SPK == 2 || SPK == 4 || SPK == 6;
     constexpr int RQ = SPK == 5 || SPK == 6 ? 2 : 1;             // record loads per lane (256 words each per wave)
     constexpr int MP = NTT * 16;                     // padded tokens
@@ -330,14 +347,16 @@ skinny_kernel(SkinnyArgs a) {
     // so a block's partials are written and read through one L2.  The grid
     // is padded to 8 * ceil(nblocks / 8) * S.
     int bid = (int)blockIdx.x;
-    if constexpr (SPK == 7) {
-        if (bid < a.sp_wgs) {  // (uniform)
-            if (a.sp_tt == 8) skinny_sparse<8, XB>(a, smem);
-            else if (a.sp_tt == 4) skinny_sparse<4, XB>(a, smem);
-            else skinny_sparse<2, XB>(a, smem);
+    if constexpr (SPK >= 7) {
+        if (SPK == 7 ? bid < a.sp_wgs : bid >= a.sp_first) {  // (uniform)
+            const unsigned id = (unsigned)(SPK == 7 ? bid : bid - a.sp_first);
+            if (SPK == 8 && skinny_plan_ok([&](int l) { return a.phdr[l]; }, a.N, a.K, a.nnz)) return;
+            if (a.sp_tt == 8) skinny_sparse<8, XB>(a, id, smem);
+            else if (a.sp_tt == 4) skinny_sparse<4, XB>(a, id, smem);
+            else skinny_sparse<2, XB>(a, id, smem);
             return;
         }
-        bid -= a.sp_wgs;
+        if (SPK == 7) bid -= a.sp_wgs;
     }
     const int q = bid >> 3;
     const int blk = (bid & 7) + 8 * (q / a.S), slice = q - (q / a.S) * a.S;
@@ -486,16 +505,18 @@ skinny_kernel(SkinnyArgs a) {
             v[u] = __builtin_bit_cast(uint16_t, a.vals[j]);
         }
     };
+    float alpha = a.alpha;
     if (SPARSE && !SREC) {
         auto word = [&](int l) -> uint32_t { return (uint32_t)__builtin_amdgcn_readlane(hw, l); };
-        auto dword = [&](int l) -> int64_t { return (int64_t)(word(l) | ((uint64_t)word(l + 1) << 32)); };
-        const bool fast = (a.phdr != nullptr) & (a.chunks != nullptr) & (word(0) == kSkPlanMagic) &
-                          (word(1) == kSkPlanVersion) & (dword(6) == a.N) & (dword(8) == (int64_t)K) &
-                          (dword(10) == (int64_t)a.nnz) & ((word(12) & kSkPlanUnsorted) == 0);
+        const bool fast = (a.phdr != nullptr) & (a.chunks != nullptr) & skinny_plan_ok(word, a.N, K, a.nnz);
         const int32_t rs = min(max(rp0, 0), a.nnz), re = min(max(rp1, rs), a.nnz);
         lo = fast ? rs + min((int32_t)ck0, re - rs) : rs;
         hi = fast ? rs + min(max((int32_t)ck1, (int32_t)ck0), re - rs) : re;
         if (n0 + sr >= a.N) hi = lo;  // rows past N
+        if (SPK == 8 && !fast) {  // the other workgroups' entries: nothing here
+            hi = lo;
+            alpha = 0.f;
+        }
         load_batch(lo, ecol, eval);
         load_batch(lo + EB, ecol2, eval2);
     }
@@ -726,7 +747,7 @@ skinny_kernel(SkinnyArgs a) {
         for (int i = 0; i < 4; i++) {
             float v = acc[tt][i];
             if (!GROUPED) v = (v - bias_acc[tt][i]) * srow;
-            if (SPARSE) v += a.alpha * (QUAD ? sp[(wave * 16 + nl) * MP + tt * 16 + 4 * g + i] : sacc[tt * 4 + i]);
+            if (SPARSE) v += alpha * (QUAD ? sp[(wave * 16 + nl) * MP + tt * 16 + 4 * g + i] : sacc[tt * 4 + i]);
             val[tt][i] = v;
         }
     }
@@ -765,7 +786,8 @@ skinny_kernel(SkinnyArgs a) {
 // block blk runs on XCD blk % 8 like the slices that wrote its partials.
 // The loads of all S slices (up to 16 per round) are issued before the
 // first add (addresses clamped to the last slice, the extra ones not
-// added); sums in slice order.
+// added); sums in slice order.  phdr: the last partial holds values only if
+// that plan does not locate the entries (SPK 8); null: it does.
 constexpr int kSkRedU = 16;
 
 static int skinny_reduce_parts(int M, int vec4) {
@@ -775,12 +797,14 @@ static int skinny_reduce_parts(int M, int vec4) {
 
 __global__ void __launch_bounds__(256) skinny_reduce_kernel(const float *part, f16 *y, int M, int64_t N, int S,
                                                             int vec4, int nblocks, int R, const void *bias,
-                                                            int bias_dtype, int xb) {
+                                                            int bias_dtype, int xb, const uint32_t *phdr, int64_t K,
+                                                            int64_t nnz) {
     constexpr int U = kSkRedU;
     const int q = (int)(blockIdx.x >> 3);
     const int blk = (int)(blockIdx.x & 7) + 8 * (q / R);
     const int r = q - (q / R) * R;
     if (blk >= nblocks) return;
+    const int added = S - (phdr && skinny_plan_ok([&](int l) { return phdr[l]; }, N, K, nnz) ? 1 : 0);
     const int64_t n0 = (int64_t)blk * kSkRows;
     const int64_t MN = (int64_t)M * N;
     const int idx = r * 256 + (int)threadIdx.x;
@@ -799,7 +823,7 @@ __global__ void __launch_bounds__(256) skinny_reduce_kernel(const float *part, f
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (s0 + u == 0) v = w[u];
-                else if (s0 + u < S) v += w[u];
+                else if (s0 + u < added) v += w[u];
             }
         }
         uint32_t h[4];
@@ -822,7 +846,7 @@ __global__ void __launch_bounds__(256) skinny_reduce_kernel(const float *part, f
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 if (s0 + u == 0) v = w[u];
-                else if (s0 + u < S) v += w[u];
+                else if (s0 + u < added) v += w[u];
             }
         }
         if (xb) reinterpret_cast<uint16_t *>(y)[o] = out_bf16(v, bias, bias_dtype, n);
@@ -880,7 +904,9 @@ static hipError_t skinny_launch_g(const SkinnyArgs &d, bool sparse, int blocks, 
             }
         }
         if constexpr (NTT > 1)
-            if (d.sp_wgs > 0) return skinny_launch_t<NTT, GMODE, C, 7, XB>(d, blocks, lds, s);
+            if (d.sp_wgs > 0)
+                return d.sp_first ? skinny_launch_t<NTT, GMODE, C, 8, XB>(d, blocks, lds, s)
+                                  : skinny_launch_t<NTT, GMODE, C, 7, XB>(d, blocks, lds, s);
         if (NTT == 1 && d.M <= 8) return skinny_launch_t<NTT, GMODE, C, (NTT == 1 ? 2 : 1), XB>(d, blocks, lds, s);
         return skinny_launch_t<NTT, GMODE, C, 1, XB>(d, blocks, lds, s);
     }
@@ -981,7 +1007,9 @@ hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float 
     d.sp_wgs = sh.sp_wgs;
     d.sp_tt = sh.sp_tt;
     d.sp_tiles = sh.sp_tiles;
-    const int blocks = sh.sp_wgs + ((sh.nblocks + 7) / 8) * 8 * sh.S;  // padded: see skinny_kernel
+    const int dense = ((sh.nblocks + 7) / 8) * 8 * sh.S;  // padded: see skinny_kernel
+    const int blocks = sh.sp_wgs + dense;
+    d.sp_first = sh.sp_own && d.phdr && d.chunks ? dense : 0;
     const bool xb = a.io_dtype == ORTH_DT_BF16;
     const hipError_t e = xb ? skinny_launch_x<true>(d, sh.ntt, gmode, sparse, blocks, lds, stream)
                             : skinny_launch_x<false>(d, sh.ntt, gmode, sparse, blocks, lds, stream);
@@ -990,7 +1018,8 @@ hipError_t launch_skinny(const ForwardArgs &a, const void *plan, int cus, float 
     const int R = skinny_reduce_parts((int)a.M, vec4);
     const unsigned rblocks = (unsigned)(((sh.nblocks + 7) / 8) * 8 * R);
     hipLaunchKernelGGL(skinny_reduce_kernel, dim3(rblocks), dim3(256), 0, stream, part, static_cast<f16 *>(a.y),
-                       (int)a.M, a.N, sh.S + (sh.sp_wgs > 0 ? 1 : 0), vec4, sh.nblocks, R, a.bias, a.bias_dtype, xb ? 1 : 0);
+                       (int)a.M, a.N, sh.S + (sh.sp_wgs > 0 ? 1 : 0), vec4, sh.nblocks, R, a.bias, a.bias_dtype, xb ? 1 : 0,
+                       d.sp_first ? d.phdr : nullptr, a.K, a.nnz);
     return hipGetLastError();
 }
 

@@ -18,6 +18,7 @@ constexpr int sk_cps_bound(int ntt) { return ntt * kSkMaxCPS > 16 ? ((16 / ntt) 
 
 constexpr int kSsRows = 16;                // rows per unit (one wave's)
 constexpr int kSsLdsMax = 150 * 1024;
+constexpr int kSsLdsCu = 160 * 1024;       // of a compute unit
 
 inline int ss_lds(int64_t K, int tt) {
     return (int)(K * 2 * tt + K / 8 * 16 + 16 + (kSkNT / 64) * kSsRows * tt * 4);
@@ -37,6 +38,7 @@ struct SkinnyShape {
     int ntt, cps, S, nblocks, xstride;
     int lds_cr, lds_xs, lds_sp, lds_xt, lds_bytes;
     int sp_wgs, sp_tt, sp_tiles;  // the ortho term's own workgroups (0: none)
+    bool sp_own;  // they take the entries only where the plan does not locate them
 };
 
 inline bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
@@ -65,15 +67,19 @@ inline bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
     if (a.has_ortho && ntt == 1) off += (kSkMaxCPS * 128 + 1) * (a.M <= 8 ? 16 : 32) + (kSkMaxCPS * 128 / 8) * 16;
     sh.lds_bytes = off;
     sh.sp_wgs = sh.sp_tt = sh.sp_tiles = 0;
+    sh.sp_own = false;
     if (a.has_ortho && ntt > 1 && S > 1 && ss_tokens(a.K) > 0 &&
         (int64_t)(S + 1) * a.M * a.N * 4 <= (int64_t)ORTH_NOALLOC_SCRATCH_BYTES) {
-        const int tt = ss_tokens(a.K), tiles = (int)((a.M + tt - 1) / tt);
+        int tt = ss_tokens(a.K), tiles = (int)((a.M + tt - 1) / tt);
         // three workgroups to four CUs, beside the dense ones (4096 -> 11008 at
         // 48 tokens, 1 %: 128 workgroups 30.3 us, 192 26.8, 256 28.8), each
         // wave with at least one unit of rows; whole rows of the XCD map
         const int64_t units = (a.N + kSsRows - 1) / kSsRows;
-        const int64_t per = std::max<int64_t>(1, std::min<int64_t>((units + 7) / 8, cus * 3 / 4 / tiles));
-        const int wgs = (int)((per * tiles + 7) / 8 * 8);
+        auto count = [&] {
+            const int64_t per = std::max<int64_t>(1, std::min<int64_t>((units + 7) / 8, cus * 3 / 4 / tiles));
+            return (int)((per * tiles + 7) / 8 * 8);
+        };
+        int wgs = count();
         // With a plan each lane can find its own entries of the slice instead.
         // That is the faster one for many entries in rows of like length, which
         // the estimates below (us; fitted to 3,048 planned calls, off by 6 and
@@ -93,12 +99,20 @@ inline bool skinny_shape(const ForwardArgs &a, int cus, SkinnyShape &sh) {
                                1.5e-6 * (S + 1) * a.M * a.N + 0.39e-6 * tiles * a.nnz;
         const double rounds = std::ceil((double)sh.nblocks * S / ((ntt == 2 ? 2 : 1) * cus));
         const double own_entries = 9.6 + rounds * (0.98 * cps + 0.36 * ntt * std::sqrt(es)) + ntt * (0.12 * es + 2.2e-6 * a.nnz);
-        if (!a.planned || (a.M > 32 && a.K > 4096) || es <= 8 || own_wgs < 1.05 * own_entries) {
-            sh.sp_tt = tt;
-            sh.sp_tiles = tiles;
-            sh.sp_wgs = wgs;
-            sh.lds_bytes = std::max(off, ss_lds(a.K, tt));
+        sh.sp_own = a.planned && (a.M <= 32 || a.K <= 4096) && es > 8 && own_wgs >= 1.05 * own_entries;
+        if (sh.sp_own) {
+            // (workgroups that mostly end at once: no more LDS than leaves room
+            // for all to start, or for as many dense ones to a CU)
+            const int all = (sh.nblocks * S + wgs + cus - 1) / cus;
+            const int room = kSsLdsCu / std::max(1, std::min(all, kSsLdsCu / off));
+            while (tt > 2 && ss_lds(a.K, tt) > room) tt /= 2;
+            tiles = (int)((a.M + tt - 1) / tt);
+            wgs = count();
         }
+        sh.sp_tt = tt;
+        sh.sp_tiles = tiles;
+        sh.sp_wgs = wgs;
+        sh.lds_bytes = std::max(off, ss_lds(a.K, tt));
     }
     return off <= 150 * 1024;
 }

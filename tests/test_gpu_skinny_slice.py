@@ -92,6 +92,25 @@ def test_many_planned_entries(gpu, oracle_mod, K, N, M, density, dtype):
         check_ortho(oracle_mod, lay, x, 1.0, dtype, plan=plan)
 
 
+@pytest.mark.parametrize("K,N,M,density,dtype", [
+    (4096, 1000, 33, 0.2, torch.float16), (4096, 2100, 64, 0.1, torch.bfloat16), (1152, 9000, 49, 0.2, torch.float16),
+    (8192, 1000, 17, 0.05, torch.bfloat16)])
+def test_many_planned_entries_out_of_order(gpu, oracle_mod, K, N, M, density, dtype):
+    """The same with columns that do not ascend, which the plan does not locate:
+    the workgroups take them as without a plan (bit for bit where they hold the
+    same 8 tokens), not each lane its whole row."""
+    lay = W.make_layer(K, N, 128, density, 9400 + K)
+    lay.col[:] = lay.col[::-1].copy()
+    x = torch.from_numpy(W.make_x(M, K, 9401 + M)).to(dtype).float().numpy()
+    y, k = run(lay, x, 1.0, dtype, plan=True)
+    z, _ = run(lay, x, 1.0, dtype)
+    assert k == "skinny"
+    check(oracle_mod, lay, x, 1.0, dtype, y)
+    check_ortho(oracle_mod, lay, x, 1.0, dtype, plan=True)
+    if M >= 49:
+        assert torch.equal(y, z)
+
+
 def test_skinny_slice_odd_csr_infinities_and_bias(gpu, oracle_mod):
     K, N, M = 1024, 777, 50
     lay = W.make_layer(K, N, 128, 0.05, 9000)
